@@ -244,14 +244,37 @@ __device__ __forceinline__ float rsq_softened(float x) { return __builtin_amdgcn
 
 // Short-range attenuation erfc(u) + 2u/sqrt(pi) exp(-u^2), u = r / (2 r_c)
 // (src/sbh_ffi.cu:151-157).  Also returns exp(-u^2) and r.
+//
+// Both terms share exp(-u^2): att = exp(-u^2) (1 + z) with
+// z = erfcx(u) - 1 + 2u/sqrt(pi) = w S(v), v = p u / (1 + p u), w = p u v,
+// p = 0.45 (z is u^2 at first order and 2u/sqrt(pi) at large u, so S is smooth
+// and bounded), and S a least-maximum fit of degree 7 on u in [0, 10]: 1.4e-8 of
+// 1 + z.  The product form keeps z's rounding relative to z, which vanishes
+// with u, where close pairs lie.  The hardware square root, reciprocal and
+// exponential (1 ulp each) make it 28 issue slots where erfcf, expf, sqrtf
+// and a division took about 110; against 64 bits att is as exact as with those
+// (root mean square of a pair's error, the softened kernel's rounding
+// included, for u <= 0.5 1.1e-7 against 1.2e-7, in (0.5, 1] 9.0e-8 against
+// 9.8e-8, in (1, 1.5] 5.2e-8 against 5.3e-8).  Periodic TreePM force of 128^3
+// particles (build and walk): 20.0 -> 17.8 ms.
 __device__ __forceinline__ float attenuation(float r2, float rc, float* exp_u2,
                                              float* dist) {
-  float r = sqrtf(r2 + 1e-12f);
-  float u = r / (2.0f * rc);
-  float e = expf(-(u * u));
+  const float t = r2 + 1e-12f;
+  const float r = __builtin_amdgcn_sqrtf(t);
+  const float e = __builtin_amdgcn_exp2f(t * ((-0.25f * 1.4426950408889634f / rc) / rc));
+  const float pu = r * (0.225f / rc);
+  const float v = pu * __builtin_amdgcn_rcpf(1.0f + pu);
+  float q = -0.0074539776f;
+  q = fmaf(q, v, 0.125911623f);
+  q = fmaf(q, v, -0.300382614f);
+  q = fmaf(q, v, 0.0324115604f);
+  q = fmaf(q, v, 0.407842994f);
+  q = fmaf(q, v, 0.628595412f);
+  q = fmaf(q, v, -3.31763482f);
+  q = fmaf(q, v, 4.93829918f);
   *exp_u2 = e;
   *dist = r;
-  return erfcf(u) + kTwoOverSqrtPi * u * e;
+  return fmaf(e, (pu * v) * q, e);
 }
 
 }  // namespace sbh
