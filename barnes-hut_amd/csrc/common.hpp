@@ -137,7 +137,8 @@ constexpr int kWsSort = 1;
 constexpr int kWsWalk = 2;
 constexpr int kWsPipeline = 3;
 constexpr int kWsRope = 4;
-constexpr int kWsSlots = 5;
+constexpr int kWsDirect = 5;
+constexpr int kWsSlots = 6;
 
 inline unsigned grid_for(int64_t n, int block, unsigned cap = 0x7fffffffu) {
   int64_t g = (n + block - 1) / block;
@@ -180,13 +181,6 @@ __device__ __forceinline__ float min_image_floor(float d, int periodic, float bo
 #pragma clang fp contract(off)
   return periodic ? d - box * floorf(d * inv_box + 0.5f) : d;
 }
-// Min-image as the direct-sum pair functions (src/sbh_ffi.cu:440-445).
-__device__ __forceinline__ float min_image_rint(float d, int periodic, float box,
-                                                float inv_box) {
-#pragma clang fp contract(off)
-  return periodic ? d - box * rintf(d * inv_box) : d;
-}
-
 // Philox4x32-10 (Salmon, Moraes, Dror, Shaw, SC'11): counter-based RNG used
 // by the stochastic walks in place of cuRAND XORWOW.
 __device__ __forceinline__ uint4 philox4x32_10(uint4 c, uint32_t k0, uint32_t k1) {
