@@ -124,15 +124,12 @@ __device__ __forceinline__ float smooth_pair(const Leaf3& L, float qx, float qy,
   return expf(-L.alpha * sqrtf(dx * dx + dy * dy + dz * dz));
 }
 
-// Pair/node contribution to the accumulator.
-template <int KIND>
-__device__ __forceinline__ void contribution(float px, float py, float pz, float m, float qx,
-                                             float qy, float qz, float gx, float gy, float gz,
-                                             const WalkParams& P, float& ax, float& ay,
-                                             float& az) {
-  float dx = min_image_floor(qx - px, P.periodic, P.box, P.inv_box);
-  float dy = min_image_floor(qy - py, P.periodic, P.box, P.inv_box);
-  float dz = min_image_floor(qz - pz, P.periodic, P.box, P.inv_box);
+// Contribution of mass m at displacement d (query - source, minimum image) to
+// the accumulator; vector kinds only.  CUT: with the attenuation (soft kinds).
+template <int KIND, bool CUT>
+__device__ __forceinline__ void pair_terms(float dx, float dy, float dz, float m, float gx,
+                                           float gy, float gz, const WalkParams& P, float& ax,
+                                           float& ay, float& az) {
   if constexpr (KIND == kGravGrad) {
     // gravityGrad (include/kernel.h:89-94)
     float t = sqrtf(dx * dx + dy * dy + dz * dz) + 1e-1f;
@@ -153,32 +150,57 @@ __device__ __forceinline__ void contribution(float px, float py, float pz, float
     ay += -m * (i3 * gy - k * dy);
     az += -m * (i3 * gz - k * dz);
   } else {
-    float r2 = dx * dx + dy * dy + dz * dz;
-    float inv_r = rsq_softened(r2 + P.eps2 + 1e-12f);
-    float s3 = inv_r * inv_r * inv_r;
-    float att = 1.0f, cc = 0.0f;
-    if (P.cutoff) {
+    float r2 = 0.f, s2, lin;
+    if constexpr (CUT) {
+      r2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+      s2 = rsq_softened(r2 + (P.eps2 + 1e-12f));
+    } else {
+      s2 = rsq_softened(fmaf(dz, dz, fmaf(dy, dy, fmaf(dx, dx, P.eps2 + 1e-12f))));
+    }
+    float s3 = s2;
+    s2 *= s2;
+    s3 *= s2;
+    float cc = 0.0f;
+    if constexpr (CUT) {
       float e, dist;
-      att = attenuation(r2, P.rc, &e, &dist);
-      if constexpr (KIND == kSoftVjp) cc = s3 * dist * e / (kTwoSqrtPi * P.rc * P.rc * P.rc);
+      lin = attenuation(r2, P.rc, &e, &dist) * s3;
+      if constexpr (KIND == kSoftVjp)
+        cc = s3 * (dist * e) * (1.0f / (kTwoSqrtPi * P.rc * P.rc * P.rc));
+    } else {
+      lin = s3;
     }
     if constexpr (KIND == kSoftForce) {
       // gravityGradSoftCutoff (src/sbh_ffi.cu:142-160)
-      float c = -m * att * s3;
-      ax += c * dx;
-      ay += c * dy;
-      az += c * dz;
+      const float c = -m * lin;
+      ax = fmaf(c, dx, ax);
+      ay = fmaf(c, dy, ay);
+      az = fmaf(c, dz, az);
     } else {
-      // gravityGradSoftCutoffVjp (src/sbh_ffi.cu:2062-2090)
-      float s5 = s3 * inv_r * inv_r;
-      float rg = dx * gx + dy * gy + dz * gz;
-      float lin = att * s3;
-      float rad = rg * (3.0f * att * s5 + cc);
-      ax += -m * (lin * gx - rad * dx);
-      ay += -m * (lin * gy - rad * dy);
-      az += -m * (lin * gz - rad * dz);
+      // gravityGradSoftCutoffVjp (src/sbh_ffi.cu:2062-2090):
+      // -m (lin g - (d.g) (3 lin s^2 + cc) d)
+      const float rg = fmaf(dz, gz, fmaf(dy, gy, dx * gx));
+      const float c = -m * lin, t = m * (rg * fmaf(3.0f * s2, lin, cc));
+      // (a pair's two parts are joined first: they partly cancel over the pairs)
+      ax += fmaf(c, gx, t * dx);
+      ay += fmaf(c, gy, t * dy);
+      az += fmaf(c, gz, t * dz);
     }
   }
+}
+
+// Pair/node contribution to the accumulator.
+template <int KIND>
+__device__ __forceinline__ void contribution(float px, float py, float pz, float m, float qx,
+                                             float qy, float qz, float gx, float gy, float gz,
+                                             const WalkParams& P, float& ax, float& ay,
+                                             float& az) {
+  const float dx = min_image_floor(qx - px, P.periodic, P.box, P.inv_box);
+  const float dy = min_image_floor(qy - py, P.periodic, P.box, P.inv_box);
+  const float dz = min_image_floor(qz - pz, P.periodic, P.box, P.inv_box);
+  if (P.cutoff)
+    pair_terms<KIND, true>(dx, dy, dz, m, gx, gy, gz, P, ax, ay, az);
+  else
+    pair_terms<KIND, false>(dx, dy, dz, m, gx, gy, gz, P, ax, ay, az);
 }
 
 template <int KIND>

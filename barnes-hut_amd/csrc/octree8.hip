@@ -8,6 +8,8 @@
 //   -> one kernel per level writing complete node records.
 // Walks (replace src/sbh_ffi.cu:1950-2144): one thread per query, depth-first
 // with the reference's push order, parameters passed by value.
+#include <type_traits>
+
 #include "common.hpp"
 #include "o8walk.hpp"
 #include "tree.hpp"
@@ -202,57 +204,141 @@ using o8::kSoftVjp;
 using o8::kWinding;
 
 
-// Node record read once per wave through the scalar data cache (the node
-// buffer is read-only during a walk; records are 4-byte aligned).
-typedef __attribute__((address_space(4))) const uint32_t cu32;
-
-__device__ __forceinline__ Node8 sload_node8(const Node8* nodes, uint32_t id) {
-  static_assert(sizeof(Node8) == 26 * 4, "Node8 is 26 dwords");
-  cu32* src = (cu32*)(nodes) + 26 * static_cast<uint64_t>(id);
-  Node8 n;
-  uint32_t* d = reinterpret_cast<uint32_t*>(&n);
-#pragma unroll
-  for (int k = 0; k < 26; ++k) d[k] = src[k];
-  return n;
-}
+// Point record read once per wave through the scalar data cache (the buffers
+// are read-only during a walk; records are 4-byte aligned).
+typedef uint32_t u32x8 __attribute__((ext_vector_type(8), aligned(4)));
+typedef __attribute__((address_space(4))) const u32x8 cu32x8;
 
 __device__ __forceinline__ Leaf3 sload_leaf3(const Leaf3* leaf, uint32_t j) {
-  cu32* src = (cu32*)(leaf) + 8 * static_cast<uint64_t>(j);
+  const u32x8 v = ((cu32x8*)(leaf))[j];
   Leaf3 r;
   uint32_t* d = reinterpret_cast<uint32_t*>(&r);
 #pragma unroll
-  for (int k = 0; k < 8; ++k) d[k] = src[k];
+  for (int k = 0; k < 8; ++k) d[k] = v[k];
   return r;
 }
 
-constexpr int kWStack = 96;  // >= 7 * 10 + 1 entries for max_depth 10
+constexpr int kRun = 4;              // points read together
+constexpr int kWStack = 96;          // >= 7 * 10 + 8 entries for max_depth 10
+constexpr uint32_t kRootEntry = ~0u;  // stack entry whose only child is node 0
+constexpr int kAccs = 4;             // partial sums per query
+
+// Partial sum of the node in child slot c: the 8 octants twice over the 4
+// sums, so that neighbours in every direction differ.
+__device__ __forceinline__ uint32_t key_of(uint32_t c) { return (c + (c >> 2)) & 3u; }
+
+// What the walk needs of a child node, as the lane that fetched it left it
+// in LDS for the wave (read back as broadcasts).
+struct alignas(16) Child {
+  float cx, cy, cz;     // cell centre
+  float open2;          // d^2 below this: nearer than beta diameters for sure
+  float bx, by, bz;     // box times the periodic image of the wave's first query (PER)
+  float far2;           // d^2 from this on: farther than beta diameters for sure
+  float lx, ly, lz;     // cell box (prune)
+  float mass;
+  float hx, hy, hz;
+  uint32_t id;
+  float px, py, pz;     // centre of mass
+  uint32_t start;
+  uint32_t end, is_leaf, key, deep;  // key: partial sum; deep: at or below split_level
+};
+static_assert(sizeof(Child) == 96, "Child is read as six float4");
+
+// Displacement q - p with the image shift b of a whole wave; *sure says that
+// it is the minimum image, i.e. that min_image_floor gives the same bits: the
+// shift is box * k with |k| <= 16 (infinite otherwise) and every component is
+// within (0.5 - 1e-5) boxes, 2e-6 being the most that the rounding of
+// d / box + 0.5 can move it there.
+template <bool PER>
+__device__ __forceinline__ float3 wave_delta(float qx, float qy, float qz, float px, float py,
+                                             float pz, const Child& c, float limit, bool* sure) {
+#pragma clang fp contract(off)
+  float3 d = make_float3(qx - px, qy - py, qz - pz);
+  *sure = true;
+  if constexpr (PER) {
+    d = make_float3(d.x - c.bx, d.y - c.by, d.z - c.bz);
+    *sure = fmaxf(fmaxf(fabsf(d.x), fabsf(d.y)), fabsf(d.z)) < limit;
+  }
+  return d;
+}
+
+// Squared distance as centre_dist() squares it (IEEE, not contracted).
+__device__ __forceinline__ float square(float3 d) {
+#pragma clang fp contract(off)
+  return d.x * d.x + d.y * d.y + d.z * d.z;
+}
+
+// should_prune() for an image-shifted query.
+__device__ __forceinline__ bool outside(const Child& c, float x, float y, float z, float r2) {
+#pragma clang fp contract(off)
+  const float dx = fmaxf(fmaxf(c.lx - x, x - c.hx), 0.0f);
+  const float dy = fmaxf(fmaxf(c.ly - y, y - c.hy), 0.0f);
+  const float dz = fmaxf(fmaxf(c.lz - z, z - c.hz), 0.0f);
+  return dx * dx + dy * dy + dz * dz > r2;
+}
 
 // Wave-coherent form of the reference's per-query DFS
 // (src/sbh_ffi.cu:1950-2144): the 64 queries of a wave share one stack of
-// (node, lanes) entries.  A popped node is evaluated by the lanes listed with
-// it; each of them skips it (empty, pruned), uses it (far field; a leaf is
-// summed exactly) or opens it, and the children are pushed, in the
-// reference's order, with the set of lanes that opened it.  Each lane thus
-// visits exactly the nodes of its own DFS and in the same order (a DFS
-// restricted to an ancestor-closed subset keeps its order), so its result is
-// bit-identical to the per-query walk, while every node and point record is
-// read once per wave through the scalar cache.  Queries run in Morton order
+// (opened node, lanes that opened it).  Popping an entry fetches the node's 8
+// children at once, one per lane, which derives what is common to the wave
+// (squared MAC bounds, cell box, image shift) and leaves it in LDS; each child
+// is then tested by the lanes of the entry, which skip it (empty, pruned), use
+// it (far field; a leaf is summed exactly) or open it.  The MAC decision is
+// that of the reference's expression dist / diameter >= beta in IEEE fp32: the
+// squared bounds stand 2^-14 to either side, and a lane between them evaluates
+// the expression itself; likewise a displacement that may not be the minimum
+// image falls back to min_image_floor.
+//
+// Every query keeps kAccs partial sums, combined in a fixed order at the end.
+// A node of level split_level, with all below it, belongs to one of them by
+// its child slot, and so does each node above (for its own far field or leaf
+// sum).  Each partial sum adds up in traversal order; a traversal restricted
+// to an ancestor-closed subset keeps its order, so a query's result depends
+// on the tree and on itself alone, bit for bit, not on the other lanes.  It
+// does not depend on SPLIT either: with SPLIT kAccs waves share a chunk of 64
+// queries, all of them walk the levels above split_level, and each takes the
+// subtrees and nodes of its own partial sum.  Queries run in Morton order
 // (order[t]) so that the lanes of a wave share most of their paths.
-// PER: periodicity as a template argument (the non-periodic walk carries no
-// minimum-image arithmetic; same bits either way).
-template <int KIND, bool PER>
-__global__ __launch_bounds__(kB) void k_walk8(const Leaf3* __restrict__ leaf,
+//
+// Bound by VALU issue where chunks fill the chip (the walk of a short-range
+// force tests 2000 children per chunk, a quarter of the lanes of which then use
+// each one), by the latency of the node fetches and by the longest chunk where
+// they do not.  Measured against one popped node at a time, tested through the
+// quotient, and one wave per chunk: softened walk of 100,003 Plummer points at
+// depth 7 12.8 -> 4.5 ms, its VJP 15.1 -> 6.2 ms; periodic short-range walk of
+// 128^3 particles 15.5 -> 11.8 ms.  Tried and dropped: deciding MAC and prune in the
+// fetching lanes for the whole bounding box of the chunk (16.9 -> 15.9 ms for the
+// pair of walks while every wave walked everything, but 13.4 -> 18.3 ms for the
+// short-range walk, whose chunks are wider than its cells), splitting only
+// the leaves' points between waves (16.9 against 13.3 ms), runs of 8 points
+// (106 scalar registers, 15.9 against 13.3 ms).
+// PER, CUT: periodicity and attenuation as template arguments: the walk without
+// them carries no such arithmetic, and no branch inside a run of points keeps
+// its loads from being issued together (same bits either way).
+template <int KIND, bool PER, bool CUT, bool SPLIT>
+__global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(
+    KIND == kSoftVjp ? 5 : KIND == kSoftForce ? 6 : 8))) void k_walk8(const Leaf3* __restrict__ leaf,
                                               const Node8* __restrict__ nodes,
                                               const float* __restrict__ queries,
                                               const float* __restrict__ cot, int64_t nq,
                                               const uint32_t* __restrict__ order,
                                               float* __restrict__ out, WalkParams P,
-                                              uint32_t num_nodes, uint32_t num_leaves) {
+                                              uint32_t num_nodes, uint32_t num_leaves,
+                                              uint32_t split_level) {
+  constexpr bool kScalar = o8::kScalarKind<KIND>;
+  constexpr int kVec = kScalar ? 1 : 3;
+  static_assert(!SPLIT || kB / 64 == kAccs, "a split chunk is one block");
   P.periodic = PER ? 1 : 0;
   __shared__ uint32_t s_node[kB / 64][kWStack];
   __shared__ uint64_t s_lanes[kB / 64][kWStack];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int64_t t = static_cast<int64_t>(blockIdx.x) * kB + threadIdx.x;
+  __shared__ uint8_t s_key[kB / 64][kWStack];  // of a deep node (its children's too), else kAccs
+  __shared__ Child s_child[kB / 64][8];
+  __shared__ float s_sum[SPLIT ? kAccs - 1 : 1][kVec][64];
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t chunk = SPLIT ? static_cast<int64_t>(blockIdx.x)
+                              : static_cast<int64_t>(blockIdx.x) * (kB / 64) + w;
+  const int64_t t = chunk * 64 + lane;
   const bool valid = t < nq;
   const int64_t q = !valid ? 0 : (order != nullptr ? static_cast<int64_t>(order[t]) : t);
   float qx = 0.f, qy = 0.f, qz = 0.f, gx = 0.f, gy = 0.f, gz = 0.f;
@@ -267,61 +353,234 @@ __global__ __launch_bounds__(kB) void k_walk8(const Leaf3* __restrict__ leaf,
     }
   }
   const uint64_t all = __ballot(valid);
-  if (all == 0) return;  // the whole wave is past the end
-  float ax = 0.f, ay = 0.f, az = 0.f;
+  if (!SPLIT && all == 0) return;  // the whole wave is past the end
+  const float limit = P.box * (0.5f - 1e-5f);
+  // sum: the partial sum in use, number cur (SPLIT: the wave's own); the
+  // others rest in acc
+  float sum[3] = {}, acc[SPLIT ? 1 : kAccs][3] = {};
+  uint32_t cur = SPLIT ? w : 0;
+  auto use_sum = [&](uint32_t k) {
+    if (SPLIT || k == cur) return;
+#pragma unroll
+    for (uint32_t m = 0; m < kAccs; ++m)
+      if (cur == m)
+        for (int a = 0; a < kVec; ++a) acc[SPLIT ? 0 : m][a] = sum[a];
+#pragma unroll
+    for (uint32_t m = 0; m < kAccs; ++m)
+      if (k == m)
+        for (int a = 0; a < kVec; ++a) sum[a] = acc[SPLIT ? 0 : m][a];
+    cur = k;
+  };
   uint32_t* stk_node = s_node[w];
   uint64_t* stk_lanes = s_lanes[w];
-  if (lane == 0) {
-    stk_node[0] = 0;
-    stk_lanes[0] = all;
+  uint8_t* stk_key = s_key[w];
+  Child* slab = s_child[w];
+  // the wave's first query picks the image shifts
+  const float rx = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(qx)));
+  const float ry = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(qy)));
+  const float rz = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(qz)));
+  int top = 0;
+  if (all != 0) {
+    if (lane == 0) {
+      stk_node[0] = kRootEntry;
+      stk_lanes[0] = all;
+      stk_key[0] = kAccs;
+    }
+    top = 1;
   }
-  int top = 1;
   __builtin_amdgcn_wave_barrier();
   while (top > 0) {
     --top;
     const uint32_t id = __builtin_amdgcn_readfirstlane(stk_node[top]);
-    const uint64_t lanes = stk_lanes[top];
-    __builtin_amdgcn_wave_barrier();
-    if (id >= num_nodes) continue;
-    const Node8 nd = sload_node8(nodes, id);
-    if (nd.contrib.mass == 0.0f) continue;
-    const bool mine = (lanes >> lane) & 1ull;
-    bool skip = !mine, far = false;
-    if (mine) {
-      if constexpr (o8::kPrunedKind<KIND>) skip = should_prune(&nd, qx, qy, qz, P);
-      if (!skip) far = use_far_field(&nd, qx, qy, qz, P);
-    }
-    if (nd.is_leaf) {
-      // a leaf always takes the far branch: the exact sum of its points
-      if (far) {
-        const uint32_t je = nd.end < num_leaves ? nd.end : num_leaves;
-        for (uint32_t j = nd.start; j < je; ++j)
-          contribution<KIND>(sload_leaf3(leaf, j), qx, qy, qz, gx, gy, gz, P, ax, ay, az);
+    // the entry's lanes as a scalar mask
+    const uint64_t entry_lanes = stk_lanes[top];
+    const uint32_t lanes_lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(entry_lanes));
+    const uint32_t lanes_hi =
+        __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(entry_lanes >> 32));
+    const uint64_t lanes = static_cast<uint64_t>(lanes_hi) << 32 | lanes_lo;
+    const uint32_t key = __builtin_amdgcn_readfirstlane(stk_key[top]);
+    // the children, one per lane
+    bool have = false;
+    if (lane < 8) {
+      uint32_t ch = 0;
+      have = lane == 0 && num_nodes > 0;
+      if (id != kRootEntry) {
+        ch = nodes[id].child[lane];
+        have = ((nodes[id].child_mask >> lane) & 1) != 0 && ch < num_nodes;
       }
-      continue;
+      if (have) {
+        const Node8* nd = nodes + ch;
+        Child c;
+        c.mass = nd->contrib.mass;
+        have = c.mass != 0.0f;
+        c.cx = nd->cx;
+        c.cy = nd->cy;
+        c.cz = nd->cz;
+        c.px = nd->contrib.pos[0];
+        c.py = nd->contrib.pos[1];
+        c.pz = nd->contrib.pos[2];
+        c.id = ch;
+        c.start = nd->start;
+        c.end = nd->end < num_leaves ? nd->end : num_leaves;
+        c.is_leaf = nd->is_leaf;
+        c.deep = nd->depth >= split_level;
+        c.key = key < kAccs ? key : key_of(lane);
+        if (SPLIT && c.deep && c.key != static_cast<uint32_t>(w)) have = false;
+        // (beta diameter)^2 and 2^-14 to either side; outside the range where
+        // the square is exact to a few ulp, every lane evaluates the quotient
+        const float r = P.beta * nd->diameter, r2 = r * r;
+        const bool plain = r2 > 1e-30f && r2 < 1e30f;
+        c.open2 = P.beta < 0.0f ? -1.0f : plain ? r2 * (1.0f - 6.1035156e-5f) : NAN;
+        c.far2 = P.beta < 0.0f ? -1.0f : plain ? r2 * (1.0f + 6.1035156e-5f) : NAN;
+        if constexpr (o8::kPrunedKind<KIND>) {
+#pragma clang fp contract(off)
+          const float h = nd->half_size;
+          c.lx = c.cx - h;
+          c.ly = c.cy - h;
+          c.lz = c.cz - h;
+          c.hx = c.cx + h;
+          c.hy = c.cy + h;
+          c.hz = c.cz + h;
+        }
+        if constexpr (PER) {
+#pragma clang fp contract(off)
+          const float kx = floorf((rx - c.cx) * P.inv_box + 0.5f);
+          const float ky = floorf((ry - c.cy) * P.inv_box + 0.5f);
+          const float kz = floorf((rz - c.cz) * P.inv_box + 0.5f);
+          const bool small = fabsf(kx) <= 16.0f && fabsf(ky) <= 16.0f && fabsf(kz) <= 16.0f;
+          c.bx = small ? P.box * kx : INFINITY;
+          c.by = P.box * ky;
+          c.bz = P.box * kz;
+        }
+        slab[lane] = c;
+      }
     }
-    if (far) contribution<KIND>(nd.contrib, qx, qy, qz, gx, gy, gz, P, ax, ay, az);
-    const uint64_t open = __ballot(!skip && !far);
-    if (open == 0) continue;
+    uint32_t todo = static_cast<uint32_t>(__ballot(have)) & 0xffu;
+    __builtin_amdgcn_wave_barrier();
+    while (todo != 0) {
+      const int slot = __builtin_ctz(todo);
+      todo &= todo - 1;
+      const Child c = slab[slot];
+      const uint32_t own = __builtin_amdgcn_readfirstlane(c.key);
+      const bool ours = !SPLIT || own == static_cast<uint32_t>(w);
+      bool sure;
+      const float3 d = wave_delta<PER>(qx, qy, qz, c.cx, c.cy, c.cz, c, limit, &sure);
+      const bool all_sure = !PER || (lanes & __ballot(!sure)) == 0;
+      // the lanes that do not prune the child
+      uint64_t use = lanes;
+      if constexpr (o8::kPrunedKind<KIND>) {
+        if (P.prune) {
+          if (all_sure) {
+#pragma clang fp contract(off)
+            use &= ~__ballot(PER ? outside(c, qx - c.bx, qy - c.by, qz - c.bz, P.r_cut_sq)
+                                 : outside(c, qx, qy, qz, P.r_cut_sq));
+          } else {
+            use &= ~__ballot(should_prune(nodes + c.id, qx, qy, qz, P));
+          }
+          if (use == 0) continue;
+        }
+      }
+      if (__builtin_amdgcn_readfirstlane(c.is_leaf) != 0) {
+        // a leaf always takes the far branch: the exact sum of its points
+        if (!ours) continue;
+        use_sum(own);
+        const uint32_t j1 = __builtin_amdgcn_readfirstlane(c.end);
+        uint32_t j = __builtin_amdgcn_readfirstlane(c.start);
+        if (__builtin_amdgcn_inverse_ballot_w64(use)) {
+          auto run = [&](auto count, uint32_t j0) {
+            constexpr int kCount = decltype(count)::value;
+            Leaf3 r[kCount];
 #pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      if ((nd.child_mask & (1u << c)) && top < kWStack && nd.child[c] < num_nodes) {
+            for (int u = 0; u < kCount; ++u) r[u] = sload_leaf3(leaf, j0 + u);
+#pragma unroll
+            for (int u = 0; u < kCount; ++u) {
+              if constexpr (kScalar) {
+                contribution<KIND>(r[u], qx, qy, qz, gx, gy, gz, P, sum[0], sum[1], sum[2]);
+              } else {
+                bool ok;
+                float3 e = wave_delta<PER>(qx, qy, qz, r[u].pos[0], r[u].pos[1], r[u].pos[2], c,
+                                           limit, &ok);
+                if (PER && __ballot(!ok) != 0)
+                  e = make_float3(
+                      min_image_floor(qx - r[u].pos[0], 1, P.box, P.inv_box),
+                      min_image_floor(qy - r[u].pos[1], 1, P.box, P.inv_box),
+                      min_image_floor(qz - r[u].pos[2], 1, P.box, P.inv_box));
+                o8::pair_terms<KIND, CUT>(e.x, e.y, e.z, r[u].mass, gx, gy, gz, P, sum[0],
+                                          sum[1], sum[2]);
+              }
+            }
+          };
+          for (; j + kRun <= j1; j += kRun) run(std::integral_constant<int, kRun>{}, j);
+          if (j + 2 <= j1) {
+            run(std::integral_constant<int, 2>{}, j);
+            j += 2;
+          }
+          if (j < j1) run(std::integral_constant<int, 1>{}, j);
+        }
+        continue;
+      }
+      uint64_t far;
+      if (all_sure) {
+        const float d2 = square(d);
+        far = __ballot(d2 >= c.far2);
+        const uint64_t between = use & ~far & ~__ballot(d2 < c.open2);
+        if (between != 0)
+          far |= between & __ballot(use_far_field(nodes + c.id, qx, qy, qz, P));
+      } else {
+        far = __ballot(use_far_field(nodes + c.id, qx, qy, qz, P));
+      }
+      far &= use;
+      if (far != 0 && ours) {
+        use_sum(own);
+        if (__builtin_amdgcn_inverse_ballot_w64(far)) {
+          if constexpr (kScalar) {
+            contribution<KIND>(nodes[c.id].contrib, qx, qy, qz, gx, gy, gz, P, sum[0], sum[1],
+                               sum[2]);
+          } else {
+            bool ok;
+            float3 e = wave_delta<PER>(qx, qy, qz, c.px, c.py, c.pz, c, limit, &ok);
+            if (PER && __ballot(!ok) != 0)
+              e = make_float3(min_image_floor(qx - c.px, 1, P.box, P.inv_box),
+                              min_image_floor(qy - c.py, 1, P.box, P.inv_box),
+                              min_image_floor(qz - c.pz, 1, P.box, P.inv_box));
+            o8::pair_terms<KIND, CUT>(e.x, e.y, e.z, c.mass, gx, gy, gz, P, sum[0], sum[1],
+                                      sum[2]);
+          }
+        }
+      }
+      const uint64_t open = use & ~far;
+      if (open != 0 && top < kWStack) {
         if (lane == 0) {
-          stk_node[top] = nd.child[c];
+          stk_node[top] = c.id;
           stk_lanes[top] = open;
+          stk_key[top] = static_cast<uint8_t>(c.deep ? own : kAccs);
         }
         ++top;
       }
     }
     __builtin_amdgcn_wave_barrier();
   }
-  if (!valid) return;
-  if constexpr (o8::kScalarKind<KIND>) {
-    out[q] = ax;
+  float r[kVec];
+  if constexpr (SPLIT) {
+    if (w > 0)
+      for (int a = 0; a < kVec; ++a) s_sum[w - 1][a][lane] = sum[a];
+    __syncthreads();
+    if (w > 0 || !valid) return;
+    for (int a = 0; a < kVec; ++a)
+      r[a] = (sum[a] + s_sum[0][a][lane]) + (s_sum[1][a][lane] + s_sum[2][a][lane]);
   } else {
-    out[3 * q + 0] = ax;
-    out[3 * q + 1] = ay;
-    out[3 * q + 2] = az;
+    if (!valid) return;
+    use_sum(0);
+    for (int a = 0; a < kVec; ++a)
+      r[a] = (sum[a] + acc[1 % (SPLIT ? 1 : kAccs)][a]) +
+             (acc[2 % (SPLIT ? 1 : kAccs)][a] + acc[3 % (SPLIT ? 1 : kAccs)][a]);
+  }
+  if constexpr (kScalar) {
+    out[q] = r[0];
+  } else {
+    out[3 * q + 0] = r[0];
+    out[3 * q + 1] = r[1];
+    out[3 * q + 2] = r[2];
   }
 }
 
@@ -336,6 +595,28 @@ uint64_t total_nodes8(int max_depth) {
 
 using o8::check_walk_common;
 using o8::make_walk_params;
+
+template <int KIND, bool SOFT, bool SPLIT>
+auto pick_walk(const WalkParams& P) {
+  if constexpr (SOFT) {
+    if (P.cutoff)
+      return P.periodic ? k_walk8<KIND, true, true, SPLIT> : k_walk8<KIND, false, true, SPLIT>;
+  }
+  return P.periodic ? k_walk8<KIND, true, false, SPLIT> : k_walk8<KIND, false, false, SPLIT>;
+}
+
+// Level whose nodes the partial sums divide: two above the leaves, so that a
+// query's neighbourhood spreads over all sums while few nodes lie above.
+uint32_t split_level(uint32_t num_nodes) {
+  int depth = 0;
+  while (depth < 10 && total_nodes8(depth) < num_nodes) ++depth;
+  return static_cast<uint32_t>(depth > 3 ? depth - 2 : 1);
+}
+
+// Chunks of 64 queries below which each is walked by kAccs waves: 4096 chunks
+// are 4 waves per SIMD, half of what fits, and the longest chunks then hold up
+// the end of the launch.
+constexpr int64_t kSplitChunks = 4096;
 
 template <int KIND>
 int launch_walk(void* stream, const SbhBuffer* leaf_bytes, const SbhBuffer* node_bytes,
@@ -353,13 +634,17 @@ int launch_walk(void* stream, const SbhBuffer* leaf_bytes, const SbhBuffer* node
     int rc = tree::query_order(s, static_cast<const float*>(queries->data), nq, ws, &order);
     if (rc != SBH_OK) return rc;
   }
-  (P.periodic ? k_walk8<KIND, true> : k_walk8<KIND, false>)<<<grid_for(nq, kB), kB, 0, s>>>(
+  const auto num_nodes = static_cast<uint32_t>(byte_count(node_bytes) / sizeof(Node8));
+  const bool split = (nq + 63) / 64 < kSplitChunks;
+  constexpr bool kSoft = o8::kPrunedKind<KIND>;
+  auto* walk = split ? pick_walk<KIND, kSoft, true>(P) : pick_walk<KIND, kSoft, false>(P);
+  walk<<<split ? grid_for(nq, 64) : grid_for(nq, kB), kB, 0, s>>>(
       static_cast<const Leaf3*>(leaf_bytes->data), static_cast<const Node8*>(node_bytes->data),
       static_cast<const float*>(queries->data),
       cot ? static_cast<const float*>(cot->data) : nullptr, nq, order,
       static_cast<float*>(out->data),
-      P, static_cast<uint32_t>(byte_count(node_bytes) / sizeof(Node8)),
-      static_cast<uint32_t>(byte_count(leaf_bytes) / sizeof(Leaf3)));
+      P, num_nodes, static_cast<uint32_t>(byte_count(leaf_bytes) / sizeof(Leaf3)),
+      split_level(num_nodes));
   SBH_LAUNCH_CHECK();
   return SBH_OK;
 }
