@@ -118,9 +118,11 @@ __device__ __forceinline__ int lanes_below(uint64_t m) {
 // lane 0 only), starting at 0.  Each wave makes at most 8 failing claims, so
 // every wave reaches the -1 exit.  With `order` (a permutation of the groups
 // that keeps each eighth's groups inside it) claim t of an eighth takes
-// group order[t] instead of group t.
+// group order[t] instead of group t, and with `small` the first small[q]
+// claims of eighth q are left to the team walk.
 __device__ __forceinline__ int next_group(Header* hdr, int num_groups, int lane, int& tries,
-                                          const int* order = nullptr) {
+                                          const int* order = nullptr,
+                                          const int32_t* small = nullptr) {
   int g = -1;
   if (lane == 0) {
     const int home = static_cast<int>(blockIdx.x & 7u);
@@ -128,7 +130,7 @@ __device__ __forceinline__ int next_group(Header* hdr, int num_groups, int lane,
       const int q = (home + tries) & 7;
       const int lo = static_cast<int>(static_cast<int64_t>(num_groups) * q / 8);
       const int hi = static_cast<int>(static_cast<int64_t>(num_groups) * (q + 1) / 8);
-      const int t = lo + atomicAdd(&hdr->xq[q], 1);
+      const int t = lo + atomicAdd(&hdr->xq[q], 1) + (small != nullptr ? small[q] : 0);
       if (t < hi) {
         g = order != nullptr ? order[t] : t;
         break;

@@ -573,7 +573,7 @@ __global__ __launch_bounds__(1024) void k_topo_scan(Header* __restrict__ hdr,
     hdr->num_nodes = static_cast<int32_t>(start);
     hdr->num_groups = gtot;
     hdr->queue = 0;
-    for (int x = 0; x < 8; ++x) hdr->xq[x] = 0;
+    for (int x = 0; x < 8; ++x) hdr->xq[x] = hdr->tq[x] = 0;
   }
 }
 
@@ -911,6 +911,7 @@ struct WalkArgs {
   unsigned long long* stats;
   const int* order;  // claim order of the groups (k_group_order)
   float* gcost;      // measured cost of each group, for the next walk's order
+  const int32_t* small;  // forests: groups of small sets at the front of each eighth
 };
 
 struct Lane {
@@ -965,7 +966,9 @@ __device__ __forceinline__ void far_batch(const WalkArgs& A, const Lane& L, cons
   // (dL/dS xx yy zz xy xz yz, minus dL/dM, minus dL/dX x) and (minus dL/dX y, z)
   float q8[8 * C];
   float q2[2 * C];
-  float mw[C];  // node masses (second-moment adjoint)
+  // node masses (second-moment adjoint; not an array: selecting between two
+  // elements by lane would put it into scratch memory)
+  float mw0 = 0.f, mw1 = 0.f, mw2 = 0.f, mw3 = 0.f;
 #pragma unroll
   for (int t = 0; t < C; ++t) {
     const float4 m = sload4(A.mp, idx[t]);
@@ -984,7 +987,10 @@ __device__ __forceinline__ void far_batch(const WalkArgs& A, const Lane& L, cons
         fy = fmaf(a, Dy, fy);
         fz = fmaf(a, Dz, fz);
       }
-      mw[t] = m.w;
+      if (t == 0) mw0 = m.w;
+      if (t == 1) mw1 = m.w;
+      if (t == 2) mw2 = m.w;
+      if (t == 3) mw3 = m.w;
       const float u3 = L.c3x * Dx + L.c3y * Dy + L.c3z * Dz;  // 3 u
       const float h = s2 * u3;
       const float ex = fmaf(h, Dx, -L.cx), ey = fmaf(h, Dy, -L.cy), ez = fmaf(h, Dz, -L.cz);
@@ -1103,7 +1109,7 @@ __device__ __forceinline__ void far_batch(const WalkArgs& A, const Lane& L, cons
       // of node 2c + (j >> 3)
       const float sum = lds_wave_sum<16>(q8 + 16 * c, L.red, lane);
       const int j = lane >> 2, slot = j & 7;
-      const float mx = SMOM ? -(lane < 32 ? mw[2 * c] : mw[2 * c + 1]) : -1.0f;
+      const float mx = !SMOM ? -1.0f : c == 0 ? -(lane < 32 ? mw0 : mw1) : -(lane < 32 ? mw2 : mw3);
       if ((lane & 3) == 0) {
         const int e = far[2 * c + (j >> 3)];
         if (e != A.sentinel) {
@@ -1118,7 +1124,7 @@ __device__ __forceinline__ void far_batch(const WalkArgs& A, const Lane& L, cons
       const int j = lane >> 3;
       float mx = -1.0f;
       if constexpr (SMOM)
-        mx = -(lane < 32 ? (lane < 16 ? mw[0] : mw[1]) : (lane < 48 ? mw[2] : mw[3]));
+        mx = -(lane < 32 ? (lane < 16 ? mw0 : mw1) : (lane < 48 ? mw2 : mw3));
       if ((lane & 7) == 0) {
         const int e = far[j >> 1];
         if (e != A.sentinel) atomicAdd(A.adj + 4 * e + 1 + (j & 1), mx * sum);
@@ -1185,65 +1191,114 @@ __device__ __forceinline__ void near_batch(const WalkArgs& A, const Lane& L, int
     scatter_batch<4 * CH, 4, 4, true, true>(part, L.red, lane, A.sgrad, 4, nullptr, -1, j0, s1);
 }
 
-// One query group (sorted points [base, base + cnt)) processed by one wave.
+// Near sources [s0, s1) (sorted points), wave-uniform bounds.
 template <bool VJP, int ORDER, bool FORCES>
+__device__ __forceinline__ void near_range(const WalkArgs& A, const Lane& L, int i, int base,
+                                           int nvalid, int s0, int s1, int lane, float& fx,
+                                           float& fy, float& fz, float& gx, float& gy, float& gz,
+                                           unsigned long long& n_near) {
+  // The monopole forward walk reads 16 sources per batch while the loads of a
+  // batch are in flight together (its registers allow it).
+  constexpr bool kWide = !VJP && ORDER == 1;
+  // self pairs are skipped
+  n_near += static_cast<unsigned long long>(s1 - s0) * nvalid -
+            static_cast<unsigned long long>(max(0, min(s1, base + nvalid) - max(s0, base)));
+  // batches of 8, then the rest exactly (4, 2, 1); the quadrupole adjoint
+  // and the adjoint that also returns forces pad their last batch of 8
+  // instead (tail variants push them past their register budget and cost
+  // more than the padding saves)
+  if constexpr (VJP && (ORDER == 2 || FORCES)) {
+    for (int j0 = s0; j0 < s1; j0 += kChunk)
+      near_batch<VJP, FORCES, kChunk, true, true>(A, L, i, j0, s1, lane, fx, fy, fz, gx, gy, gz);
+  } else {
+    int j0 = s0;
+    if constexpr (VJP) {
+      // ranges away from the group's own points skip the self-pair test
+      if (s1 <= base || s0 >= base + nvalid) {
+        for (; j0 + kChunk <= s1; j0 += kChunk)
+          near_batch<VJP, FORCES, kChunk, false>(A, L, i, j0, s1, lane, fx, fy, fz, gx, gy, gz);
+      }
+    }
+    if constexpr (kWide) {
+      for (; j0 + 2 * kChunk <= s1; j0 += 2 * kChunk)
+        near_batch<VJP, FORCES, 2 * kChunk>(A, L, i, j0, s1, lane, fx, fy, fz, gx, gy, gz);
+    }
+    for (; j0 + kChunk <= s1; j0 += kChunk)
+      near_batch<VJP, FORCES, kChunk>(A, L, i, j0, s1, lane, fx, fy, fz, gx, gy, gz);
+    if (j0 + 4 <= s1) {
+      near_batch<VJP, FORCES, 4>(A, L, i, j0, s1, lane, fx, fy, fz, gx, gy, gz);
+      j0 += 4;
+    }
+    if (j0 + 2 <= s1) {
+      near_batch<VJP, FORCES, 2>(A, L, i, j0, s1, lane, fx, fy, fz, gx, gy, gz);
+      j0 += 2;
+    }
+    if (j0 < s1) near_batch<VJP, FORCES, 1>(A, L, i, j0, s1, lane, fx, fy, fz, gx, gy, gz);
+  }
+}
+
+// Position and cotangent of the lane's query (idle lanes repeat the group's
+// first point, without a cotangent).
+template <bool VJP>
+__device__ __forceinline__ Lane load_lane(const WalkArgs& A, int base, int cnt, int lane,
+                                          float* red) {
+  const int i = base + lane;
+  const bool valid = lane < cnt;
+  Lane L;
+  L.red = red;
+  const float4 me = A.sp[valid ? i : base];
+  L.x = me.x;
+  L.y = me.y;
+  L.z = me.z;
+  L.cx = L.cy = L.cz = 0.f;
+  if constexpr (VJP) {
+    if (valid) {
+      const float4 c = A.sc[i];
+      L.cx = c.x;
+      L.cy = c.y;
+      L.cz = c.z;
+    }
+  }
+  L.c3x = 3.0f * L.cx;
+  L.c3y = 3.0f * L.cy;
+  L.c3z = 3.0f * L.cz;
+  return L;
+}
+
+// One query group (sorted points [base, base + cnt)) by one wave, monopole
+// terms.
+template <bool VJP, bool FORCES>
 __device__ __forceinline__ void walk_group(const WalkArgs& A, int base, int cnt, int lane,
                                            int* stack, int* far, int* near, float* red,
                                            unsigned long long& n_far,
                                            unsigned long long& n_near) {
   const int i = base + lane;
-  const bool valid = lane < cnt;
-  Lane L;
-  L.red = red;
-  {
-    const float4 me = A.sp[valid ? i : base];
-    L.x = me.x;
-    L.y = me.y;
-    L.z = me.z;
-    L.cx = L.cy = L.cz = 0.f;
-    if constexpr (VJP) {
-      if (valid) {
-        const float4 c = A.sc[i];
-        L.cx = c.x;
-        L.cy = c.y;
-        L.cz = c.z;
-      }
-    }
-    L.c3x = 3.0f * L.cx;
-    L.c3y = 3.0f * L.cy;
-    L.c3z = 3.0f * L.cz;
-  }
+  const Lane L = load_lane<VJP>(A, base, cnt, lane, red);
   const Box box = wave_box(L.x, L.y, L.z);
-  const int nvalid = cnt;
-
   float fx = 0.f, fy = 0.f, fz = 0.f;
   float gx = 0.f, gy = 0.f, gz = 0.f;
 
-  // The quadrupole and second-moment adjoints hold 10 partials per node:
-  // batches of 4 nodes, not 8 (8 spill).
-  constexpr int C = (VJP && ORDER != 1) ? kChunk / 2 : kChunk;
-  // The monopole forward walk reads 16 nodes / sources per batch while the
-  // loads of a batch are in flight together (its registers allow it); the
-  // rest of a list or range is done in batches of 8 as the others.
-  constexpr bool kWide = !VJP && ORDER == 1;
+  // The forward walk reads 16 nodes per batch while the loads of a batch are
+  // in flight together (its registers allow it), the rest of a list 8 at a
+  // time.
   auto flush_far = [&](int nfar) {
-    n_far += static_cast<unsigned long long>(nfar) * nvalid;
-    const int padded = (nfar + C - 1) & ~(C - 1);
+    n_far += static_cast<unsigned long long>(nfar) * cnt;
+    const int padded = (nfar + kChunk - 1) & ~(kChunk - 1);
     if (lane < padded - nfar) far[nfar + lane] = A.sentinel;
     __builtin_amdgcn_wave_barrier();
     int f0 = 0;
-    if constexpr (kWide) {
-      for (; f0 + 2 * C <= padded; f0 += 2 * C)
-        far_batch<VJP, ORDER, FORCES, 2 * C>(A, L, far + f0, lane, fx, fy, fz, gx, gy, gz);
+    if constexpr (!VJP) {
+      for (; f0 + 2 * kChunk <= padded; f0 += 2 * kChunk)
+        far_batch<VJP, 1, FORCES, 2 * kChunk>(A, L, far + f0, lane, fx, fy, fz, gx, gy, gz);
     }
-    for (; f0 < padded; f0 += C)
-      far_batch<VJP, ORDER, FORCES, C>(A, L, far + f0, lane, fx, fy, fz, gx, gy, gz);
+    for (; f0 < padded; f0 += kChunk)
+      far_batch<VJP, 1, FORCES, kChunk>(A, L, far + f0, lane, fx, fy, fz, gx, gy, gz);
     __builtin_amdgcn_wave_barrier();
   };
 
   // Near leaves whose points directly follow each other in sorted order
   // (sibling leaves, appended in order by the traversal) are merged into one
-  // source range, so only a range end pads its last batch of kChunk.
+  // source range.
   auto flush_near = [&](int nnear) {
     int b = 0;
     while (b < nnear) {
@@ -1257,43 +1312,8 @@ __device__ __forceinline__ void walk_group(const WalkArgs& A, int base, int cnt,
         ++b;
       }
       s1 = __builtin_amdgcn_readfirstlane(s1);  // wave-uniform: keeps source loads scalar
-      // self pairs are skipped
-      n_near += static_cast<unsigned long long>(s1 - s0) * nvalid -
-                static_cast<unsigned long long>(max(0, min(s1, base + nvalid) - max(s0, base)));
-      // batches of 8, then the rest exactly (4, 2, 1); the quadrupole adjoint
-      // and the adjoint that also returns forces pad their last batch of 8
-      // instead (tail variants push them past their register budget and cost
-      // more than the padding saves)
-      if constexpr (VJP && (ORDER == 2 || FORCES)) {
-        for (int j0 = s0; j0 < s1; j0 += kChunk)
-          near_batch<VJP, FORCES, kChunk, true, true>(A, L, i, j0, s1, lane, fx, fy, fz, gx, gy,
-                                                      gz);
-      } else {
-        int j0 = s0;
-        if constexpr (VJP) {
-          // ranges away from the group's own points skip the self-pair test
-          if (s1 <= base || s0 >= base + nvalid) {
-            for (; j0 + kChunk <= s1; j0 += kChunk)
-              near_batch<VJP, FORCES, kChunk, false>(A, L, i, j0, s1, lane, fx, fy, fz, gx, gy,
-                                                     gz);
-          }
-        }
-        if constexpr (kWide) {
-          for (; j0 + 2 * kChunk <= s1; j0 += 2 * kChunk)
-            near_batch<VJP, FORCES, 2 * kChunk>(A, L, i, j0, s1, lane, fx, fy, fz, gx, gy, gz);
-        }
-        for (; j0 + kChunk <= s1; j0 += kChunk)
-          near_batch<VJP, FORCES, kChunk>(A, L, i, j0, s1, lane, fx, fy, fz, gx, gy, gz);
-        if (j0 + 4 <= s1) {
-          near_batch<VJP, FORCES, 4>(A, L, i, j0, s1, lane, fx, fy, fz, gx, gy, gz);
-          j0 += 4;
-        }
-        if (j0 + 2 <= s1) {
-          near_batch<VJP, FORCES, 2>(A, L, i, j0, s1, lane, fx, fy, fz, gx, gy, gz);
-          j0 += 2;
-        }
-        if (j0 < s1) near_batch<VJP, FORCES, 1>(A, L, i, j0, s1, lane, fx, fy, fz, gx, gy, gz);
-      }
+      near_range<VJP, 1, FORCES>(A, L, i, base, cnt, s0, s1, lane, fx, fy, fz, gx, gy, gz,
+                                 n_near);
     }
   };
 
@@ -1301,7 +1321,7 @@ __device__ __forceinline__ void walk_group(const WalkArgs& A, int base, int cnt,
   traverse<true>(A.hdr, &A.hdr->overflow, A.topo, A.geo, A.mp, A.beta, box, lane, root, stack,
                  far, near, flush_far, flush_near);
 
-  if (valid) {
+  if (lane < cnt) {
     const int64_t o = static_cast<int64_t>(A.perm[i]);
     if constexpr (FORCES) {
       A.forces[3 * o + 0] = fx;
@@ -1320,8 +1340,13 @@ __device__ __forceinline__ void walk_group(const WalkArgs& A, int base, int cnt,
 // at the end, and dealing the cheap groups last shortens that tail.  Costs
 // are binned (256 bins, heaviest first) and the order inside a bin is that
 // of the atomics.  Only the schedule depends on the costs, never a result.
+// Forests: the groups of sets below kSinglePoints, which the teams walk, come
+// first in their eighth (bin 0) and hdr->small counts them; without costs the
+// others keep about their order.  A forest of such sets only keeps its order.
 constexpr int kOrderBins = 256;
-__global__ __launch_bounds__(1024) void k_group_order(const Header* __restrict__ hdr,
+__global__ __launch_bounds__(1024) void k_group_order(Header* __restrict__ hdr,
+                                                      const int32_t* __restrict__ offs, int nsets,
+                                                      const int2* __restrict__ groups,
                                                       const float* __restrict__ cost_own,
                                                       const float* __restrict__ cost_other,
                                                       int* __restrict__ gorder, Sched* sched_own,
@@ -1335,12 +1360,23 @@ __global__ __launch_bounds__(1024) void k_group_order(const Header* __restrict__
   const bool own = sched_own->magic == kSchedMagic && sched_own->groups == ng;
   const bool other = sched_other->magic == kSchedMagic && sched_other->groups == ng;
   const float* gcost = own ? cost_own : cost_other;
-  if (!own && !other) {
+  const bool cost = own || other;
+  if (nsets > 1) {
+    int large = 0;
+    for (int k = threadIdx.x; k < nsets; k += 1024)
+      large |= offs[k + 1] - offs[k] >= kSinglePoints ? 1 : 0;
+    if (__syncthreads_or(large) == 0) {
+      for (int t = r.x + static_cast<int>(threadIdx.x); t < r.y; t += 1024) gorder[t] = t;
+      if (threadIdx.x == 0) hdr->small[blockIdx.x] = r.y - r.x;
+      return;
+    }
+  }
+  if (!cost && nsets <= 1) {
     for (int t = r.x + static_cast<int>(threadIdx.x); t < r.y; t += 1024) gorder[t] = t;
   } else {
     auto clean = [](float c) { return c > 0.0f && c < 3.0e38f ? c : 0.0f; };  // NaN -> 0
     float m = 0.0f;
-    for (int t = r.x + static_cast<int>(threadIdx.x); t < r.y; t += 1024)
+    for (int t = r.x + static_cast<int>(threadIdx.x); cost && t < r.y; t += 1024)
       m = fmaxf(m, clean(gcost[t]));
     m = gw::wave_max(m);
     if ((threadIdx.x & 63) == 0) s_max[threadIdx.x >> 6] = m;
@@ -1348,16 +1384,24 @@ __global__ __launch_bounds__(1024) void k_group_order(const Header* __restrict__
     __syncthreads();
     m = 0.0f;
     for (int k = 0; k < 16; ++k) m = fmaxf(m, s_max[k]);
-    const float scale = m > 0.0f ? (kOrderBins - 0.5f) / m : 0.0f;
+    const float scale = m > 0.0f ? (kOrderBins - 1.5f) / m : 0.0f;
     auto bin_of = [&](int t) {
+      if (nsets > 1) {
+        const int set = set_of(offs, nsets, groups[t].x);
+        if (offs[set + 1] - offs[set] < kSinglePoints) return 0;
+      }
+      if (!cost)
+        return 1 + static_cast<int>(static_cast<int64_t>(t - r.x) * (kOrderBins - 1) /
+                                    (r.y - r.x));
       const int b = static_cast<int>(clean(gcost[t]) * scale);
-      return kOrderBins - 1 - min(max(b, 0), kOrderBins - 1);  // heaviest in bin 0
+      return kOrderBins - 1 - min(max(b, 0), kOrderBins - 2);  // heaviest in bin 1
     };
     for (int t = r.x + static_cast<int>(threadIdx.x); t < r.y; t += 1024)
       atomicAdd(&s_bin[bin_of(t)], 1);
     __syncthreads();
     if (threadIdx.x == 0) {  // exclusive scan of the bins (256 entries)
       int run = r.x;
+      hdr->small[blockIdx.x] = s_bin[0];
       for (int b = 0; b < kOrderBins; ++b) {
         const int c = s_bin[b];
         s_bin[b] = run;
@@ -1374,14 +1418,17 @@ __global__ __launch_bounds__(1024) void k_group_order(const Header* __restrict__
   }
 }
 
-// Persistent walk: each wave takes query groups from a device work queue
-// until none are left (heavy groups do not hold up a static schedule).
-// Occupancy targets: the adjoint walks at 4 waves per SIMD (at most 128
-// VGPRs; their 40 KB of LDS per 4-wave block allow no more), the forward
-// walks at 7 (at most 72 VGPRs; 22 KB of LDS per block, 7 blocks per CU;
-// 6 waves were 5% slower).  WPB waves per block (the block size is a tuning
-// dimension; every wave walks on its own).
-template <bool VJP, int ORDER, bool FORCES, int WPB>
+// Persistent walk of large sets with monopole terms: each wave takes query
+// groups from a device work queue until none are left (heavy groups do not hold
+// up a static schedule).  The adjoints at 4 waves per SIMD (at most 128 VGPRs;
+// their 40 KB of LDS per 4-wave block allow no more), the forward walk at 7 (at
+// most 72 VGPRs; 6 waves were 5% slower).  WPB waves per block (the block size
+// is a tuning dimension; every wave walks on its own).  From 700,000 points on
+// it is up to 9% faster than the teams below, whose lists are padded and merged
+// in smaller pieces (2^20 points, Plummer / uniform / blobs: forces 6.6, 4.1, 3.4
+// against 7.1, 4.45, 3.6 ms, adjoint 16.1, 9.5, 7.8 against 16.6, 10.1, 8.0;
+// at 500,000 points forces 3.8, 2.06, 1.62 against 3.5, 1.95, 1.54).
+template <bool VJP, bool FORCES, int WPB>
 __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(VJP ? 4 : 7))) void k_walk(
     WalkArgs A) {
   __shared__ int s_stack[WPB][kRunStackWords];
@@ -1393,17 +1440,22 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(VJP ? 
   const int w = threadIdx.x >> 6;
   const int num_groups = A.hdr->num_groups;
   unsigned long long n_far = 0, n_near = 0, n_groups = 0;
+  if (A.small != nullptr) {  // a forest of small sets has nothing to claim
+    int left = num_groups;
+    for (int q = 0; q < 8; ++q) left -= A.small[q];
+    if (left == 0) return;
+  }
   int tries = 0;
   while (true) {
-    const int g = next_group(A.hdr, num_groups, lane, tries, A.order);
+    const int g = next_group(A.hdr, num_groups, lane, tries, A.order, A.small);
     if (g < 0) break;  // every wave reaches this exit
     const int2 grp = A.groups[g];
     const int base = __builtin_amdgcn_readfirstlane(grp.x);
     const int cnt = __builtin_amdgcn_readfirstlane(grp.y);
     if (cnt < 1 || cnt > 64 || base < 0 || base + cnt > A.n) continue;  // corrupt entry
     const uint64_t t0 = __builtin_amdgcn_s_memtime();
-    walk_group<VJP, ORDER, FORCES>(A, base, cnt, lane, s_stack[w], s_far[w], s_near[w],
-                                   s_red[w], n_far, n_near);
+    walk_group<VJP, FORCES>(A, base, cnt, lane, s_stack[w], s_far[w], s_near[w], s_red[w], n_far,
+                            n_near);
     const uint64_t t1 = __builtin_amdgcn_s_memtime();
     if (lane == 0) A.gcost[g] = static_cast<float>(t1 - t0);
     ++n_groups;
@@ -1412,6 +1464,250 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(VJP ? 
     atomicAdd(&A.stats[0], n_far);
     atomicAdd(&A.stats[1], n_near);
     atomicAdd(&A.stats[2], n_groups);
+  }
+}
+
+// ------------------------------------------------------------------ team walk
+// Walk with the TEAM waves of a block sharing each group.  The threads test
+// candidate nodes (up to kTeamWidth at once), the accepted nodes and near
+// leaves go to lists in LDS in a fixed order (block scans), and the lists are
+// dealt to kShares shares in turn: nodes in runs of kTeamRun, leaves in runs of
+// kTeamLeaves (neighbours in the list are often siblings, whose points adjoin
+// and are summed as one range).  Each share has its own sums, combined in
+// order at the end.  What enters a share depends on the tree and the group
+// alone, not on TEAM or the launch, so forces are reproducible bit for bit,
+// between single sets and forests too.
+//
+// With one wave per group, sets below ~2^17 points leave most of the 1024 SIMDs
+// empty or with too few waves to hide a record load (10,000 points: 157
+// groups), and the launch lasts as long as its longest group; where the chip
+// is full it still ends in a tail of single groups.  What bounds a team:
+// barriers and latency in small sets, VALU issue in large ones.  Whole calls,
+// one wave per group -> teams: forces (quadrupole) of 2,003 Plummer points 0.37 ->
+// 0.19 ms; 10,000 uniform points, leaf 32, forces 0.57 -> 0.23, second-moment
+// adjoint 0.97 -> 0.30; 150,001 Plummer points forces 2.13 -> 1.30, adjoint 5.4 ->
+// 3.4; 2^20 Plummer points quadrupole forces 11.1 -> 9.8, second-moment adjoint
+// 24.6 -> 22.7, quadrupole adjoint 32.8 -> 30.0 ms.  Teams of 4 waves were slower
+// than of 8 everywhere (2^20 Plummer points: adjoint 23.7 against 22.6), shares
+// that are contiguous pieces of the lists up to 5% slower (they balance worse).
+constexpr int kShares = 16;
+constexpr int kTeamWidth = 512;
+constexpr int kTeamFar = 1024;        // the lists are evaluated from here on
+// Leaf list and stack (see kStackSoft).  Walks that give forces share their
+// sizes, which enter the sums; with six sums per share two blocks of 8 waves
+// just fit on a CU.  The others evaluate less often.
+template <bool FORCES>
+constexpr int kTeamNear = FORCES ? 256 : 512;
+template <bool FORCES>
+constexpr int kTeamSoft = FORCES ? 2048 : 3072;
+constexpr int kTeamLeaves = 4;
+constexpr int kTeamBig = 128;         // a leaf of more sources is dealt 64 sources at a time
+template <int ORDER>
+constexpr int kTeamRun = ORDER == 2 ? kChunk : 2 * kChunk;
+
+template <bool VJP, int ORDER, bool FORCES, int TEAM>
+__global__ __launch_bounds__(64 * TEAM) __attribute__((amdgpu_waves_per_eu(VJP ? 4 : 8))) void
+k_walk_team(WalkArgs A) {
+  static_assert(64 * TEAM >= kTeamWidth && kShares % TEAM == 0, "team size");
+  constexpr int kVals = (FORCES ? 3 : 0) + (VJP ? 3 : 0);
+  constexpr int kPer = kTeamRun<ORDER>;
+  constexpr int C = (VJP && ORDER != 1) ? kChunk / 2 : (!VJP && ORDER == 1) ? kPer : kChunk;
+  constexpr int kSoft = kTeamSoft<FORCES>, kStack = kSoft + 8 * 24;
+  constexpr int kNear = kTeamNear<FORCES>;
+  __shared__ int s_stack[kStack];
+  __shared__ int s_far[kTeamFar + kTeamWidth + kPer];
+  __shared__ int2 s_near[kNear + kTeamWidth];
+  __shared__ float s_sum[kShares][kVals][64];
+  __shared__ __align__(16) float s_red[TEAM][VJP ? kRedMax * kRedRow : 4];  // adjoint wave sums
+  __shared__ int s_cnt[2][TEAM];
+  __shared__ unsigned long long s_pairs[TEAM];  // statistics
+  __shared__ int s_claim;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int num_groups = A.hdr->num_groups, num_nodes = A.hdr->num_nodes;
+  unsigned long long n_far = 0, n_groups = 0;
+  if (lane == 0) s_pairs[w] = 0;
+  // thread 0 claims groups, one ahead of its use to hide the claim's round
+  // trips: eighth by eighth from the block's own XCD's on (see next_group)
+  int tries = 0;
+  auto claim = [&]() {
+    for (; tries < 8; ++tries) {
+      const int q = (static_cast<int>(blockIdx.x & 7u) + tries) & 7;
+      const int2 r = eighth_range(num_groups, q);
+      const int t = atomicAdd(&A.hdr->tq[q], 1);
+      if (t < (A.small != nullptr ? A.small[q] : r.y - r.x))
+        return A.small != nullptr ? A.order[r.x + t] : r.x + t;
+    }
+    return -1;
+  };
+  if (tid == 0) s_claim = claim();
+  __syncthreads();
+  while (true) {
+    const int g = __builtin_amdgcn_readfirstlane(s_claim);
+    if (g < 0) break;  // at most 8 failing claims: every block reaches this exit
+    const int2 grp = A.groups[g];
+    const int base = __builtin_amdgcn_readfirstlane(grp.x);
+    const int cnt = __builtin_amdgcn_readfirstlane(grp.y);
+    int next = -1;
+    if (tid == 0) next = claim();
+    if (cnt < 1 || cnt > 64 || base < 0 || base + cnt > A.n) {  // corrupt entry
+      __syncthreads();
+      if (tid == 0) s_claim = next;
+      __syncthreads();
+      continue;
+    }
+    const int i = base + lane;
+    const Lane L = load_lane<VJP>(A, base, cnt, lane, s_red[w]);
+    const Box b = wave_box(L.x, L.y, L.z);
+    for (int v = w; v < kShares; v += TEAM)
+      for (int c = 0; c < kVals; ++c) s_sum[v][c][lane] = 0.f;
+    int top = 1, nfar = 0, nnear = 0, iters = 0;
+    bool big = false;
+    if (tid == 0) s_stack[0] = A.nsets > 1 ? set_of(A.offs, A.nsets, base) : 0;
+    __syncthreads();
+    while (true) {
+      // (every node is pushed at most once and each round pops at least one)
+      if (top > 0 && iters++ > num_nodes) top = 0;
+      if (top > 0) {
+        int k = min(kTeamWidth, top);
+        k = min(k, max(1, (kSoft - top) / 7));
+        top -= k;
+        int node = -1, kind = 0, nch = 0, incl = 0;
+        int4 t = make_int4(0, 0, 0, 0);
+        if (w * 64 < k) {  // (waves without a candidate only keep the counts)
+          node = tid < k ? s_stack[top + tid] : -1;
+          const bool have = node >= 0 && node < num_nodes;
+          const int nd = have ? node : 0;
+          const float4 m = A.mp[nd];
+          const float4 gg = A.geo[nd];
+          t = A.topo[nd];
+          if (have && m.w != 0.0f) {
+            if (group_accept(b.lx, b.ly, b.lz, b.hx, b.hy, b.hz, gg, A.beta))
+              kind = 1;
+            else if (t.w == 0)
+              kind = 2;
+            else
+              nch = t.w;
+          }
+          incl = wave_incl_scan(nch);
+        }
+        // per wave: accepted nodes | near leaves << 11; children | any large
+        // leaf << 14 (sums over the waves stay below 2^24)
+        const uint64_t bf = __ballot(kind == 1), bn = __ballot(kind == 2);
+        const int large = __ballot(kind == 2 && t.y > kTeamBig) != 0 ? 1 : 0;
+        if (lane == 63) {
+          s_cnt[0][w] = __popcll(bf) | __popcll(bn) << 11;
+          s_cnt[1][w] = incl | large << 14;
+        }
+        __syncthreads();  // the popped entries are read, the counts written
+        const int sum0 = wave_incl_scan(lane < TEAM ? s_cnt[0][lane] : 0);
+        const int sum1 = wave_incl_scan(lane < TEAM ? s_cnt[1][lane] : 0);
+        const int all0 = __builtin_amdgcn_readlane(sum0, TEAM - 1);
+        const int all1 = __builtin_amdgcn_readlane(sum1, TEAM - 1);
+        const int pre0 = w > 0 ? __builtin_amdgcn_readlane(sum0, w - 1) : 0;
+        const int pre1 = w > 0 ? __builtin_amdgcn_readlane(sum1, w - 1) : 0;
+        if (kind == 1) s_far[nfar + (pre0 & 2047) + lanes_below(bf)] = node;
+        if (kind == 2) s_near[nnear + (pre0 >> 11) + lanes_below(bn)] = make_int2(t.x, t.y);
+        nfar += all0 & 2047;
+        nnear += all0 >> 11;
+        big |= (all1 >> 14) != 0;
+        const int pushed = all1 & 16383;
+        if (top + pushed > kStack) {  // unreachable for depth <= 10
+          if (tid == 0) atomicOr(&A.hdr->overflow, 4);
+          top = 0;
+        } else {
+          int* dst = s_stack + (top + (pre1 & 16383) + incl - nch);
+          for (int c = 0; c < nch; ++c) dst[c] = t.z + c;
+          top += pushed;
+        }
+        __syncthreads();  // entries and lists written, the counts read
+      }
+      if (top > 0 && nfar < kTeamFar && nnear < kNear) continue;
+      // evaluate the lists
+      if (w == 0) n_far += static_cast<unsigned long long>(nfar) * cnt;
+      const int runs = (nfar + kPer - 1) / kPer;
+      if (tid < runs * kPer - nfar) s_far[nfar + tid] = A.sentinel;
+      __syncthreads();
+#pragma unroll 1
+      for (int v = w; v < kShares; v += TEAM) {
+        float fx = 0.f, fy = 0.f, fz = 0.f, gx = 0.f, gy = 0.f, gz = 0.f;
+#pragma unroll 1
+        for (int run = v; run < runs; run += kShares)
+#pragma unroll 1
+          for (int f0 = run * kPer; f0 < (run + 1) * kPer; f0 += C)
+            far_batch<VJP, ORDER, FORCES, C>(A, L, s_far + f0, lane, fx, fy, fz, gx, gy, gz);
+        unsigned long long pairs = 0;
+        // runs of the share's leaves, adjoining ones as one range
+#pragma unroll 1
+        for (int e0 = v * kTeamLeaves; e0 < nnear; e0 += kShares * kTeamLeaves) {
+          const int e_end = min(e0 + kTeamLeaves, nnear);
+          int e = e0;
+          while (e < e_end) {
+            const int s0 = __builtin_amdgcn_readfirstlane(s_near[e].x);
+            int s1 = s0;
+            do {
+              const int c = __builtin_amdgcn_readfirstlane(s_near[e].y);
+              if (c > kTeamBig) break;
+              s1 += c;
+              ++e;
+            } while (e < e_end && __builtin_amdgcn_readfirstlane(s_near[e].x) == s1);
+            if (s1 == s0) {  // a large leaf (leaves are not empty): dealt below
+              ++e;
+              continue;
+            }
+            near_range<VJP, ORDER, FORCES>(A, L, i, base, cnt, s0, s1, lane, fx, fy, fz, gx, gy,
+                                           gz, pairs);
+          }
+        }
+        // large leaves (points that share a cell at the depth limit, or a large
+        // leaf size), 64 sources at a time
+#pragma unroll 1
+        for (int e = 0; big && e < nnear; ++e) {
+          const int s0 = __builtin_amdgcn_readfirstlane(s_near[e].x);
+          const int s1 = s0 + __builtin_amdgcn_readfirstlane(s_near[e].y);
+          if (s1 - s0 <= kTeamBig) continue;
+#pragma unroll 1
+          for (int j = s0 + 64 * v; j < s1; j += 64 * kShares)
+            near_range<VJP, ORDER, FORCES>(A, L, i, base, cnt, j, min(j + 64, s1), lane, fx, fy,
+                                           fz, gx, gy, gz, pairs);
+        }
+        if (lane == 0) s_pairs[w] += pairs;
+        float* sum = &s_sum[v][0][lane];
+        if constexpr (FORCES) {
+          sum[0] += fx;
+          sum[64] += fy;
+          sum[128] += fz;
+        }
+        if constexpr (VJP) {
+          constexpr int o = FORCES ? 192 : 0;
+          sum[o] += gx;
+          sum[o + 64] += gy;
+          sum[o + 128] += gz;
+        }
+      }
+      nfar = nnear = 0;
+      big = false;
+      __syncthreads();  // the lists are read, the sums written
+      if (top == 0) break;
+    }
+    if (w < kVals && lane < cnt) {
+      float v = 0.f;
+      for (int k = 0; k < kShares; ++k) v += s_sum[k][w][lane];
+      if (FORCES && w < 3)
+        A.forces[3 * static_cast<int64_t>(A.perm[i]) + w] = v;
+      else
+        reinterpret_cast<float*>(A.qgrad)[4 * static_cast<int64_t>(i) + (w % 3)] = v;
+    }
+    ++n_groups;
+    if (tid == 0) s_claim = next;
+    __syncthreads();  // the sums are read, the claim written
+  }
+  if (A.stats != nullptr && lane == 0) {
+    if (w == 0) {
+      atomicAdd(&A.stats[0], n_far);
+      atomicAdd(&A.stats[2], n_groups);
+    }
+    atomicAdd(&A.stats[1], s_pairs[w]);
   }
 }
 
@@ -1712,25 +2008,37 @@ int build_forest(hipStream_t s, char* ws, const Layout& L, const float* pts, con
 }
 
 namespace {
-template <int WPB>
-void launch_walk(hipStream_t s, unsigned grid, bool vjp, int order, bool f, const WalkArgs& A) {
-  const unsigned block = 64 * WPB;
+template <int TEAM>
+void launch_team(hipStream_t s, unsigned grid, bool vjp, int order, bool f, const WalkArgs& A) {
+
+  const unsigned block = 64 * TEAM;
   if (vjp && order == 2 && f)
-    k_walk<true, 2, true, WPB><<<grid, block, 0, s>>>(A);
+    k_walk_team<true, 2, true, TEAM><<<grid, block, 0, s>>>(A);
   else if (vjp && order == 2)
-    k_walk<true, 2, false, WPB><<<grid, block, 0, s>>>(A);
+    k_walk_team<true, 2, false, TEAM><<<grid, block, 0, s>>>(A);
   else if (vjp && order == 3 && f)
-    k_walk<true, 3, true, WPB><<<grid, block, 0, s>>>(A);
+    k_walk_team<true, 3, true, TEAM><<<grid, block, 0, s>>>(A);
   else if (vjp && order == 3)
-    k_walk<true, 3, false, WPB><<<grid, block, 0, s>>>(A);
+    k_walk_team<true, 3, false, TEAM><<<grid, block, 0, s>>>(A);
   else if (vjp && f)
-    k_walk<true, 1, true, WPB><<<grid, block, 0, s>>>(A);
+    k_walk_team<true, 1, true, TEAM><<<grid, block, 0, s>>>(A);
   else if (vjp)
-    k_walk<true, 1, false, WPB><<<grid, block, 0, s>>>(A);
+    k_walk_team<true, 1, false, TEAM><<<grid, block, 0, s>>>(A);
   else if (order == 2)
-    k_walk<false, 2, true, WPB><<<grid, block, 0, s>>>(A);
+    k_walk_team<false, 2, true, TEAM><<<grid, block, 0, s>>>(A);
   else
-    k_walk<false, 1, true, WPB><<<grid, block, 0, s>>>(A);
+    k_walk_team<false, 1, true, TEAM><<<grid, block, 0, s>>>(A);
+}
+
+template <int WPB>
+void launch_walk(hipStream_t s, unsigned grid, bool vjp, bool f, const WalkArgs& A) {
+  const unsigned block = 64 * WPB;
+  if (vjp && f)
+    k_walk<true, true, WPB><<<grid, block, 0, s>>>(A);
+  else if (vjp)
+    k_walk<true, false, WPB><<<grid, block, 0, s>>>(A);
+  else
+    k_walk<false, true, WPB><<<grid, block, 0, s>>>(A);
 }
 }  // namespace
 
@@ -1741,7 +2049,9 @@ int schedule_groups(hipStream_t s, char* ws, const Layout& L, int64_t n, int kin
   const int64_t nn = n > 0 ? n : 1, own = kind != 0 ? 1 : 0;
   *order = reinterpret_cast<const int*>(ws + L.gorder);
   *cost = costs + own * nn;
-  k_group_order<<<8, 1024, 0, s>>>(reinterpret_cast<const Header*>(ws + L.header), *cost,
+  k_group_order<<<8, 1024, 0, s>>>(reinterpret_cast<Header*>(ws + L.header),
+                                   reinterpret_cast<const int32_t*>(ws + L.offs), L.nsets,
+                                   reinterpret_cast<const int2*>(ws + L.groups), *cost,
                                    costs + (1 - own) * nn, reinterpret_cast<int*>(ws + L.gorder),
                                    tags + own, tags + (1 - own));
   SBH_LAUNCH_CHECK();
@@ -1776,34 +2086,58 @@ int walk(hipStream_t s, char* ws, const Layout& L, int64_t n, float beta, float 
   A.adj = reinterpret_cast<float*>(ws + L.adj);
   A.adjq = reinterpret_cast<float*>(ws + L.adjq);
   A.stats = want_stats ? hdr->stats : nullptr;
-  {
-    const int* order = nullptr;
+  // teams walk every set, except with monopole terms those of kSinglePoints
+  // and more (a forest may hold both kinds)
+  const bool singles = order == 1 && n >= kSinglePoints;
+  const bool teams = !singles || L.nsets > 1;
+  A.order = nullptr;
+  A.gcost = nullptr;
+  A.small = nullptr;
+  if (singles) {
+    const int* claims = nullptr;
     float* cost = nullptr;
-    const int rc = schedule_groups(s, ws, L, n, vjp ? 1 : 0, &order, &cost);
+    const int rc = schedule_groups(s, ws, L, n, vjp ? 1 : 0, &claims, &cost);
     if (rc != SBH_OK) return rc;
-    A.order = order;
+    A.order = claims;
     A.gcost = cost;
+    if (L.nsets > 1) A.small = hdr->small;
   }
-  SBH_LAUNCH_CHECK();
   if (vjp) {
     k_zero_adjoint<<<grid_for(4 * n + 12 * L.cap, kB, 8192), kB, 0, s>>>(hdr, n, A.sgrad, A.adj,
                                                                         A.adjq);
     SBH_LAUNCH_CHECK();
   }
-  // Persistent waves drain the group queue: 8192 waves by default (8 per
-  // SIMD, twice what fits at once, so that every CU stays busy to the end),
-  // never more than one wave per point.
-  const int threads = walk_threads > 0 ? walk_threads : kB;
-  const int wpb = threads / 64;
-  const int64_t waves_cap = walk_blocks > 0 ? static_cast<int64_t>(walk_blocks) * wpb : 8192;
-  unsigned grid = grid_for(n, 64 * wpb, static_cast<unsigned>((waves_cap + wpb - 1) / wpb));
   if (ev_walk != nullptr) SBH_HIP_TRY(hipEventRecord(ev_walk[0], s));
   const bool f = forces != nullptr;
-  switch (wpb) {
-    case 1: launch_walk<1>(s, grid, vjp, order, f, A); break;
-    case 2: launch_walk<2>(s, grid, vjp, order, f, A); break;
-    case 8: launch_walk<8>(s, grid, vjp, order, f, A); break;
-    default: launch_walk<4>(s, grid, vjp, order, f, A); break;
+  if (teams) {
+    // persistent blocks: two (adjoint) or four (forward) of 8 waves fit on a
+    // CU, half as many of 16
+    const bool wide = n < kWidePoints;
+    unsigned cap = vjp ? 512 : 1024;
+    if (wide) cap /= 2;
+    if (walk_blocks > 0) cap = std::min(cap, static_cast<unsigned>(walk_blocks));
+    const unsigned grid = grid_for(n, 16, cap);
+    if (wide)
+      launch_team<16>(s, grid, vjp, order, f, A);
+    else
+      launch_team<8>(s, grid, vjp, order, f, A);
+    SBH_LAUNCH_CHECK();
+  }
+  if (singles) {
+    // Persistent waves drain the group queue: 8192 waves by default (8 per
+    // SIMD, so that every CU stays busy to the end), never more than one wave
+    // per point.
+    const int threads = walk_threads > 0 ? walk_threads : kB;
+    const int wpb = threads / 64;
+    const int64_t waves_cap = walk_blocks > 0 ? static_cast<int64_t>(walk_blocks) * wpb : 8192;
+    const unsigned grid =
+        grid_for(n, 64 * wpb, static_cast<unsigned>((waves_cap + wpb - 1) / wpb));
+    switch (wpb) {
+      case 1: launch_walk<1>(s, grid, vjp, f, A); break;
+      case 2: launch_walk<2>(s, grid, vjp, f, A); break;
+      case 8: launch_walk<8>(s, grid, vjp, f, A); break;
+      default: launch_walk<4>(s, grid, vjp, f, A); break;
+    }
   }
   SBH_LAUNCH_CHECK();
   if (ev_walk != nullptr) SBH_HIP_TRY(hipEventRecord(ev_walk[1], s));

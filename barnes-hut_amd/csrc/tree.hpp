@@ -28,6 +28,8 @@ struct Header {
   int32_t queue;       // unused by the walks (kept zero)
   int32_t xq[8];       // per-XCD work queues: next group of each eighth of the groups
   unsigned long long stats[8];  // far interactions, near pairs, groups
+  int32_t small[8];    // per eighth: groups of sets below kSinglePoints, dealt to the teams
+  int32_t tq[8];       // the teams' work queues, as xq
 };
 
 // Tag of the walk schedule: the group costs in the workspace were measured
@@ -39,6 +41,13 @@ struct Sched {
   int32_t groups;
 };
 
+// Sets from which single waves walk the groups with monopole terms (k_walk).
+constexpr int kSinglePoints = 700000;
+// Calls with fewer points use teams of 16 waves, which fill more of the chip
+// with the few groups there are (10,000 points: fwd 0.21 against 0.26 ms,
+// second-moment adjoint 0.29 / 0.35), others teams of 8, of which more fit
+// (100,000 points: forward 0.61 against 0.64 ms; 2^20: 7.1 / 9.2).
+constexpr int kWidePoints = 98304;
 constexpr int kGroupMax = 64;     // one wavefront per query group
 constexpr int kGroupCell = 2048;  // groups are runs inside cells of at most this many points
 // Query trees (queries walked against a separate source tree): topology and
