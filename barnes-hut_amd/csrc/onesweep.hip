@@ -10,7 +10,7 @@
 //                ticket, counts the tile's digits, publishes them, looks back
 //                over the earlier tiles' published counts (decoupled look-back)
 //                for its exclusive prefix per digit, ranks the tile's keys in
-//                (round, wave, lane) order (which keeps the sort stable),
+//                (wave, round, lane) order (which keeps the sort stable),
 //                stages them in LDS sorted by digit and writes them out so
 //                that consecutive threads fill consecutive slots of a digit
 //
@@ -30,13 +30,20 @@
 namespace sbh {
 namespace {
 
-constexpr int kBlock = 256;
-constexpr int kItems = 8;
-constexpr int kTile = kBlock * kItems;  // 2048 keys per tile
+constexpr int kBlock = 512;
+// Keys per thread: a tile of kBlock items(n) keys.  A pass waits for one key's
+// ranking after another, so few keys are better with few tiles; the look-back
+// reads grow with the square of the tiles, which bounds large sorts: 10^4
+// keys 7 us a pass with 2 and 12 with 8 (2^20 keys: 21 with 8, 27 with 2048 keys a
+// tile).
+constexpr int kMaxItems = 8;
+int items_for(int64_t n) { return n <= (int64_t{1} << 15) ? 2 : n <= (int64_t{1} << 17) ? 4 : 8; }
 constexpr int kRadix = 256;
 constexpr int kWaves = kBlock / 64;
 constexpr int kHistBlocks = 128;
+constexpr int kHistBlock = 1024;
 constexpr int kMaxPasses = 8;
+constexpr int kBack = 16;  // tiles looked back over per round trip
 constexpr uint32_t kAgg = 1u << 30;    // status: tile count published
 constexpr uint32_t kIncl = 2u << 30;   // status: inclusive prefix published
 constexpr uint32_t kValue = (1u << 30) - 1u;
@@ -52,7 +59,8 @@ struct OsLayout {
 
 OsLayout os_layout(int64_t n, int passes) {
   auto align = [](size_t x) { return (x + 255) & ~size_t{255}; };
-  const size_t tiles = static_cast<size_t>((n + kTile - 1) / kTile);
+  const int64_t tile = static_cast<int64_t>(kBlock) * items_for(n);
+  const size_t tiles = static_cast<size_t>((n + tile - 1) / tile);
   OsLayout L;
   size_t o = 0;
   L.hist = o; o = align(o + 4ull * kHistBlocks * kMaxPasses * kRadix);
@@ -71,7 +79,10 @@ __device__ __forceinline__ int row_set(const int32_t* __restrict__ set_offs, int
 // Per-block digit histograms of every pass: code passes from the codes, set
 // passes from the set of each row (the same set_of the passes use, so the
 // counts match the digits scattered whatever the offsets hold).
-__global__ __launch_bounds__(kBlock) void k_os_hist(const uint32_t* __restrict__ codes, int64_t n,
+// Blocks of kHistBlock threads: the reads are few and each is followed by LDS
+// adds (and a search for the row's set), so it takes many waves to hide them.
+// 2^20 keys 7 us, 2.3e6 rows of 48 sets 19 (blocks of 256: 15 and 48).
+__global__ __launch_bounds__(kHistBlock) void k_os_hist(const uint32_t* __restrict__ codes, int64_t n,
                                                     int code_passes, int set_passes,
                                                     const int32_t* __restrict__ set_offs,
                                                     int nsets, uint32_t* __restrict__ hist,
@@ -79,10 +90,10 @@ __global__ __launch_bounds__(kBlock) void k_os_hist(const uint32_t* __restrict__
                                                     int64_t status_words) {
   __shared__ uint32_t cnt[kMaxPasses][kRadix];
   const int passes = code_passes + set_passes;
-  for (int p = 0; p < passes; ++p) cnt[p][threadIdx.x] = 0;
+  for (int p = threadIdx.x; p < kMaxPasses * kRadix; p += kHistBlock) cnt[p / kRadix][p % kRadix] = 0;
   __syncthreads();
-  for (int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x; i < n;
-       i += static_cast<int64_t>(gridDim.x) * kBlock) {
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * kHistBlock + threadIdx.x; i < n;
+       i += static_cast<int64_t>(gridDim.x) * kHistBlock) {
     const uint32_t k = codes[i];
     for (int p = 0; p < code_passes; ++p) atomicAdd(&cnt[p][(k >> (8 * p)) & 255u], 1u);
     if (set_passes > 0) {
@@ -91,80 +102,83 @@ __global__ __launch_bounds__(kBlock) void k_os_hist(const uint32_t* __restrict__
         atomicAdd(&cnt[code_passes + q][(sid >> (8 * q)) & 255u], 1u);
     }
   }
-  for (int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x; i < status_words;
-       i += static_cast<int64_t>(gridDim.x) * kBlock)
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * kHistBlock + threadIdx.x; i < status_words;
+       i += static_cast<int64_t>(gridDim.x) * kHistBlock)
     status[i] = 0u;
   __syncthreads();
-  for (int p = 0; p < passes; ++p)
-    hist[(static_cast<int64_t>(blockIdx.x) * kMaxPasses + p) * kRadix + threadIdx.x] =
-        cnt[p][threadIdx.x];
+  for (int p = threadIdx.x; p < passes * kRadix; p += kHistBlock)
+    hist[static_cast<int64_t>(blockIdx.x) * kMaxPasses * kRadix + p] = cnt[p / kRadix][p % kRadix];
 }
 
-// Global exclusive digit offsets of every pass; resets the tile tickets.
-// Thread (quarter q, digit d) sums a quarter of the block histograms.
+// Global exclusive digit offsets, one block per pass; resets the pass's tile
+// ticket.  Thread (quarter q, digit d) sums a quarter of the block histograms;
+// the digits are then scanned in four waves.  (One block for all passes took
+// 12.5 us for four, whatever n.)
 __global__ __launch_bounds__(4 * kRadix) void k_os_offsets(const uint32_t* __restrict__ hist,
-                                                           int passes,
+                                                           int blocks,
                                                            uint32_t* __restrict__ offs,
                                                            uint32_t* __restrict__ ticket) {
   __shared__ uint32_t part[4][kRadix];
-  __shared__ uint32_t sh[kRadix];
+  __shared__ uint32_t s_wave[4];
   const int d = threadIdx.x & (kRadix - 1), q = threadIdx.x / kRadix;
-  constexpr int kPer = kHistBlocks / 4;
-  for (int p = 0; p < passes; ++p) {
-    uint32_t c = 0;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, p = blockIdx.x;
+  uint32_t c = 0;
 #pragma unroll 8
-    for (int b = q * kPer; b < (q + 1) * kPer; ++b)
-      c += hist[(static_cast<int64_t>(b) * kMaxPasses + p) * kRadix + d];
-    part[q][d] = c;
-    __syncthreads();
-    if (q == 0) {
-      const uint32_t tot = part[0][d] + part[1][d] + part[2][d] + part[3][d];
-      // exclusive scan of the 256 digit counts (one block-level scan per pass)
-      sh[d] = tot;
-      part[0][d] = tot;
-    }
-    __syncthreads();
-    for (int off = 1; off < kRadix; off <<= 1) {
-      uint32_t v = 0;
-      if (q == 0 && d >= off) v = sh[d - off];
-      __syncthreads();
-      if (q == 0) sh[d] += v;
-      __syncthreads();
-    }
-    if (q == 0) offs[p * kRadix + d] = sh[d] - part[0][d];
-    __syncthreads();
+  for (int b = q; b < blocks; b += 4)
+    c += hist[(static_cast<int64_t>(b) * kMaxPasses + p) * kRadix + d];
+  part[q][d] = c;
+  __syncthreads();
+  const uint32_t tot = part[0][d] + part[1][d] + part[2][d] + part[3][d];
+  uint32_t incl = tot;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t t = __shfl_up(incl, o, 64);
+    if (lane >= o) incl += t;
   }
-  if (threadIdx.x < kMaxPasses) ticket[threadIdx.x] = 0u;
+  if (lane == 63 && w < 4) s_wave[w] = incl;
+  __syncthreads();
+  if (q == 0) {
+    uint32_t before = 0;
+    for (int k = 0; k < w; ++k) before += s_wave[k];
+    offs[p * kRadix + d] = before + incl - tot;
+  }
+  if (threadIdx.x == 0) ticket[p] = 0u;
 }
 
 // One digit pass: (key, value) pairs move to their sorted slots.  The digit
 // is a byte of the key (code pass) or of the set holding the row (set pass);
-// on the first pass vals_in == nullptr makes the values the rows.
-template <bool SET_PASS>
+// on the first pass vals_in == nullptr makes the values the rows.  A wave ranks
+// a run of 64 kItems consecutive keys of the tile by itself, round after round,
+// with counts of its own in LDS, and the waves' counts are joined once; with
+// rounds across the block and three barriers in each a pass over one tile took 9.5
+// us instead of 7.
+template <bool SET_PASS, int kItems>
 __global__ __launch_bounds__(kBlock) void k_os_pass(
     const uint32_t* __restrict__ keys_in, const uint32_t* __restrict__ vals_in, int64_t n,
     int shift, const uint32_t* __restrict__ offs, uint32_t* __restrict__ ticket,
     uint32_t* __restrict__ status, const int32_t* __restrict__ set_offs, int nsets,
     uint32_t* __restrict__ keys_out, uint32_t* __restrict__ vals_out, int32_t* __restrict__ flag) {
+  constexpr int kTile = kBlock * kItems;
   __shared__ uint32_t s_tile;
-  __shared__ uint32_t s_count[kRadix];
   __shared__ uint32_t s_base[kRadix];
   __shared__ uint32_t s_lstart[kRadix];
   __shared__ uint32_t s_wcnt[kWaves][kRadix];
+  __shared__ uint32_t s_wave[kWaves];
   __shared__ uint32_t s_key[kTile];
   __shared__ uint32_t s_val[kTile];
   __shared__ uint8_t s_dig[kTile];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
   if (tid == 0) s_tile = atomicAdd(ticket, 1u);
-  s_count[tid] = 0u;
+  for (int k = tid; k < kWaves * kRadix; k += kBlock) (&s_wcnt[0][0])[k] = 0u;
   __syncthreads();
   const uint32_t tile = s_tile;
   const int64_t base = static_cast<int64_t>(tile) * kTile;
+  const int64_t run = base + wave * (64 * kItems) + lane;
   uint32_t key[kItems], val[kItems], dig[kItems], loc[kItems];
 #pragma unroll
   for (int r = 0; r < kItems; ++r) {
-    const int64_t i = base + r * kBlock + tid;
+    const int64_t i = run + r * 64;
     const bool ok = i < n;
     key[r] = (ok && keys_in != nullptr) ? keys_in[i] : 0u;
     val[r] = ok ? (vals_in != nullptr ? vals_in[i] : static_cast<uint32_t>(i)) : 0u;
@@ -174,12 +188,11 @@ __global__ __launch_bounds__(kBlock) void k_os_pass(
     else
       dig[r] = ok ? (key[r] >> shift) & 255u : kRadix;
   }
-  // rank the keys in (round, wave, lane) order: loc = the key's offset among
-  // the tile's keys of its digit; s_count accumulates the tile's counts
+  // rank the keys in (wave, round, lane) order, the input's: loc = the key's
+  // offset among its wave's keys of the digit.  Only this wave touches its counts
+  // here, and its LDS operations complete in order.
 #pragma unroll
   for (int r = 0; r < kItems; ++r) {
-    for (int w = 0; w < kWaves; ++w) s_wcnt[w][tid] = 0u;
-    __syncthreads();
     const bool ok = dig[r] < kRadix;
     uint64_t peers = __ballot(ok);
 #pragma unroll
@@ -189,58 +202,68 @@ __global__ __launch_bounds__(kBlock) void k_os_pass(
       peers &= bit ? bal : ~bal;
     }
     const uint32_t rank = static_cast<uint32_t>(__popcll(peers & lt));
-    if (ok && rank == 0) s_wcnt[wave][dig[r]] = static_cast<uint32_t>(__popcll(peers));
-    __syncthreads();
-    if (ok) {
-      uint32_t lp = s_count[dig[r]] + rank;
-      for (int w = 0; w < wave; ++w) lp += s_wcnt[w][dig[r]];
-      loc[r] = lp;
-    }
-    __syncthreads();
-    uint32_t add = 0;
-    for (int w = 0; w < kWaves; ++w) add += s_wcnt[w][tid];
-    s_count[tid] += add;
+    const uint32_t have = ok ? s_wcnt[wave][dig[r]] : 0u;
+    loc[r] = have + rank;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (ok && rank == 0) s_wcnt[wave][dig[r]] = have + static_cast<uint32_t>(__popcll(peers));
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
   }
   __syncthreads();
+  // counts of the tile per digit; each wave's become the keys before its own
+  const bool digit = tid < kRadix;  // the first kRadix threads: one per digit
+  uint32_t mine = 0;
+  if (digit) {
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      const uint32_t c = s_wcnt[w][tid];
+      s_wcnt[w][tid] = mine;
+      mine += c;
+    }
+  }
   // publish this tile's counts, then look back for the exclusive prefix
   uint32_t* st = status + static_cast<int64_t>(tile) * kRadix;
-  const uint32_t mine = s_count[tid];
-  __hip_atomic_store(st + tid, kAgg | mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  // look back 8 tiles per round trip: the 8 status words are loaded
-  // together, then consumed nearest first (aggregates added) up to the first
-  // inclusive prefix; a word not yet published is re-read until it is
+  if (digit)
+    __hip_atomic_store(st + tid, kAgg | mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  // look back kBack tiles per round trip: their status words are loaded
+  // together and the published ones consumed nearest first (aggregates added) up
+  // to the first inclusive prefix; from the first not yet published, again
   uint32_t excl = 0;
-  bool done = false;
-  for (int64_t k = static_cast<int64_t>(tile) - 1; k >= 0 && !done; k -= 8) {
-    uint32_t v[8];
+  int spins = 0;
+  bool done = !digit;
+  for (int64_t k = static_cast<int64_t>(tile) - 1; k >= 0 && !done;) {
+    uint32_t v[kBack];
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
+    for (int j = 0; j < kBack; ++j)
       v[j] = k - j >= 0 ? __hip_atomic_load(status + (k - j) * kRadix + tid, __ATOMIC_RELAXED,
                                             __HIP_MEMORY_SCOPE_AGENT)
                         : kIncl;
+    bool ready = true;
+    int used = 0;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      if (done || k - j < 0) break;
-      uint32_t x = v[j];
-      int spins = 0;
-      while ((x & ~kValue) == 0u && spins < kSpinLimit) {
-        __builtin_amdgcn_s_sleep(1);
-        x = __hip_atomic_load(status + (k - j) * kRadix + tid, __ATOMIC_RELAXED,
-                              __HIP_MEMORY_SCOPE_AGENT);
-        ++spins;
-      }
-      if ((x & ~kValue) == 0u) {
+    for (int j = 0; j < kBack; ++j) {
+      ready = ready && !done && (v[j] & ~kValue) != 0u;
+      excl += ready ? v[j] & kValue : 0u;
+      used += ready ? 1 : 0;
+      done = done || (ready && (v[j] & kIncl) != 0u);
+    }
+    k -= used;
+    if (used == 0) {
+      if (++spins >= kSpinLimit) {
         atomicOr(flag, 1 << 16);
-        done = true;
         break;
       }
-      excl += x & kValue;
-      if (x & kIncl) done = true;
+      __builtin_amdgcn_s_sleep(1);
+    } else {
+      spins = 0;
     }
   }
-  __hip_atomic_store(st + tid, kIncl | ((excl + mine) & kValue), __ATOMIC_RELAXED,
-                     __HIP_MEMORY_SCOPE_AGENT);
-  s_base[tid] = offs[tid] + excl;
+  if (digit) {
+    __hip_atomic_store(st + tid, kIncl | ((excl + mine) & kValue), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+    s_base[tid] = offs[tid] + excl;
+  }
   // local start of each digit inside the tile (exclusive scan of the counts)
   {
     uint32_t incl = mine;
@@ -248,18 +271,18 @@ __global__ __launch_bounds__(kBlock) void k_os_pass(
       const uint32_t t = __shfl_up(incl, d, 64);
       if (lane >= d) incl += t;
     }
-    if (lane == 63) s_wcnt[0][wave] = incl;
+    if (lane == 63) s_wave[wave] = incl;
     __syncthreads();
     uint32_t before = 0;
-    for (int w = 0; w < wave; ++w) before += s_wcnt[0][w];
-    s_lstart[tid] = before + incl - mine;
+    for (int w = 0; w < wave; ++w) before += s_wave[w];
+    if (digit) s_lstart[tid] = before + incl - mine;
     __syncthreads();
   }
   // stage the tile in LDS sorted by digit (stable: loc keeps the order)
 #pragma unroll
   for (int r = 0; r < kItems; ++r) {
     if (dig[r] < kRadix) {
-      const uint32_t lp = s_lstart[dig[r]] + loc[r];
+      const uint32_t lp = s_lstart[dig[r]] + s_wcnt[wave][dig[r]] + loc[r];
       s_key[lp] = key[r];
       s_val[lp] = val[r];
       s_dig[lp] = static_cast<uint8_t>(dig[r]);
@@ -304,12 +327,16 @@ int morton_sort(hipStream_t s, const uint32_t* codes, int64_t n, int key_bits,
   auto* offs = reinterpret_cast<uint32_t*>(t + L.offs);
   auto* ticket = reinterpret_cast<uint32_t*>(t + L.ticket);
   auto* status = reinterpret_cast<uint32_t*>(t + L.status);
-  const int64_t tiles = (n + kTile - 1) / kTile;
-  k_os_hist<<<kHistBlocks, kBlock, 0, s>>>(codes, n, code_passes, set_passes, set_offs, nsets,
+  const int items = items_for(n);
+  const int64_t tile = static_cast<int64_t>(kBlock) * items;
+  const int64_t tiles = (n + tile - 1) / tile;
+  const int blocks = static_cast<int>(
+      std::min<int64_t>(kHistBlocks, (n + kHistBlock - 1) / kHistBlock));
+  k_os_hist<<<blocks, kHistBlock, 0, s>>>(codes, n, code_passes, set_passes, set_offs, nsets,
                                             hist, status,
                                             static_cast<int64_t>(passes) * tiles * kRadix);
   SBH_LAUNCH_CHECK();
-  k_os_offsets<<<1, 4 * kRadix, 0, s>>>(hist, passes, offs, ticket);
+  k_os_offsets<<<passes, 4 * kRadix, 0, s>>>(hist, blocks, offs, ticket);
   SBH_LAUNCH_CHECK();
   const uint32_t* kin = codes;
   const uint32_t* vin = nullptr;
@@ -318,15 +345,18 @@ int morton_sort(hipStream_t s, const uint32_t* codes, int64_t n, int key_bits,
     uint32_t* vout = (p & 1) ? vals_b : vals_a;
     uint32_t* st = status + static_cast<int64_t>(p) * tiles * kRadix;
     // the keys travel through every pass: the last one leaves them sorted
-    if (p < code_passes) {
-      k_os_pass<false><<<static_cast<unsigned>(tiles), kBlock, 0, s>>>(
-          kin, vin, n, 8 * p, offs + p * kRadix, ticket + p, st, set_offs, nsets, kout, vout,
-          flag);
-    } else {
-      k_os_pass<true><<<static_cast<unsigned>(tiles), kBlock, 0, s>>>(
-          kin, vin, n, 8 * (p - code_passes), offs + p * kRadix, ticket + p, st, set_offs, nsets,
-          kout, vout, flag);
-    }
+    const bool set_pass = p >= code_passes;
+    auto pass = [&](auto kernel) {
+      kernel<<<static_cast<unsigned>(tiles), kBlock, 0, s>>>(
+          kin, vin, n, 8 * (set_pass ? p - code_passes : p), offs + p * kRadix, ticket + p, st,
+          set_offs, nsets, kout, vout, flag);
+    };
+    if (items == 2)
+      set_pass ? pass(k_os_pass<true, 2>) : pass(k_os_pass<false, 2>);
+    else if (items == 4)
+      set_pass ? pass(k_os_pass<true, 4>) : pass(k_os_pass<false, 4>);
+    else
+      set_pass ? pass(k_os_pass<true, kMaxItems>) : pass(k_os_pass<false, kMaxItems>);
     SBH_LAUNCH_CHECK();
     kin = kout;
     vin = vout;

@@ -29,7 +29,9 @@
 // position order.
 //
 // Functions here are __host__ __device__ so that the same code can be run on
-// the CPU against the breadth-first builder of the oracle.
+// the CPU against the breadth-first builder of the oracle.  `codes` is anything
+// indexed by the position of a point (an array, or a window of one), I its type
+// (signed).
 #pragma once
 
 #include <cstdint>
@@ -60,11 +62,11 @@ __host__ __device__ inline int common_digits(uint32_t a, uint32_t b, int D) {
 
 // First position e in [lo, hi) with common_digits(codes[r], codes[e]) < l
 // (hi if none); the predicate is monotone over the sorted codes.
-__host__ __device__ inline int64_t run_end(const uint32_t* codes, int64_t r, int64_t lo,
-                                           int64_t hi, int l, int D) {
+template <class I, class Codes>
+__host__ __device__ inline I run_end(const Codes& codes, I r, I lo, I hi, int l, int D) {
   const uint32_t cr = codes[r];
   while (lo < hi) {
-    const int64_t mid = lo + ((hi - lo) >> 1);
+    const I mid = lo + ((hi - lo) >> 1);
     if (common_digits(cr, codes[mid], D) >= l)
       lo = mid + 1;
     else
@@ -74,12 +76,12 @@ __host__ __device__ inline int64_t run_end(const uint32_t* codes, int64_t r, int
 }
 
 // First position k in [lo, r] with common_digits(codes[k], codes[r]) >= l.
-__host__ __device__ inline int64_t run_begin(const uint32_t* codes, int64_t r, int64_t lo,
-                                             int l, int D) {
+template <class I, class Codes>
+__host__ __device__ inline I run_begin(const Codes& codes, I r, I lo, int l, int D) {
   const uint32_t cr = codes[r];
-  int64_t hi = r;
+  I hi = r;
   while (lo < hi) {
-    const int64_t mid = lo + ((hi - lo) >> 1);
+    const I mid = lo + ((hi - lo) >> 1);
     if (common_digits(codes[mid], cr, D) >= l)
       hi = mid;
     else
@@ -91,18 +93,19 @@ __host__ __device__ inline int64_t run_begin(const uint32_t* codes, int64_t r, i
 // Whether the level-l cell holding r (which began before r when r > sb)
 // holds more than `cap` points: the points of the cell before r (at most
 // cap) plus those from r (at most cap + 1) reach cap + 1.
-__host__ __device__ inline bool cell_exceeds(const uint32_t* codes, int64_t r, int64_t sb,
-                                             int64_t se, int l, int D, int64_t cap) {
+template <class I, class Codes>
+__host__ __device__ inline bool cell_exceeds(const Codes& codes, I r, I sb, I se, int l, int D,
+                                             I cap) {
   // quick answer from two probes: with at most h points before r and at
   // most cap - h from r, the cell holds at most cap
-  const int64_t h = cap / 2;
+  const I h = cap / 2;
   const bool few_before = r - h - 1 < sb || common_digits(codes[r - h - 1], codes[r], D) < l;
   const bool few_after = r + cap - h >= se || common_digits(codes[r], codes[r + cap - h], D) < l;
   if (few_before && few_after) return false;
-  const int64_t lo = r - cap > sb ? r - cap : sb;
-  const int64_t before = r - run_begin(codes, r, lo, l, D);
-  const int64_t hi = r + cap + 1 < se ? r + cap + 1 : se;
-  const int64_t from = run_end(codes, r, r + 1, hi, l, D) - r;
+  const I lo = r - cap > sb ? r - cap : sb;
+  const I before = r - run_begin(codes, r, lo, l, D);
+  const I hi = r + cap + 1 < se ? r + cap + 1 : se;
+  const I from = run_end(codes, r, r + 1, hi, l, D) - r;
   return before + from >= cap + 1;
 }
 
@@ -113,8 +116,9 @@ struct PointNodes {
   int top;    // deepest level begun (a leaf); first..top are r's nodes
 };
 
-__host__ __device__ inline PointNodes point_nodes(const uint32_t* codes, int64_t r, int64_t sb,
-                                                  int64_t se, int D, int leaf_size) {
+template <class I, class Codes>
+__host__ __device__ inline PointNodes point_nodes(const Codes& codes, I r, I sb, I se, int D,
+                                                  int leaf_size) {
   PointNodes p;
   p.d = r == sb ? 0 : common_digits(codes[r - 1], codes[r], D);
   p.w = r + leaf_size < se ? common_digits(codes[r], codes[r + leaf_size], D) : -1;
@@ -123,7 +127,7 @@ __host__ __device__ inline PointNodes point_nodes(const uint32_t* codes, int64_t
   if (p.d >= D) return p;
   // the level-d cell holding r is split iff it holds more than leaf_size
   // points (d < D here); the window from r decides it when it fits inside
-  const bool split = p.w >= p.d || cell_exceeds(codes, r, sb, se, p.d, D, leaf_size);
+  const bool split = p.w >= p.d || cell_exceeds<I>(codes, r, sb, se, p.d, D, leaf_size);
   if (!split) return p;
   p.first = p.d + 1;
   const int t = p.w + 1 > p.first ? p.w + 1 : p.first;
@@ -137,9 +141,10 @@ __host__ __device__ inline PointNodes point_nodes(const uint32_t* codes, int64_t
 // kGroupCell points whose parent holds more (a root has no parent), or the
 // deepest (a leaf) when even that holds more.  r's node at `first` has as
 // parent the level-d cell, begun before r unless r == sb (then the root).
-__host__ __device__ inline int group_cell_level(const uint32_t* codes, int64_t r, int64_t sb,
-                                                int64_t se, int D, const PointNodes& p) {
-  const int64_t g = kGroupCell;
+template <class I, class Codes>
+__host__ __device__ inline int group_cell_level(const Codes& codes, I r, I sb, I se, int D,
+                                                const PointNodes& p) {
+  const I g = kGroupCell;
   // r's cell at level l (one of its nodes, or the root) holds more than g
   // points iff the run from r does: iff l <= wg
   const int wg = r + g < se ? common_digits(codes[r], codes[r + g], D) : -1;
@@ -152,7 +157,7 @@ __host__ __device__ inline int group_cell_level(const uint32_t* codes, int64_t r
   if (l > p.top) return p.top;  // every node of r holds more than g: over-full leaf
   if (l > p.first || r == sb) return l;  // parent: r's node at l - 1, or the root
   // l == first: the parent is the level-d cell begun before r
-  return cell_exceeds(codes, r, sb, se, p.d, D, g) ? l : -1;
+  return cell_exceeds<I>(codes, r, sb, se, p.d, D, g) ? l : -1;
 }
 
 }  // namespace topo

@@ -65,8 +65,8 @@ __global__ __launch_bounds__(kB) void k_bbox_partial(const float* __restrict__ p
 
 // Reduces the per-block partials: bounds[0..3) = min - 1e-3, bounds[3..6) =
 // max + 1e-3 (python/jax_sbh_ffi.py:879-884); an empty set gives +-1e-3.
-__global__ __launch_bounds__(kB) void k_bbox_reduce(const float* __restrict__ part, int nparts,
-                                                    int64_t n, float* __restrict__ bounds) {
+__device__ __forceinline__ void bbox_reduce(const float* __restrict__ part, int nparts, int64_t n,
+                                            float* bounds) {
   float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
   for (int b = threadIdx.x; b < nparts; b += kB)
     for (int a = 0; a < 3; ++a) {
@@ -95,6 +95,11 @@ __global__ __launch_bounds__(kB) void k_bbox_reduce(const float* __restrict__ pa
   }
 }
 
+__global__ __launch_bounds__(kB) void k_bbox_reduce(const float* __restrict__ part, int nparts,
+                                                    int64_t n, float* __restrict__ bounds) {
+  bbox_reduce(part, nparts, n, bounds);
+}
+
 // Order-preserving map of floats to unsigned ints (for atomic min / max).
 __device__ __forceinline__ uint32_t f2ord(float f) {
   const uint32_t b = __float_as_uint(f);
@@ -112,8 +117,10 @@ __global__ __launch_bounds__(kB) void k_setbox_init(uint32_t* __restrict__ box, 
 // Per-set data bounds of the input rows (sets are contiguous row ranges).
 // Pass 1: one block per tile of kB consecutive points.  A tile
 // inside one set stores its box in part[6 t ..]; a tile that straddles set
-// boundaries (at most nsets - 1 of them) stores the neutral box and adds its
-// points to the set boxes with ordered-integer atomics.
+// boundaries (at most nsets - 1 of them) stores the neutral box and adds to
+// the set boxes with ordered-integer atomics what a segmented scan over each
+// wave leaves: one box per set and wave.  (One atomic per point and axis, all
+// of a tile on a few words: 101 us for 48 sets of 2.3e6 points in all, now 13.)
 __global__ __launch_bounds__(kB) void k_set_bbox_tiles(const float* __restrict__ pts, int64_t n,
                                                        const int32_t* __restrict__ offs,
                                                        int nsets, uint32_t* __restrict__ box,
@@ -135,13 +142,24 @@ __global__ __launch_bounds__(kB) void k_set_bbox_tiles(const float* __restrict__
   }
   if (s_first != s_last) {
     if (threadIdx.x < 6) part[6 * t + threadIdx.x] = threadIdx.x < 3 ? INFINITY : -INFINITY;
-    if (ok) {
-      const int my = set_of(offs, nsets, static_cast<int>(i));
+    const int my = ok ? set_of(offs, nsets, static_cast<int>(i)) : nsets;
+    uint32_t u[6];
+    for (int a = 0; a < 6; ++a) u[a] = f2ord(v[a]);
+    for (int d = 1; d < 64; d <<= 1) {
+      const int other = __shfl_up(my, d, 64);
+      const bool same = lane >= d && other == my;
       for (int a = 0; a < 3; ++a) {
-        atomicMin(&box[6 * my + a], f2ord(v[a]));
-        atomicMax(&box[6 * my + 3 + a], f2ord(v[3 + a]));
+        const uint32_t l = __shfl_up(u[a], d, 64), h = __shfl_up(u[3 + a], d, 64);
+        u[a] = same && l < u[a] ? l : u[a];
+        u[3 + a] = same && h > u[3 + a] ? h : u[3 + a];
       }
     }
+    const int next = __shfl_down(my, 1, 64);
+    if (ok && (lane == 63 || next != my))
+      for (int a = 0; a < 3; ++a) {
+        atomicMin(&box[6 * my + a], u[a]);
+        atomicMax(&box[6 * my + 3 + a], u[3 + a]);
+      }
     return;
   }
   for (int d = 32; d > 0; d >>= 1)
@@ -198,17 +216,25 @@ __global__ __launch_bounds__(kB) void k_set_bbox_sets(const int32_t* __restrict_
 
 // Initialises the forest: per-set cube geometry, one root per set (node k is
 // the root of set k), the level table and the zero-mass sentinel node.  The
-// bounds come either as six final floats (one set: min xyz, max xyz) or as
-// the per-set atomics of k_set_bbox (expanded by 1e-3 here; an empty set
+// bounds come either as six final floats (one set: min xyz, max xyz; with
+// nparts > 0 bounds6 holds the partials of k_bbox_partial instead, reduced here)
+// or as the per-set atomics of k_set_bbox (expanded by 1e-3 here; an empty set
 // gets the cube of the origin).
 __global__ __launch_bounds__(kB) void k_forest_init(
-    int64_t n, int nsets, const float* __restrict__ bounds6,
+    int64_t n, int nsets, const float* __restrict__ bounds6, int nparts,
     const uint32_t* __restrict__ setbox, int32_t* __restrict__ offs, CubeGeom* __restrict__ geoms,
     Header* __restrict__ hdr, int4* __restrict__ topo, uint32_t* __restrict__ prefix,
     float4* __restrict__ geo, int32_t* __restrict__ parent, float4* __restrict__ mp,
     float4* __restrict__ qd, int sentinel) {
   __shared__ int bad;
+  __shared__ float box6[6];
   if (threadIdx.x == 0) bad = 0;
+  if (setbox == nullptr) {
+    if (nparts > 0)
+      bbox_reduce(bounds6, nparts, n, box6);
+    else if (threadIdx.x < 6)
+      box6[threadIdx.x] = bounds6[threadIdx.x];
+  }
   __syncthreads();
   if (setbox == nullptr) {
     if (threadIdx.x == 0) {
@@ -228,8 +254,8 @@ __global__ __launch_bounds__(kB) void k_forest_init(
     int32_t s0, cnt;
     if (setbox == nullptr) {
       for (int a = 0; a < 3; ++a) {
-        lo[a] = bounds6[a];
-        hi[a] = bounds6[3 + a];
+        lo[a] = box6[a];
+        hi[a] = box6[3 + a];
       }
       s0 = 0;
       cnt = static_cast<int32_t>(n);
@@ -330,7 +356,8 @@ __global__ __launch_bounds__(kB) void k_gather(const float* __restrict__ pts,
 //   k_topo_finalize  counts and child counts of the records, group sizes, and
 //                    the moments of every leaf (a row of 16 lanes per node);
 //                    k_moments_internal then does the internal levels, one
-//                    launch per level, deepest first
+//                    launch per level, deepest first, and k_moments_top the
+//                    last, small ones together
 constexpr int kTopoTile = 1024;  // one point per thread, one tile per block
 constexpr int kTopoWaves = kTopoTile / 64;
 constexpr int kTopoCols = topo::kLevels;
@@ -362,32 +389,47 @@ __device__ __forceinline__ SetRange set_range(const int32_t* __restrict__ offs, 
   return q;
 }
 
-// Value of the last thread of the block at or before this one with `has`
-// set, else `fallback`.  All threads of the block must call it.
-__device__ __forceinline__ int block_last(bool has, int v, int fallback, int* s_w, int lane,
-                                          int w) {
-  const uint64_t b = __ballot(has);
-  const uint64_t le = b & (lane == 63 ? ~0ull : ((2ull << lane) - 1ull));
-  // every lane takes part in both shuffles (sources are lanes with `has`)
-  const int src = le != 0ull ? 63 - __clzll(static_cast<long long>(le)) : lane;
-  const int got = __shfl(v, src, 64);
-  int mine = le != 0ull ? got : fallback;
-  const int wsrc = b != 0ull ? 63 - __clzll(static_cast<long long>(b)) : 0;
-  const int wlast = __shfl(v, wsrc, 64);
-  if (lane == 0) s_w[2 * w] = b != 0ull ? 1 : 0;
-  if (lane == 0) s_w[2 * w + 1] = wlast;
-  __syncthreads();
-  if (le == 0ull) {
-    for (int k = w - 1; k >= 0; --k)
-      if (s_w[2 * k]) {
-        mine = s_w[2 * k + 1];
-        break;
-      }
+// For two values >= 0 a thread (-1: none): the value of the last thread of the
+// block at or before this one that has one, else -1.  All threads of the block
+// must call it, once per kernel (s_last is not guarded against reuse).
+__device__ __forceinline__ void block_last2(int v0, int v1, int (*s_last)[kTopoWaves], int lane,
+                                            int w, int* got0, int* got1) {
+  int mine[2];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int v = q == 0 ? v0 : v1;
+    const uint64_t b = __ballot(v >= 0);
+    const uint64_t le = b & (lane == 63 ? ~0ull : ((2ull << lane) - 1ull));
+    // every lane takes part in the shuffles (sources are lanes with a value)
+    const int src = le != 0ull ? 63 - __clzll(static_cast<long long>(le)) : lane;
+    const int got = __shfl(v, src, 64);
+    mine[q] = le != 0ull ? got : -1;
+    const int last = __shfl(v, b != 0ull ? 63 - __clzll(static_cast<long long>(b)) : 0, 64);
+    if (lane == 0) s_last[q][w] = last;
   }
-  __syncthreads();  // s_w is reused by the next call
-  return mine;
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int x = lane < w ? s_last[q][lane] : -1;  // the earlier waves' last values
+    const uint64_t b = __ballot(x >= 0);
+    const int before = __shfl(x, b != 0ull ? 63 - __clzll(static_cast<long long>(b)) : 0, 64);
+    if (mine[q] < 0 && b != 0ull) mine[q] = before;
+  }
+  *got0 = mine[0];
+  *got1 = mine[1];
 }
 
+// Sorted codes of a tile and of all that its points' searches read beyond it
+// when leaf_size <= kGroupCell, staged in LDS and indexed from the tile's first
+// point less kTopoHalo.
+constexpr int kTopoHalo = kGroupCell + 2;
+constexpr int kTopoWindow = kTopoTile + 2 * kTopoHalo;
+
+// Bound by the searches' dependent reads.  WINDOW (leaf_size <= kGroupCell):
+// from LDS, in 32-bit positions; else from the array.  2003 points 9 us and 2^20
+// points 23 (from the array and with the block's last values found by five block
+// scans in turn 16 and 40).
+template <bool WINDOW>
 __global__ __launch_bounds__(kTopoTile) void k_topo_count(const Header* __restrict__ hdr,
                                                           int64_t n,
                                                    const uint32_t* __restrict__ codes,
@@ -396,55 +438,73 @@ __global__ __launch_bounds__(kTopoTile) void k_topo_count(const Header* __restri
                                                    int32_t* __restrict__ tiles,
                                                    uint32_t* __restrict__ prec) {
   __shared__ int s_cnt[kTopoWaves][kTopoCols];
-  __shared__ int s_w[2 * kTopoWaves];
+  __shared__ int s_last[2][kTopoWaves];
+  __shared__ uint32_t s_codes[WINDOW ? kTopoWindow : 1];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int64_t r = static_cast<int64_t>(blockIdx.x) * kTopoTile + threadIdx.x;
+  const int64_t tile0 = static_cast<int64_t>(blockIdx.x) * kTopoTile;
+  const int64_t r = tile0 + threadIdx.x;
+  if (WINDOW) {
+    for (int k = threadIdx.x; k < kTopoWindow; k += kTopoTile) {
+      const int64_t i = tile0 - kTopoHalo + k;
+      s_codes[k] = i >= 0 && i < n ? codes[i] : 0u;
+    }
+    __syncthreads();
+  }
   const bool ok = r < n && (hdr->overflow & 2) == 0;
   topo::PointNodes p{0, -1, 0, -1};
   int gl = -1;
   bool sb = false;
   if (ok) {
     const SetRange q = set_range(offs, nsets, r);
-    p = topo::point_nodes(codes, r, q.sb, q.se, D, leaf_size);
-    gl = topo::group_cell_level(codes, r, q.sb, q.se, D, p);
+    if (WINDOW) {
+      // n < 2^30: positions relative to the window fit an int
+      const int64_t first = tile0 - kTopoHalo;
+      const int rw = kTopoHalo + static_cast<int>(threadIdx.x);
+      const int sbw = static_cast<int>(q.sb - first), sew = static_cast<int>(q.se - first);
+      p = topo::point_nodes<int>(s_codes, rw, sbw, sew, D, leaf_size);
+      gl = topo::group_cell_level<int>(s_codes, rw, sbw, sew, D, p);
+    } else {
+      p = topo::point_nodes<int64_t>(codes, r, q.sb, q.se, D, leaf_size);
+      gl = topo::group_cell_level<int64_t>(codes, r, q.sb, q.se, D, p);
+    }
     sb = r == q.sb;
     prec[r] = pack_point(p, gl);
   }
-  const int ri = static_cast<int>(r);
+  const int tid = static_cast<int>(threadIdx.x);
   const bool has_g = ok && gl >= 0;
-  const int gs = block_last(has_g, ri, -1, s_w, lane, w);
-  const bool gstart = ok && gs >= 0 && ((ri - gs) % kGroupMax) == 0;
   const bool lam_src = ok && (p.first > 0 || sb);
-  // tile summary: first / last group cell, last lambda source (thread 255 sees all)
-  const int lastg = block_last(has_g, ri, -1, s_w, lane, w);
-  const int lampos = block_last(lam_src, ri, -1, s_w, lane, w);
-  const int lamtop = block_last(lam_src, p.first > 0 ? p.top : 0, -1, s_w, lane, w);
   const uint64_t bg = __ballot(has_g);
-  const int fsrc = bg != 0ull ? __ffsll(static_cast<long long>(bg)) - 1 : 0;
-  const int fval = __shfl(ri, fsrc, 64);
-  if (lane == 0) s_cnt[w][kColFirstG] = bg != 0ull ? fval : -1;
-  const int cg = __popcll(__ballot(gstart));
-  if (lane == 0) s_cnt[w][kColGroups] = cg;
+  if (lane == 0) s_cnt[w][kColFirstG] = bg != 0ull ? tid + __ffsll(static_cast<long long>(bg)) - 1 : -1;
+#pragma unroll
   for (int l = 1; l <= 10; ++l) {
     const int c = __popcll(__ballot(ok && l <= D && p.first > 0 && l >= p.first && l <= p.top));
     if (lane == 0) s_cnt[w][l] = c;
   }
+  int gs, lam;
+  block_last2(has_g ? tid : -1, lam_src ? tid << 4 | (p.first > 0 ? p.top : 0) : -1, s_last, lane,
+              w, &gs, &lam);
+  const bool gstart = ok && gs >= 0 && ((tid - gs) % kGroupMax) == 0;
+  const int cg = __popcll(__ballot(gstart));
+  if (lane == 0) s_cnt[w][kColGroups] = cg;
   __syncthreads();
   int32_t* out = tiles + static_cast<int64_t>(blockIdx.x) * kTopoCols;
+  const int base = static_cast<int>(tile0);
   if (threadIdx.x <= 10) {
     int c = 0;
+#pragma unroll
     for (int k = 0; k < kTopoWaves; ++k) c += s_cnt[k][threadIdx.x];
     out[threadIdx.x] = c;
   }
-  if (threadIdx.x == 0) {
-    int f = -1;
-    for (int k = 0; k < kTopoWaves && f < 0; ++k) f = s_cnt[k][kColFirstG];
-    out[kColFirstG] = f;
+  if (w == 1) {
+    const int f = lane < kTopoWaves ? s_cnt[lane][kColFirstG] : -1;
+    const uint64_t b = __ballot(f >= 0);
+    if (b == 0ull ? lane == 0 : lane == __ffsll(static_cast<long long>(b)) - 1)
+      out[kColFirstG] = b == 0ull ? -1 : base + f;
   }
-  if (threadIdx.x == kTopoTile - 1) {
-    out[kColLastG] = lastg;
-    out[kColLamPos] = lampos;
-    out[kColLamTop] = lamtop;
+  if (threadIdx.x == kTopoTile - 1) {  // sees the whole tile
+    out[kColLastG] = gs >= 0 ? base + gs : -1;
+    out[kColLamPos] = lam >= 0 ? base + (lam >> 4) : -1;
+    out[kColLamTop] = lam >= 0 ? lam & 15 : -1;
     out[15] = 0;
   }
 }
@@ -456,104 +516,90 @@ __device__ __forceinline__ int64_t lead_groups(int64_t g, int64_t t0, int64_t t1
   return le(t1 - 1) - le(t0 - 1);
 }
 
-// Exclusive block scan (sum, or max with identity -1) of one value per
-// thread of a 1024-thread block; the block total (maximum) through *all.
-template <typename T, bool SUM>
-__device__ __forceinline__ T block_scan1(T v, T* s_w, T* all) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  T incl = v;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const T t = __shfl_up(incl, d, 64);
-    if (lane >= d) incl = SUM ? incl + t : (incl > t ? incl : t);
-  }
-  T ex = __shfl_up(incl, 1, 64);
-  if (lane == 0) ex = SUM ? T(0) : T(-1);
-  if (lane == 63) s_w[w] = incl;
-  __syncthreads();
-  T before = SUM ? T(0) : T(-1), tot = SUM ? T(0) : T(-1);
-  for (int j = 0; j < 16; ++j) {
-    const T x = s_w[j];
-    if (SUM) {
-      if (j < w) before += x;
-      tot += x;
-    } else {
-      if (j < w) before = before > x ? before : x;
-      tot = tot > x ? tot : x;
-    }
-  }
-  __syncthreads();
-  *all = tot;
-  return SUM ? before + ex : (before > ex ? before : ex);
+// Exclusive sum over the lanes of a wave, continuing *carry, which becomes the
+// sum over all 64 (shifts within rows of 16 lanes, then two row broadcasts).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp_add(int v) {
+  return v + __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false);
 }
+__device__ __forceinline__ int wave_excl_sum(int v, int* carry) {
+  int x = dpp_add<0x111, 0xf>(v);  // row_shr:1
+  x = dpp_add<0x112, 0xf>(x);      // row_shr:2
+  x = dpp_add<0x114, 0xf>(x);      // row_shr:4
+  x = dpp_add<0x118, 0xf>(x);      // row_shr:8
+  x = dpp_add<0x142, 0xa>(x);      // row_bcast:15 into rows 1 and 3
+  x = dpp_add<0x143, 0xc>(x);      // row_bcast:31 into rows 2 and 3
+  const int before = *carry;
+  *carry = before + __builtin_amdgcn_readlane(x, 63);
+  return before + x - v;
+}
+
+// Value of the nearest earlier lane with one (>= 0), else *carry, which becomes
+// the last lane's.
+__device__ __forceinline__ int wave_last(int v, int lane, int* carry) {
+  const uint64_t b = __ballot(v >= 0);
+  const uint64_t lt = b & ((1ull << lane) - 1ull);
+  const int got = __shfl(v, lt != 0ull ? 63 - __clzll(static_cast<long long>(lt)) : lane, 64);
+  const int ex = lt != 0ull ? got : *carry;
+  if (b != 0ull)
+    *carry = __builtin_amdgcn_readlane(v, 63 - __clzll(static_cast<long long>(b)));
+  return ex;
+}
+
+// One block; every wave scans a column of its own over the tiles, 64 tiles at
+// a time, the loads of kScanAhead such rounds issued together: waves 1-10 the
+// level begins, wave 0 the last group cell and the group starts that depend on
+// it, wave 11 lambda.  Bound by the latency of the loads: one tile 4 us,
+// 1024 tiles 16 (one block scan per column in turn: 12 and 20).
+constexpr int kScanAhead = 8;
 
 __global__ __launch_bounds__(1024) void k_topo_scan(Header* __restrict__ hdr,
                                                     int32_t* __restrict__ tiles, int64_t ntiles,
                                                     int64_t n, int nsets, int D, int64_t cap) {
-  __shared__ int32_t s_w32[16];
-  __shared__ int64_t s_w64[16];
-  __shared__ int32_t s_tot[11];
-  __shared__ int32_t s_lvl[10][1024];  // exclusive level offsets entering each chunk
-  const int tid = threadIdx.x;
-  const int64_t per = (ntiles + 1023) / 1024;
-  const int64_t t0 = tid * per, t1 = t0 + per < ntiles ? t0 + per : ntiles;
-#pragma unroll 1
-  for (int l = 0; l < 10; ++l) {
-    int32_t sum = 0;
-    for (int64_t t = t0; t < t1; ++t) sum += tiles[t * kTopoCols + 1 + l];
-    int32_t tot;
-    s_lvl[l][tid] = block_scan1<int32_t, true>(sum, s_w32, &tot);
-    if (tid == 0) s_tot[l] = tot;
-  }
-  // carries entering the chunk: the last group cell (positions rise, so a
-  // max) and the last lambda source as (position << 4 | top)
-  int64_t cg = -1, cl = -1;
-  for (int64_t t = t0; t < t1; ++t) {
-    const int32_t* c = tiles + t * kTopoCols;
-    if (c[kColLastG] >= 0) cg = c[kColLastG];
-    if (c[kColLamPos] >= 0) cl = (static_cast<int64_t>(c[kColLamPos]) << 4) | c[kColLamTop];
-  }
-  int64_t dummy;
-  const int64_t g_in = block_scan1<int64_t, false>(cg, s_w64, &dummy);
-  const int64_t l_in = block_scan1<int64_t, false>(cl, s_w64, &dummy);
-  // group starts per chunk (the leading ones need the carried cell)
-  int32_t gsum = 0;
-  {
-    int64_t g = g_in;
-    for (int64_t t = t0; t < t1; ++t) {
-      const int32_t* c = tiles + t * kTopoCols;
-      const int64_t x = t * kTopoTile, e = x + kTopoTile < n ? x + kTopoTile : n;
-      gsum += static_cast<int32_t>(lead_groups(g, x, c[kColFirstG] >= 0 ? c[kColFirstG] : e)) +
-              c[kColGroups];
-      if (c[kColLastG] >= 0) g = c[kColLastG];
+  __shared__ int32_t s_tot[11];  // levels 1..10, groups
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  int32_t sum = 0;
+  int last = -1;
+  for (int64_t t0 = 0; t0 < ntiles && w < 12; t0 += 64 * kScanAhead) {
+    int32_t a[kScanAhead], b[kScanAhead], c[kScanAhead];
+    // wave 0: group starts, first and last group cell; 11: lambda; else begins
+    const int ca = w == 11 ? kColLamPos : w;
+    const int cb = w == 11 ? kColLamTop : kColLastG;
+#pragma unroll
+    for (int j = 0; j < kScanAhead; ++j) {
+      const int64_t t = t0 + 64 * j + lane;
+      const bool in = t < ntiles;
+      const int32_t* row = tiles + (in ? t : 0) * kTopoCols;
+      a[j] = in ? row[ca] : (w == 11 ? -1 : 0);
+      b[j] = in && (w == 0 || w == 11) ? row[cb] : -1;
+      c[j] = in && w == 0 ? row[kColFirstG] : -1;
     }
-  }
-  int32_t gtot;
-  int32_t goff = block_scan1<int32_t, true>(gsum, s_w32, &gtot);
-  // per-tile outputs
-  {
-    int64_t g = g_in;
-    int32_t lam = l_in >= 0 ? static_cast<int32_t>(l_in & 15) : -1;
-    for (int64_t t = t0; t < t1; ++t) {
-      int32_t* c = tiles + t * kTopoCols;
-      const int64_t x = t * kTopoTile, e = x + kTopoTile < n ? x + kTopoTile : n;
-      const int32_t first_g = c[kColFirstG], last_g = c[kColLastG];
-      const int32_t lam_pos = c[kColLamPos], lam_top = c[kColLamTop];
-      const int32_t here =
-          static_cast<int32_t>(lead_groups(g, x, first_g >= 0 ? first_g : e)) + c[kColGroups];
-      c[kColGroups] = goff;
-      goff += here;
-      for (int l = 0; l < 10; ++l) {
-        const int32_t v = c[1 + l];
-        c[1 + l] = s_lvl[l][tid];
-        s_lvl[l][tid] += v;
+#pragma unroll
+    for (int j = 0; j < kScanAhead; ++j) {
+      const int64_t t = t0 + 64 * j + lane;
+      const bool in = t < ntiles;
+      int32_t* row = tiles + (in ? t : 0) * kTopoCols;
+      if (w == 0) {
+        // the last group cell entering the tile, then the group starts (the
+        // leading ones of a tile need that cell)
+        const int32_t g = wave_last(b[j], lane, &last);
+        const int64_t x = t * kTopoTile, e = x + kTopoTile < n ? x + kTopoTile : n;
+        const int32_t starts =
+            in ? static_cast<int32_t>(lead_groups(g, x, c[j] >= 0 ? c[j] : e)) + a[j] : 0;
+        const int32_t off = wave_excl_sum(starts, &sum);
+        if (in) row[kColGroups] = off;
+        if (in) row[kColLastG] = g;
+      } else if (w == 11) {
+        const int32_t l = wave_last(a[j] >= 0 ? b[j] : -1, lane, &last);
+        if (in) row[kColLamTop] = l;
+      } else {
+        const int32_t off = wave_excl_sum(a[j], &sum);
+        if (in) row[w] = off;
       }
-      c[kColLastG] = static_cast<int32_t>(g);
-      c[kColLamTop] = lam;
-      if (last_g >= 0) g = last_g;
-      if (lam_pos >= 0) lam = lam_top;
     }
   }
+  if (lane == 0 && w <= 10) s_tot[w == 0 ? 10 : w - 1] = sum;
+  __syncthreads();
   if (tid == 0) {
     int64_t start = nsets;
     for (int l = 1; l < kMaxLevels; ++l) {
@@ -571,7 +617,7 @@ __global__ __launch_bounds__(1024) void k_topo_scan(Header* __restrict__ hdr,
       start = nsets;
     }
     hdr->num_nodes = static_cast<int32_t>(start);
-    hdr->num_groups = gtot;
+    hdr->num_groups = s_tot[10];
     hdr->queue = 0;
     for (int x = 0; x < 8; ++x) hdr->xq[x] = hdr->tq[x] = 0;
   }
@@ -584,7 +630,7 @@ __global__ __launch_bounds__(kTopoTile) void k_topo_emit(
     int4* __restrict__ topo, uint32_t* __restrict__ prefix, float4* __restrict__ geo,
     int32_t* __restrict__ parent, int2* __restrict__ ends, int2* __restrict__ groups) {
   __shared__ int s_cnt[kTopoWaves][kTopoCols];
-  __shared__ int s_w[2 * kTopoWaves];
+  __shared__ int s_last[2][kTopoWaves];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
   const int64_t r = static_cast<int64_t>(blockIdx.x) * kTopoTile + threadIdx.x;
@@ -603,54 +649,68 @@ __global__ __launch_bounds__(kTopoTile) void k_topo_emit(
   }
   const int ri = static_cast<int>(r);
   const bool sb = ok && r == q.sb;
-  const int gs = block_last(ok && gl >= 0, ri, base[kColLastG], s_w, lane, w);
-  const int lam = block_last(ok && (p.first > 0 || sb), p.first > 0 ? p.top : 0,
-                             base[kColLamTop], s_w, lane, w);
+  const int tid = static_cast<int>(threadIdx.x);
+  int gs, lam;
+  block_last2(ok && gl >= 0 ? tid : -1, ok && (p.first > 0 || sb) ? (p.first > 0 ? p.top : 0) : -1,
+              s_last, lane, w, &gs, &lam);
+  gs = gs >= 0 ? ri - tid + gs : base[kColLastG];
+  if (lam < 0) lam = base[kColLamTop];
   const bool gstart = ok && gs >= 0 && ((ri - gs) % kGroupMax) == 0;
-  int rank[kTopoCols];
-  {
-    const uint64_t b = __ballot(gstart);
-    rank[0] = __popcll(b & lt);
-    if (lane == 0) s_cnt[w][0] = __popcll(b);
-  }
+  // ranks in the wave, 6 bits a level (indexed by a variable level below)
+  uint64_t ranks = 0;
+  const uint64_t bs = __ballot(gstart);
+  const int grank = __popcll(bs & lt);
+  if (lane == 0) s_cnt[w][0] = __popcll(bs);
+#pragma unroll
   for (int l = 1; l <= 10; ++l) {
     const uint64_t b = __ballot(ok && l <= D && p.first > 0 && l >= p.first && l <= p.top);
-    rank[l] = __popcll(b & lt);
+    ranks |= static_cast<uint64_t>(__popcll(b & lt)) << (6 * (l - 1));
     if (lane == 0) s_cnt[w][l] = __popcll(b);
   }
   __syncthreads();
+  // s_cnt[wave][column] becomes the index that the wave's first node of the
+  // level (first group, column 0) gets: level start + tile offset + the earlier
+  // waves' counts
+  int start = 0;
+  const int col = threadIdx.x % kTopoCols, wave = threadIdx.x / kTopoCols;
+  if (wave < kTopoWaves && col <= 10) {
+    start = base[col] + (col > 0 ? hdr->level_start[col] : 0);
+    for (int k = 0; k < wave; ++k) start += s_cnt[k][col];
+  }
+  __syncthreads();
+  if (wave < kTopoWaves && col <= 10) s_cnt[wave][col] = start;
+  __syncthreads();
   if (!ok) return;
-  auto rank_of = [&](int l) {
-    int v = base[l] + rank[l];
-    for (int k = 0; k < w; ++k) v += s_cnt[k][l];
-    return v;
+  // index of r's node at level l (as if r began one)
+  auto index_of = [&](int l) {
+    return s_cnt[w][l] + static_cast<int>((ranks >> (6 * (l - 1))) & 63u);
   };
   auto begins = [&](int l) { return p.first > 0 && l >= p.first && l <= p.top ? 1 : 0; };
-  if (gstart) groups[rank_of(0)] = make_int2(ri, 0);
+  if (gstart) groups[s_cnt[w][0] + grank] = make_int2(ri, 0);
   if (!nodes_ok) return;
   // records of the nodes r begins
-  if (sb && p.first == 1) topo[q.set].z = hdr->level_start[1] + rank_of(1);
+  if (sb && p.first == 1) topo[q.set].z = index_of(1);
   if (p.first > 0) {
     const CubeGeom gm = geoms[q.set];
     for (int l = p.first; l <= p.top; ++l) {
-      const int idx = hdr->level_start[l] + rank_of(l);
+      const int idx = index_of(l);
       const uint32_t pre = codes[r] >> (3 * (D - l));
-      const int fc = l < p.top ? hdr->level_start[l + 1] + rank_of(l + 1) : -1;
+      const int fc = l < p.top ? index_of(l + 1) : -1;
       topo[idx] = make_int4(ri, 0, fc, 0);
       prefix[idx] = pre;
       parent[idx] = l == 1 ? q.set
-                           : hdr->level_start[l - 1] + rank_of(l - 1) - (l - 1 >= p.first ? 0 : 1);
+                           : index_of(l - 1) - (l - 1 >= p.first ? 0 : 1);
       geo[idx] = cell_geometry(gm, pre, l);
     }
   }
   // ends and last children of the nodes r closes
   const int dn = r + 1 < q.se ? topo::common_digits(codes[r], codes[r + 1], D) : -1;
   for (int l = dn + 1 > 1 ? dn + 1 : 1; l <= lam; ++l) {
-    const int idx = hdr->level_start[l] + rank_of(l) + begins(l) - 1;
+    const int idx = index_of(l) + begins(l) - 1;
     ends[idx].x = ri + 1;
-    if (l < lam) ends[idx].y = hdr->level_start[l + 1] + rank_of(l + 1) + begins(l + 1) - 1;
+    if (l < lam) ends[idx].y = index_of(l + 1) + begins(l + 1) - 1;
   }
-  if (r + 1 == q.se && lam >= 1) ends[q.set].y = hdr->level_start[1] + rank_of(1) + begins(1) - 1;
+  if (r + 1 == q.se && lam >= 1) ends[q.set].y = index_of(1) + begins(1) - 1;
 }
 
 // Sum over a row of 16 lanes (every lane of the row active), by DPP moves:
@@ -830,6 +890,31 @@ __global__ __launch_bounds__(kB) void k_moments_internal(const Header* __restric
     const int k = start + u;
     const int4 t = topo[k];
     if (t.w > 0) node_moments(k, t, sl, geo, sp, mp, qd, sv, wd);
+  }
+}
+
+// The same for levels top .. 0 by one block, a barrier between levels.
+__global__ __launch_bounds__(1024) void k_moments_top(const Header* __restrict__ hdr, int top,
+                                                      const int4* __restrict__ topo,
+                                                      const float4* __restrict__ geo,
+                                                      const float4* __restrict__ sp, float4* mp,
+                                                      float4* qd, const float4* __restrict__ sv,
+                                                      float4* wd) {
+  __shared__ int s_start[kMaxLevels], s_count[kMaxLevels];
+  if (threadIdx.x < kMaxLevels) {
+    s_start[threadIdx.x] = hdr->level_start[threadIdx.x];
+    s_count[threadIdx.x] = hdr->level_count[threadIdx.x];
+  }
+  __syncthreads();
+  const int sl = threadIdx.x & 15;
+  for (int l = top; l >= 0; --l) {
+    const int start = s_start[l], count = s_count[l];
+    if (count == 0) continue;
+    for (int u = threadIdx.x >> 4; u < count; u += 1024 / 16) {
+      const int4 t = topo[start + u];
+      if (t.w > 0) node_moments(start + u, t, sl, geo, sp, mp, qd, sv, wd);
+    }
+    __syncthreads();
   }
 }
 
@@ -1866,9 +1951,15 @@ Layout layout(int64_t n, int max_depth, int leaf_size, int nsets) {
   return L;
 }
 
-int data_bounds(hipStream_t s, const float* pts, int64_t n, float* tmp, float** bounds) {
-  const unsigned nb = static_cast<unsigned>(
+namespace {
+unsigned bbox_blocks(int64_t n) {
+  return static_cast<unsigned>(
       std::min<int64_t>(kBboxBlocks, std::max<int64_t>(1, (n + kB - 1) / kB)));
+}
+}  // namespace
+
+int data_bounds(hipStream_t s, const float* pts, int64_t n, float* tmp, float** bounds) {
+  const unsigned nb = bbox_blocks(n);
   k_bbox_partial<<<nb, kB, 0, s>>>(pts, n, tmp);
   SBH_LAUNCH_CHECK();
   *bounds = tmp + 6 * kBboxBlocks;
@@ -1878,6 +1969,13 @@ int data_bounds(hipStream_t s, const float* pts, int64_t n, float* tmp, float** 
 }
 
 namespace {
+
+// Levels of at most this many internal nodes (and all above them, which hold no
+// more) get their moments from one block in one launch: a launch costs more
+// than the rounds of 64 nodes a block needs: 10 levels of 2003 points 46 us
+// in ten launches, 12 in one; with 1024, 10^4 points of leaf size 16 took 32 us
+// instead of 18 + 6 x 2.
+constexpr int64_t kTopRows = 512;
 
 // Everything after the roots exist: codes, sort, gather, levels, moments, groups.
 int build_rest(hipStream_t s, char* ws, const Layout& L, const float* pts, const float* ms,
@@ -1919,8 +2017,12 @@ int build_rest(hipStream_t s, char* ws, const Layout& L, const float* pts, const
   auto* groups = reinterpret_cast<int2*>(ws + L.groups);
   const int64_t ntiles = (n + kTopoTile - 1) / kTopoTile;
   if (ntiles > 0) {
-    k_topo_count<<<static_cast<unsigned>(ntiles), kTopoTile, 0, s>>>(hdr, n, codes, offs, nsets,
-                                                              max_depth, leaf_size, tiles, prec);
+    if (leaf_size <= kGroupCell)
+      k_topo_count<true><<<static_cast<unsigned>(ntiles), kTopoTile, 0, s>>>(
+          hdr, n, codes, offs, nsets, max_depth, leaf_size, tiles, prec);
+    else
+      k_topo_count<false><<<static_cast<unsigned>(ntiles), kTopoTile, 0, s>>>(
+          hdr, n, codes, offs, nsets, max_depth, leaf_size, tiles, prec);
     SBH_LAUNCH_CHECK();
   }
   k_topo_scan<<<1, 1024, 0, s>>>(hdr, tiles, ntiles, n, nsets, max_depth, L.cap);
@@ -1944,6 +2046,11 @@ int build_rest(hipStream_t s, char* ws, const Layout& L, const float* pts, const
       const int64_t cap_l = std::min<int64_t>(
           l < 18 ? static_cast<int64_t>(nsets) << (3 * l) : INT64_MAX,
           std::max<int64_t>(nsets, internal_max));
+      if (cap_l <= kTopRows) {
+        k_moments_top<<<1, 1024, 0, s>>>(hdr, l, topo, geo, sp, mp, qd, sc, wd);
+        SBH_LAUNCH_CHECK();
+        break;
+      }
       k_moments_internal<<<grid_for(cap_l, kB / 16, 1024), kB, 0, s>>>(hdr, l, topo, geo, sp,
                                                                         mp, qd, sc, wd);
       SBH_LAUNCH_CHECK();
@@ -1953,9 +2060,9 @@ int build_rest(hipStream_t s, char* ws, const Layout& L, const float* pts, const
 }
 
 int init_roots(hipStream_t s, char* ws, const Layout& L, int64_t n, const float* bounds6,
-               const uint32_t* setbox) {
+               int nparts, const uint32_t* setbox) {
   k_forest_init<<<1, kB, 0, s>>>(
-      n, L.nsets, bounds6, setbox, reinterpret_cast<int32_t*>(ws + L.offs),
+      n, L.nsets, bounds6, nparts, setbox, reinterpret_cast<int32_t*>(ws + L.offs),
       reinterpret_cast<CubeGeom*>(ws + L.geoms), reinterpret_cast<Header*>(ws + L.header),
       reinterpret_cast<int4*>(ws + L.topo), reinterpret_cast<uint32_t*>(ws + L.prefix),
       reinterpret_cast<float4*>(ws + L.geo), reinterpret_cast<int32_t*>(ws + L.parent),
@@ -1971,13 +2078,15 @@ int build(hipStream_t s, char* ws, const Layout& L, const float* pts, const floa
           const float* cot, int64_t n, int max_depth, int leaf_size,
           const float* user_bounds, int parts, float4* dipoles) {
   if (L.nsets != 1) return fail_internal_msg("build: layout is a forest");
+  int nparts = 0;
   if (user_bounds == nullptr) {
-    float* b = nullptr;
-    int rc = data_bounds(s, pts, n, reinterpret_cast<float*>(ws + L.bbox_tmp), &b);
-    if (rc != SBH_OK) return rc;
-    user_bounds = b;
+    auto* parts6 = reinterpret_cast<float*>(ws + L.bbox_tmp);
+    nparts = static_cast<int>(bbox_blocks(n));
+    k_bbox_partial<<<static_cast<unsigned>(nparts), kB, 0, s>>>(pts, n, parts6);
+    SBH_LAUNCH_CHECK();
+    user_bounds = parts6;
   }
-  int rc = init_roots(s, ws, L, n, user_bounds, nullptr);
+  int rc = init_roots(s, ws, L, n, user_bounds, nparts, nullptr);
   if (rc != SBH_OK) return rc;
   return build_rest(s, ws, L, pts, ms, cot, n, reinterpret_cast<const int32_t*>(ws + L.offs),
                     max_depth, leaf_size, parts, dipoles);
@@ -2002,7 +2111,7 @@ int build_forest(hipStream_t s, char* ws, const Layout& L, const float* pts, con
     k_set_bbox_sets<<<static_cast<unsigned>(L.nsets), kB, 0, s>>>(ofs, part, box);
     SBH_LAUNCH_CHECK();
   }
-  int rc = init_roots(s, ws, L, n, nullptr, box);
+  int rc = init_roots(s, ws, L, n, nullptr, 0, box);
   if (rc != SBH_OK) return rc;
   return build_rest(s, ws, L, pts, ms, cot, n, ofs, max_depth, leaf_size, parts, nullptr);
 }
