@@ -48,9 +48,16 @@ constexpr uint32_t kAgg = 1u << 30;    // status: tile count published
 constexpr uint32_t kIncl = 2u << 30;   // status: inclusive prefix published
 constexpr uint32_t kValue = (1u << 30) - 1u;
 constexpr int kSpinLimit = 1 << 22;
+constexpr int64_t kMaxKeys = int64_t{1} << 30;  // counts share a word with two flags
+
+// Blocks of k_os_hist for n keys.
+int hist_blocks(int64_t n) {
+  return static_cast<int>(std::max<int64_t>(
+      1, std::min<int64_t>(kHistBlocks, (n + kHistBlock - 1) / kHistBlock)));
+}
 
 struct OsLayout {
-  size_t hist;    // kHistBlocks x code passes x 256 u32
+  size_t hist;    // hist_blocks(n) x kMaxPasses x 256 u32
   size_t offs;    // passes x 256 u32: global exclusive digit offsets
   size_t ticket;  // passes u32 (padded)
   size_t status;  // passes x tiles x 256 u32
@@ -63,7 +70,7 @@ OsLayout os_layout(int64_t n, int passes) {
   const size_t tiles = static_cast<size_t>((n + tile - 1) / tile);
   OsLayout L;
   size_t o = 0;
-  L.hist = o; o = align(o + 4ull * kHistBlocks * kMaxPasses * kRadix);
+  L.hist = o; o = align(o + 4ull * hist_blocks(n) * kMaxPasses * kRadix);
   L.offs = o; o = align(o + 4ull * kMaxPasses * kRadix);
   L.ticket = o; o = align(o + 4ull * 64);
   L.status = o; o = align(o + 4ull * static_cast<size_t>(passes) * tiles * kRadix);
@@ -315,7 +322,7 @@ int morton_sort(hipStream_t s, const uint32_t* codes, int64_t n, int key_bits,
   *keys = nullptr;
   *perm = nullptr;
   if (n <= 0) return SBH_OK;
-  if (n >= (int64_t{1} << 30)) return fail_invalid("too many points for the sort");
+  if (n >= kMaxKeys) return fail_invalid("too many points for the sort");
   const int code_passes = key_bits <= 0 ? 1 : (key_bits + 7) / 8;
   int set_passes = 0;
   while (nsets > 1 && (int64_t{1} << (8 * set_passes)) < nsets) ++set_passes;
@@ -330,8 +337,7 @@ int morton_sort(hipStream_t s, const uint32_t* codes, int64_t n, int key_bits,
   const int items = items_for(n);
   const int64_t tile = static_cast<int64_t>(kBlock) * items;
   const int64_t tiles = (n + tile - 1) / tile;
-  const int blocks = static_cast<int>(
-      std::min<int64_t>(kHistBlocks, (n + kHistBlock - 1) / kHistBlock));
+  const int blocks = hist_blocks(n);
   k_os_hist<<<blocks, kHistBlock, 0, s>>>(codes, n, code_passes, set_passes, set_offs, nsets,
                                             hist, status,
                                             static_cast<int64_t>(passes) * tiles * kRadix);
@@ -364,6 +370,32 @@ int morton_sort(hipStream_t s, const uint32_t* codes, int64_t n, int key_bits,
   *keys = kin;
   *perm = vin;
   return SBH_OK;
+}
+
+namespace {
+__global__ __launch_bounds__(kBlock) void k_rows(uint32_t* __restrict__ vals, int64_t n) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+  if (i < n) vals[i] = static_cast<uint32_t>(i);
+}
+size_t flag_bytes() { return 256; }
+}  // namespace
+
+size_t order_temp_bytes(int64_t n) {
+  return n < kMaxKeys ? morton_sort_temp_bytes(n, 1) + flag_bytes() : radix_sort_temp_bytes(n);
+}
+
+int order_by_key(hipStream_t s, uint32_t* keys, int64_t n, int key_bits, uint32_t* vals,
+                 uint32_t* keys2, uint32_t* vals2, void* temp, const uint32_t** sorted,
+                 const uint32_t** perm) {
+  if (n < kMaxKeys)
+    return morton_sort(s, keys, n, key_bits, nullptr, 1, keys2, vals2, keys, vals,
+                       static_cast<char*>(temp) + flag_bytes(), static_cast<int32_t*>(temp),
+                       sorted, perm);
+  k_rows<<<grid_for(n, kBlock), kBlock, 0, s>>>(vals, n);
+  SBH_LAUNCH_CHECK();
+  *sorted = keys2;
+  *perm = vals2;
+  return radix_sort_pairs(s, keys, vals, keys2, vals2, n, key_bits, temp);
 }
 
 }  // namespace sbh

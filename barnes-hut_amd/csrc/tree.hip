@@ -2276,15 +2276,13 @@ namespace {
 // 30-bit Morton key of each query in the queries' own bounding box.
 __global__ __launch_bounds__(kB) void k_query_keys(const float* __restrict__ q, int64_t nq,
                                                    const float* __restrict__ bounds,
-                                                   uint32_t* __restrict__ keys,
-                                                   uint32_t* __restrict__ vals) {
+                                                   uint32_t* __restrict__ keys) {
   const float lx = bounds[0], ly = bounds[1], lz = bounds[2];
   const float span = fmaxf(fmaxf(bounds[3] - lx, bounds[4] - ly), fmaxf(bounds[5] - lz, 1e-30f));
   for (int64_t i = static_cast<int64_t>(blockIdx.x) * kB + threadIdx.x; i < nq;
        i += static_cast<int64_t>(gridDim.x) * kB) {
     keys[i] = morton3(quantize_axis(q[3 * i], lx, span, 10), quantize_axis(q[3 * i + 1], ly, span, 10),
                       quantize_axis(q[3 * i + 2], lz, span, 10));
-    vals[i] = static_cast<uint32_t>(i);
   }
 }
 
@@ -2302,7 +2300,7 @@ QueryOrderLayout query_order_layout(int64_t nq) {
   L.vals = o; o = align(o + n4);
   L.keys_out = o; o = align(o + n4);
   L.perm = o; o = align(o + n4);
-  L.sort = o; o = align(o + radix_sort_temp_bytes(nq));
+  L.sort = o; o = align(o + order_temp_bytes(nq));
   L.total = o;
   return L;
 }
@@ -2317,15 +2315,12 @@ int query_order(hipStream_t s, const float* q, int64_t nq, char* ws, const uint3
   int rc = data_bounds(s, q, nq, reinterpret_cast<float*>(ws + L.tmp), &bounds);
   if (rc != SBH_OK) return rc;
   auto* keys = reinterpret_cast<uint32_t*>(ws + L.keys);
-  auto* vals = reinterpret_cast<uint32_t*>(ws + L.vals);
-  auto* out = reinterpret_cast<uint32_t*>(ws + L.perm);
-  k_query_keys<<<grid_for(nq, kB, 4096), kB, 0, s>>>(q, nq, bounds, keys, vals);
+  k_query_keys<<<grid_for(nq, kB, 4096), kB, 0, s>>>(q, nq, bounds, keys);
   SBH_LAUNCH_CHECK();
-  rc = radix_sort_pairs(s, keys, vals, reinterpret_cast<uint32_t*>(ws + L.keys_out), out, nq, 30,
-                        ws + L.sort);
-  if (rc != SBH_OK) return rc;
-  *perm = out;
-  return SBH_OK;
+  const uint32_t* sorted = nullptr;
+  return order_by_key(s, keys, nq, 30, reinterpret_cast<uint32_t*>(ws + L.vals),
+                      reinterpret_cast<uint32_t*>(ws + L.keys_out),
+                      reinterpret_cast<uint32_t*>(ws + L.perm), ws + L.sort, &sorted, perm);
 }
 
 }  // namespace tree
