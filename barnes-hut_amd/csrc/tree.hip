@@ -1403,7 +1403,7 @@ __device__ __forceinline__ void walk_group(const WalkArgs& A, int base, int cnt,
   };
 
   const int root = A.nsets > 1 ? set_of(A.offs, A.nsets, base) : 0;
-  traverse<true>(A.hdr, &A.hdr->overflow, A.topo, A.geo, A.mp, A.beta, box, lane, root, stack,
+  traverse(A.hdr, &A.hdr->overflow, A.topo, A.geo, A.mp, A.beta, box, lane, root, stack,
                  far, near, flush_far, flush_near);
 
   if (lane < cnt) {
@@ -1578,7 +1578,8 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(VJP ? 
 constexpr int kShares = 16;
 constexpr int kTeamWidth = 512;
 constexpr int kTeamFar = 1024;        // the lists are evaluated from here on
-// Leaf list and stack (see kStackSoft).  Walks that give forces share their
+// Leaf list and stack (a pop takes at most (kTeamSoft - top) / 7 nodes near the
+// soft limit, so a push of <= 8 children each fits).  Walks that give forces share their
 // sizes, which enter the sums; with six sums per share two blocks of 8 waves
 // just fit on a CU.  The others evaluate less often.
 template <bool FORCES>

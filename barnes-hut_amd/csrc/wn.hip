@@ -12,7 +12,7 @@
 // sign, so the truncated series is less accurate than the dipole alone.
 //
 // Queries are a separate cloud with a tree of their own (topology only, in
-// their own cube); its cell groups of <= 64 queries (one wavefront each) are
+// their own cube); its cell groups of <= 64 queries (one team of waves each) are
 // walked against the element tree with the group MAC and traversal of the
 // gravity walk.  (Plain runs of 64 Morton-sorted queries are not used: runs
 // that cross a coarse cell boundary have boxes spanning much of the domain
@@ -120,69 +120,220 @@ __device__ __forceinline__ float wn_near_batch(const WnArgs& A, float qx, float 
   return w;
 }
 
-__global__ __launch_bounds__(kB) void k_wn_walk(WnArgs A) {
-  __shared__ int s_stack[kWavesPerBlock][kStackCap];
-  __shared__ int s_far[kWavesPerBlock][kFarCap];
-  __shared__ int s_near[kWavesPerBlock][kNearCap];
-  const int lane = threadIdx.x & 63;
-  const int wv = threadIdx.x >> 6;
-  int* stack = s_stack[wv];
-  int* far = s_far[wv];
-  int* near = s_near[wv];
-  const int num_groups = A.qhdr->num_groups;
-  unsigned long long n_far = 0, n_near = 0, n_groups = 0;
+// Elements [s0, s1) against the lane's query.
+__device__ __forceinline__ float wn_range(const WnArgs& A, float qx, float qy, float qz, int s0,
+                                          int s1) {
+  float w = 0.f;
+  int j0 = s0;
+  for (; j0 + kChunk <= s1; j0 += kChunk) w += wn_near_batch<false>(A, qx, qy, qz, j0, s1);
+  if (j0 < s1) w += wn_near_batch<true>(A, qx, qy, qz, j0, s1);
+  return w;
+}
+
+// Walk with the TEAM waves of a block sharing each group of queries, as the
+// teams of the gravity walk (tree.hip) do: the threads test candidate nodes, the
+// accepted nodes and near leaves go to lists in LDS in a fixed order, and the
+// lists are dealt to kShares shares in turn, each with a sum of its own,
+// combined in order at the end: the values depend on tree and group alone, not
+// on TEAM.
+//
+// Groups near the surface cost 10 times the mean and there are few groups (1e6
+// queries: 17,500, two for each wave that fits the chip), so that one wave per
+// group ended in a tail as long as the rest: half of the waves were done after
+// 0.55 of 1.06 ms.  Whole calls, one wave per group -> teams: 204,020 elements at
+// 2^20 queries 1.44 -> 1.17 ms, at 2^18 1.10 -> 0.75, at 10^4 3.0 -> 1.0, at 1000
+// 19.8 -> 4.9; 1000 elements at 1000 queries 0.22 -> 0.15.
+constexpr int kShares = 16;
+constexpr int kWidth = 512;         // candidates tested at once
+constexpr int kFarList = 1024;      // the lists are evaluated from here on
+constexpr int kNearList = 256;
+// Stack: a pop takes at most (kTeamSoft - top) / 7 nodes near the soft limit, so a
+// push of <= 8 children each stays under kTeamStack.
+constexpr int kTeamSoft = 2048;
+constexpr int kTeamStack = kTeamSoft + 8 * 24;
+constexpr int kLeafRun = 4;         // consecutive leaves of a share
+constexpr int kBigLeaf = 128;       // a leaf of more elements is dealt 64 at a time
+
+// Teams of 16 up to kWideQueries queries: few groups, so that each should be short
+// (against teams of 8, 204,020 elements at 10^4 queries 1.03 and 1.55 ms, at 2^18 0.75
+// and 0.78); above, teams of 8, which wait less at barriers (2^20: 1.17 against 1.36).
+constexpr int64_t kWideQueries = int64_t{1} << 18;
+
+template <int TEAM>
+__global__ __launch_bounds__(64 * TEAM) __attribute__((amdgpu_waves_per_eu(8))) void k_wn_walk(
+    WnArgs A) {
+  static_assert(64 * TEAM >= kWidth && kShares % TEAM == 0, "team size");
+  __shared__ int s_stack[kTeamStack];
+  __shared__ int s_far[kFarList + kWidth + kChunk];
+  __shared__ int2 s_near[kNearList + kWidth];
+  __shared__ float s_sum[kShares][64];
+  __shared__ int s_cnt[2][TEAM];
+  __shared__ unsigned long long s_pairs[TEAM];  // statistics
+  __shared__ int s_claim;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int num_groups = A.qhdr->num_groups, num_nodes = A.hdr->num_nodes;
+  unsigned long long n_far = 0, n_groups = 0;
+  if (lane == 0) s_pairs[w] = 0;
+  // thread 0 claims groups, one ahead of its use: eighth by eighth from the
+  // block's own XCD's on (see next_group)
   int tries = 0;
+  auto claim = [&]() {
+    for (; tries < 8; ++tries) {
+      const int q = (static_cast<int>(blockIdx.x & 7u) + tries) & 7;
+      const int2 r = eighth_range(num_groups, q);
+      const int t = atomicAdd(&A.qhdr->tq[q], 1);
+      if (t < r.y - r.x) return r.x + t;
+    }
+    return -1;
+  };
+  if (tid == 0) s_claim = claim();
+  __syncthreads();
   while (true) {
-    const int g = next_group(A.qhdr, num_groups, lane, tries);
-    if (g < 0) break;  // every wave reaches this exit
+    const int g = __builtin_amdgcn_readfirstlane(s_claim);
+    if (g < 0) break;  // at most 8 failing claims: every block reaches this exit
     const int2 grp = A.groups[g];
     const int base = __builtin_amdgcn_readfirstlane(grp.x);
     const int cnt = __builtin_amdgcn_readfirstlane(grp.y);
-    if (cnt < 1 || cnt > 64 || base < 0 || base + cnt > A.m) continue;  // corrupt entry
-    const bool valid = lane < cnt;
-    const int i = base + (valid ? lane : 0);
+    int next = -1;
+    if (tid == 0) next = claim();
+    if (cnt < 1 || cnt > 64 || base < 0 || base + cnt > A.m) {  // corrupt entry
+      __syncthreads();
+      if (tid == 0) s_claim = next;
+      __syncthreads();
+      continue;
+    }
+    const int i = base + (lane < cnt ? lane : 0);
     const float4 q = A.qs[i];
-    const Box box = wave_box(q.x, q.y, q.z);
-    float w = 0.f;
-    constexpr int C = kChunk;
-    auto flush_far = [&](int nfar) {
-      n_far += static_cast<unsigned long long>(nfar) * cnt;
-      const int padded = (nfar + C - 1) & ~(C - 1);
-      if (lane < padded - nfar) far[nfar + lane] = A.sentinel;
-      __builtin_amdgcn_wave_barrier();
-      for (int f0 = 0; f0 < padded; f0 += C) w += wn_far_batch<C>(A, q.x, q.y, q.z, far + f0);
-      __builtin_amdgcn_wave_barrier();
-    };
-    // consecutive near leaves with adjacent element ranges are merged
-    auto flush_near = [&](int nnear) {
-      int b = 0;
-      while (b < nnear) {
-        const int4 t = sload4(A.topo, __builtin_amdgcn_readfirstlane(near[b++]));
-        const int s0 = t.x;
-        int s1 = t.x + t.y;
-        while (b < nnear) {
-          const int4 tn = sload4(A.topo, __builtin_amdgcn_readfirstlane(near[b]));
-          if (tn.x != s1) break;
-          s1 += tn.y;
-          ++b;
+    const Box b = wave_box(q.x, q.y, q.z);
+    for (int v = w; v < kShares; v += TEAM) s_sum[v][lane] = 0.f;
+    int top = 1, nfar = 0, nnear = 0, iters = 0;
+    if (tid == 0) s_stack[0] = 0;
+    __syncthreads();
+    while (true) {
+      // (every node is pushed at most once and each round pops at least one)
+      if (top > 0 && iters++ > num_nodes) top = 0;
+      if (top > 0) {
+        int k = min(kWidth, top);
+        k = min(k, max(1, (kTeamSoft - top) / 7));
+        top -= k;
+        int node = -1, kind = 0, nch = 0, incl = 0;
+        int4 t = make_int4(0, 0, 0, 0);
+        if (w * 64 < k) {  // (waves without a candidate only keep the counts)
+          node = tid < k ? s_stack[top + tid] : -1;
+          const bool have = node >= 0 && node < num_nodes;
+          const int nd = have ? node : 0;
+          const float4 m = A.mp[nd];
+          const float4 gg = A.geo[nd];
+          t = A.topo[nd];
+          if (have && m.w != 0.0f) {
+            if (group_accept(b.lx, b.ly, b.lz, b.hx, b.hy, b.hz, gg, A.beta))
+              kind = 1;
+            else if (t.w == 0)
+              kind = 2;
+            else
+              nch = t.w;
+          }
+          incl = wave_incl_scan(nch);
         }
-        s1 = __builtin_amdgcn_readfirstlane(s1);  // wave-uniform: keeps element loads scalar
-        n_near += static_cast<unsigned long long>(s1 - s0) * cnt;
-        int j0 = s0;
-        for (; j0 + kChunk <= s1; j0 += kChunk)
-          w += wn_near_batch<false>(A, q.x, q.y, q.z, j0, s1);
-        if (j0 < s1) w += wn_near_batch<true>(A, q.x, q.y, q.z, j0, s1);
+        // per wave: accepted nodes | near leaves << 11; children
+        const uint64_t bf = __ballot(kind == 1), bn = __ballot(kind == 2);
+        if (lane == 63) {
+          s_cnt[0][w] = __popcll(bf) | __popcll(bn) << 11;
+          s_cnt[1][w] = incl;
+        }
+        __syncthreads();  // the popped entries are read, the counts written
+        const int sum0 = wave_incl_scan(lane < TEAM ? s_cnt[0][lane] : 0);
+        const int sum1 = wave_incl_scan(lane < TEAM ? s_cnt[1][lane] : 0);
+        const int all0 = __builtin_amdgcn_readlane(sum0, TEAM - 1);
+        const int pushed = __builtin_amdgcn_readlane(sum1, TEAM - 1);
+        const int pre0 = w > 0 ? __builtin_amdgcn_readlane(sum0, w - 1) : 0;
+        const int pre1 = w > 0 ? __builtin_amdgcn_readlane(sum1, w - 1) : 0;
+        if (kind == 1) s_far[nfar + (pre0 & 2047) + lanes_below(bf)] = node;
+        if (kind == 2) s_near[nnear + (pre0 >> 11) + lanes_below(bn)] = make_int2(t.x, t.y);
+        nfar += all0 & 2047;
+        nnear += all0 >> 11;
+        if (top + pushed > kTeamStack) {  // unreachable for depth <= 10
+          if (tid == 0) atomicOr(&A.qhdr->overflow, 4);
+          top = 0;
+        } else {
+          int* dst = s_stack + (top + pre1 + incl - nch);
+          for (int c = 0; c < nch; ++c) dst[c] = t.z + c;
+          top += pushed;
+        }
+        __syncthreads();  // entries and lists written, the counts read
       }
-    };
-    traverse<false>(A.hdr, &A.qhdr->overflow, A.topo, A.geo, A.mp, A.beta, box, lane, 0,
-                    stack, far, near, flush_far, flush_near);
-    if (valid) A.out[A.qperm[i]] = w * kInvFourPi;
+      if (top > 0 && nfar < kFarList && nnear < kNearList) continue;
+      // evaluate the lists
+      const int runs = (nfar + kChunk - 1) / kChunk;
+      if (tid < runs * kChunk - nfar) s_far[nfar + tid] = A.sentinel;
+      __syncthreads();
+      if (w == 0) n_far += static_cast<unsigned long long>(nfar) * cnt;
+#pragma unroll 1
+      for (int v = w; v < kShares; v += TEAM) {
+        float sum = 0.f;
+#pragma unroll 1
+        for (int run = v; run < runs; run += kShares)
+          sum += wn_far_batch<kChunk>(A, q.x, q.y, q.z, s_far + run * kChunk);
+        int near = 0;
+#pragma unroll 1
+        for (int e0 = v * kLeafRun; e0 < nnear; e0 += kShares * kLeafRun) {
+          const int e_end = min(e0 + kLeafRun, nnear);
+          int e = e0;
+          while (e < e_end) {
+            // leaves whose elements adjoin, as one range
+            const int s0 = __builtin_amdgcn_readfirstlane(s_near[e].x);
+            int s1 = s0;
+            do {
+              const int c = __builtin_amdgcn_readfirstlane(s_near[e].y);
+              if (c > kBigLeaf) break;
+              s1 += c;
+              ++e;
+            } while (e < e_end && __builtin_amdgcn_readfirstlane(s_near[e].x) == s1);
+            if (s1 == s0) {  // a large leaf (leaves are not empty): dealt below
+              ++e;
+              continue;
+            }
+            near += s1 - s0;
+            sum += wn_range(A, q.x, q.y, q.z, s0, s1);
+          }
+        }
+        // large leaves (elements that share a cell at the depth limit, or a large
+        // leaf size), 64 elements at a time
+#pragma unroll 1
+        for (int e = 0; e < nnear; ++e) {
+          const int s0 = __builtin_amdgcn_readfirstlane(s_near[e].x);
+          const int s1 = s0 + __builtin_amdgcn_readfirstlane(s_near[e].y);
+          if (s1 - s0 <= kBigLeaf) continue;
+#pragma unroll 1
+          for (int j = s0 + 64 * v; j < s1; j += 64 * kShares) {
+            const int j1 = min(j + 64, s1);
+            near += j1 - j;
+            sum += wn_range(A, q.x, q.y, q.z, j, j1);
+          }
+        }
+        if (lane == 0) s_pairs[w] += static_cast<unsigned long long>(near) * cnt;
+        s_sum[v][lane] += sum;
+      }
+      nfar = nnear = 0;
+      __syncthreads();  // the lists are read, the sums written
+      if (top == 0) break;
+    }
+    if (w == 0 && lane < cnt) {
+      float v = 0.f;
+      for (int k = 0; k < kShares; ++k) v += s_sum[k][lane];
+      A.out[A.qperm[i]] = v * kInvFourPi;
+    }
     ++n_groups;
+    if (tid == 0) s_claim = next;
+    __syncthreads();  // the sums are read, the claim written
   }
   if (A.stats && lane == 0) {
-    atomicAdd(&A.qhdr->stats[0], n_far);
-    atomicAdd(&A.qhdr->stats[1], n_near);
-    atomicAdd(&A.qhdr->stats[2], n_groups);
+    if (w == 0) {
+      atomicAdd(&A.qhdr->stats[0], n_far);
+      atomicAdd(&A.qhdr->stats[2], n_groups);
+    }
+    atomicAdd(&A.qhdr->stats[1], s_pairs[w]);
   }
 }
 
@@ -301,12 +452,17 @@ extern "C" int sbh_winding_number(void* stream, const SbhBuffer* points, const S
     A.beta = beta;
     A.out = static_cast<float*>(out->data);
     A.stats = stats != nullptr;
-    const unsigned grid = grid_for(m, 64 * tree::gw::kWavesPerBlock, 256 * 8);
+    // a block per 64 queries up to what fits the chip (32 waves a CU)
+    const bool wide = m <= tree::kWideQueries;
+    const unsigned grid = grid_for(m, 64, 256 * 32 / (wide ? 16 : 8));
     if (profiled) {
       SBH_HIP_TRY(hipEventRecord(pr.rec().ev[1], s));
       SBH_HIP_TRY(hipEventRecord(pr.rec().ev[2], s));
     }
-    tree::k_wn_walk<<<grid, tree::gw::kB, 0, s>>>(A);
+    if (wide)
+      tree::k_wn_walk<16><<<grid, 64 * 16, 0, s>>>(A);
+    else
+      tree::k_wn_walk<8><<<grid, 64 * 8, 0, s>>>(A);
     SBH_LAUNCH_CHECK();
     if (profiled) {
       SBH_HIP_TRY(hipEventRecord(pr.rec().ev[3], s));
