@@ -14,8 +14,9 @@
 // Children that are leaves are summed exactly.  Its expectation is the exact
 // sum over the subdomain (the differences telescope).
 //
-// Wave64 design: one wavefront per query group (<= 64 queries of a query
-// tree cell, the groups of the classic walk).  The group shares every draw
+// Wave64 design: a query group (<= 64 queries of a query tree cell, the groups
+// of the classic walk) is one query per lane, its subdomains dealt to the waves
+// of a block.  The group shares every draw
 // -- the sampled source and the roulette uniforms, Philox4x32-10 keyed by
 // (seed, first sorted query of the group, subdomain node, sample, step) --
 // so all lanes walk ONE path per (subdomain, sample): the nodes, children
@@ -253,23 +254,50 @@ __device__ __forceinline__ float centre_ratio(const Q& L, float4 g) {
   return sqrtf(dx * dx + dy * dy + dz * dz) / g.w;
 }
 
-// Persistent waves over the query groups (XCD-aware queue of groupwalk.hpp).
-template <int KIND, bool QUAD>
-__global__ __launch_bounds__(kB) void k_stoch_walk(StochArgs A) {
+// Persistent blocks over the query groups (XCD-aware queue of groupwalk.hpp), the
+// TEAM waves of a block sharing a group: subdomain number sd belongs to share
+// sd mod kShares, a wave takes every TEAM-th share, and the shares are added in
+// order, so that the values do not depend on TEAM.
+//
+// Bound by VALU and scalar issue (the draws) once the chip is full.  With a wave
+// per group, 262,144 queries made 4400 groups for 4096 resident waves, and the
+// // second round was nearly empty; subdomains differ, too.  Forces of 262,144 points
+// 1.89 -> 1.57 ms in all, 65,536 1.00 -> 0.50, 4000 0.43 -> 0.22, 2^20 8.96 -> 8.72.
+constexpr int kShares = 16;
+constexpr int kTeam = 4;
+// Teams of 16 up to here (16,000 queries 0.26 ms against 0.34 with 4), where the groups
+// do not fill the chip; of 4 above (65,536: 0.50 against 0.54; 262,144: 1.57 against
+// 2.0, a block of 16 waves being alone on its CU).
+constexpr int64_t kWideQueries = 32768;
+
+template <int KIND, bool QUAD, int TEAM>
+__global__ __launch_bounds__(64 * TEAM) void k_stoch_walk(StochArgs A) {
+  static_assert(kShares % TEAM == 0, "team size");
   constexpr bool kVec = KIND != kSWn;
+  __shared__ float s_sum[kShares][kVec ? 3 : 1][64];
+  __shared__ int s_claim;
   const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int num_groups = A.qhdr->num_groups;
   const int nsub = __builtin_amdgcn_readfirstlane(A.subs[0]);
   const float inv_s = A.samples > 0 ? 1.0f / static_cast<float>(A.samples) : 0.0f;
   unsigned long long n_node = 0, n_pair = 0, n_groups = 0;
   int tries = 0;
   while (true) {
-    const int g = next_group(A.qhdr, num_groups, lane, tries);
-    if (g < 0) break;  // every wave reaches this exit
+    if (w == 0) {
+      const int claim = next_group(A.qhdr, num_groups, lane, tries);
+      if (lane == 0) s_claim = claim;
+    }
+    __syncthreads();
+    const int g = __builtin_amdgcn_readfirstlane(s_claim);
+    if (g < 0) break;  // every block reaches this exit
     const int2 grp = A.groups[g];
     const int base = __builtin_amdgcn_readfirstlane(grp.x);
     const int cnt = __builtin_amdgcn_readfirstlane(grp.y);
-    if (cnt < 1 || cnt > 64 || base < 0 || base + cnt > A.m) continue;  // corrupt entry
+    if (cnt < 1 || cnt > 64 || base < 0 || base + cnt > A.m) {  // corrupt entry
+      __syncthreads();
+      continue;
+    }
     const bool valid = lane < cnt;
     const int i = base + (valid ? lane : 0);
     Q L;
@@ -287,101 +315,105 @@ __global__ __launch_bounds__(kB) void k_stoch_walk(StochArgs A) {
       }
     }
     const uint32_t key = static_cast<uint32_t>(base);
-    float tx = 0.f, ty = 0.f, tz = 0.f;
     unsigned long long w_node = 0, w_pair = 0;  // terms this wave evaluates
-    for (int sd = 0; sd < nsub; ++sd) {
-      const int k = __builtin_amdgcn_readfirstlane(A.subs[1 + sd]);
-      const int4 t = sload4(A.topo, k);
-      if (t.w == 0) {
-        leaf_sum<KIND>(A, t.x, t.x + t.y, L, tx, ty, tz);
-        w_pair += static_cast<unsigned>(t.y);
-        continue;
-      }
-      node_term<KIND, QUAD>(A, k, L, tx, ty, tz);
-      ++w_node;
-      if (A.samples <= 0) continue;
-      const float4 g0 = sload4(A.geo, k);
-      const uint32_t n_sub = static_cast<uint32_t>(t.y);
-      float sx = 0.f, sy = 0.f, sz = 0.f;
-      for (int s = 0; s < A.samples; ++s) {
-        const float u0 = sbh_uniform(A.seed, key, static_cast<uint32_t>(k),
-                                     static_cast<uint32_t>(s), 0u);
-        const uint32_t sidx = __builtin_amdgcn_readfirstlane(
-            min(static_cast<uint32_t>(static_cast<float>(n_sub) * u0) +
-                    static_cast<uint32_t>(t.x),
-                static_cast<uint32_t>(t.x + t.y - 1)));
-        int cur = k;
-        int4 tc = t;
-        float4 gc = g0;
-        float ep = 1.0f;
-        bool alive = valid;
-        float cur_beta = fmaxf(A.beta, centre_ratio(L, gc));
-        float wx = 0.f, wy = 0.f, wz = 0.f;
-        uint32_t step = 1;
-        while (tc.w > 0 && step < 64) {
-          const float ratio = centre_ratio(L, gc);
-          float tp;
-          {
-#pragma clang fp contract(off)
-            tp = fminf(cur_beta / ratio, 1.0f);
-          }
-          const float pu = sbh_uniform(A.seed, key, static_cast<uint32_t>(k),
-                                       static_cast<uint32_t>(s), step++);
-          alive = alive && !(pu > tp);
-          if (__ballot(alive) == 0ull) break;  // every lane has stopped
-          if (alive) ep *= tp;
-          const int prev = cur;
-          const int fc = __builtin_amdgcn_readfirstlane(tc.z);
-          const int nch = __builtin_amdgcn_readfirstlane(tc.w);
-          const int cnt_prev = __builtin_amdgcn_readfirstlane(tc.y);
-          // the child holding the sampled source (children partition the range)
-          int nxt = fc;
-          for (int c = 1; c < nch; ++c)
-            if (static_cast<uint32_t>(sload4(A.topo, fc + c).x) <= sidx) nxt = fc + c;
-          cur = __builtin_amdgcn_readfirstlane(nxt);
-          cur_beta = fmaxf(cur_beta, ratio);
-          // sum of prev's children minus prev's own term
-          float cx = 0.f, cy = 0.f, cz = 0.f;
-          for (int c = 0; c < nch; ++c) {
-            const int4 tk = sload4(A.topo, fc + c);
-            if (tk.w == 0) {
-              leaf_sum<KIND>(A, tk.x, tk.x + tk.y, L, cx, cy, cz);
-              w_pair += static_cast<unsigned>(tk.y);
-            } else {
-              node_term<KIND, QUAD>(A, fc + c, L, cx, cy, cz);
-              ++w_node;
-            }
-          }
-          float px = 0.f, py = 0.f, pz = 0.f;
-          node_term<KIND, QUAD>(A, prev, L, px, py, pz);
-          ++w_node;
-          const float w =
-              alive ? static_cast<float>(n_sub) / (ep * static_cast<float>(cnt_prev)) : 0.0f;
-          wx += w * (cx - px);
-          if constexpr (kVec) {
-            wy += w * (cy - py);
-            wz += w * (cz - pz);
-          }
-          tc = sload4(A.topo, cur);
-          gc = sload4(A.geo, cur);
+    for (int v = w; v < kShares; v += TEAM) {
+      float tx = 0.f, ty = 0.f, tz = 0.f;
+      for (int sd = v; sd < nsub; sd += kShares) {
+        const int k = __builtin_amdgcn_readfirstlane(A.subs[1 + sd]);
+        const int4 t = sload4(A.topo, k);
+        if (t.w == 0) {
+          leaf_sum<KIND>(A, t.x, t.x + t.y, L, tx, ty, tz);
+          w_pair += static_cast<unsigned>(t.y);
+          continue;
         }
-        sx += wx;
-        sy += wy;
-        sz += wz;
+        node_term<KIND, QUAD>(A, k, L, tx, ty, tz);
+        ++w_node;
+        if (A.samples <= 0) continue;
+        const float4 g0 = sload4(A.geo, k);
+        const uint32_t n_sub = static_cast<uint32_t>(t.y);
+        float sx = 0.f, sy = 0.f, sz = 0.f;
+        for (int s = 0; s < A.samples; ++s) {
+          const float u0 = sbh_uniform(A.seed, key, static_cast<uint32_t>(k),
+                                       static_cast<uint32_t>(s), 0u);
+          const uint32_t sidx = __builtin_amdgcn_readfirstlane(
+              min(static_cast<uint32_t>(static_cast<float>(n_sub) * u0) +
+                      static_cast<uint32_t>(t.x),
+                  static_cast<uint32_t>(t.x + t.y - 1)));
+          int cur = k;
+          int4 tc = t;
+          float4 gc = g0;
+          float ep = 1.0f;
+          bool alive = valid;
+          float cur_beta = fmaxf(A.beta, centre_ratio(L, gc));
+          float wx = 0.f, wy = 0.f, wz = 0.f;
+          uint32_t step = 1;
+          while (tc.w > 0 && step < 64) {
+            const float ratio = centre_ratio(L, gc);
+            float tp;
+            {
+  #pragma clang fp contract(off)
+              tp = fminf(cur_beta / ratio, 1.0f);
+            }
+            const float pu = sbh_uniform(A.seed, key, static_cast<uint32_t>(k),
+                                         static_cast<uint32_t>(s), step++);
+            alive = alive && !(pu > tp);
+            if (__ballot(alive) == 0ull) break;  // every lane has stopped
+            if (alive) ep *= tp;
+            const int prev = cur;
+            const int fc = __builtin_amdgcn_readfirstlane(tc.z);
+            const int nch = __builtin_amdgcn_readfirstlane(tc.w);
+            const int cnt_prev = __builtin_amdgcn_readfirstlane(tc.y);
+            // the child holding the sampled source (children partition the range)
+            int nxt = fc;
+            for (int c = 1; c < nch; ++c)
+              if (static_cast<uint32_t>(sload4(A.topo, fc + c).x) <= sidx) nxt = fc + c;
+            cur = __builtin_amdgcn_readfirstlane(nxt);
+            cur_beta = fmaxf(cur_beta, ratio);
+            // sum of prev's children minus prev's own term
+            float cx = 0.f, cy = 0.f, cz = 0.f;
+            for (int c = 0; c < nch; ++c) {
+              const int4 tk = sload4(A.topo, fc + c);
+              if (tk.w == 0) {
+                leaf_sum<KIND>(A, tk.x, tk.x + tk.y, L, cx, cy, cz);
+                w_pair += static_cast<unsigned>(tk.y);
+              } else {
+                node_term<KIND, QUAD>(A, fc + c, L, cx, cy, cz);
+                ++w_node;
+              }
+            }
+            float px = 0.f, py = 0.f, pz = 0.f;
+            node_term<KIND, QUAD>(A, prev, L, px, py, pz);
+            ++w_node;
+            const float w =
+                alive ? static_cast<float>(n_sub) / (ep * static_cast<float>(cnt_prev)) : 0.0f;
+            wx += w * (cx - px);
+            if constexpr (kVec) {
+              wy += w * (cy - py);
+              wz += w * (cz - pz);
+            }
+            tc = sload4(A.topo, cur);
+            gc = sload4(A.geo, cur);
+          }
+          sx += wx;
+          sy += wy;
+          sz += wz;
+        }
+        tx += sx * inv_s;
+        ty += sy * inv_s;
+        tz += sz * inv_s;
       }
-      tx += sx * inv_s;
-      ty += sy * inv_s;
-      tz += sz * inv_s;
-    }
-    if (valid) {
-      const int64_t o = static_cast<int64_t>(A.qperm[i]);
+      s_sum[v][0][lane] = tx;
       if constexpr (kVec) {
-        A.out[3 * o + 0] = tx;
-        A.out[3 * o + 1] = ty;
-        A.out[3 * o + 2] = tz;
-      } else {
-        A.out[o] = tx;
+        s_sum[v][1][lane] = ty;
+        s_sum[v][2][lane] = tz;
       }
+    }
+    __syncthreads();  // the sums are written, the claim is read
+    constexpr int kVals = kVec ? 3 : 1;
+    for (int a = w; a < kVals; a += TEAM) {
+      float t = 0.f;
+      for (int k = 0; k < kShares; ++k) t += s_sum[k][a][lane];
+      if (valid) A.out[kVals * static_cast<int64_t>(A.qperm[i]) + a] = t;
     }
     n_node += w_node * static_cast<unsigned>(cnt);
     n_pair += w_pair * static_cast<unsigned>(cnt);
@@ -390,7 +422,7 @@ __global__ __launch_bounds__(kB) void k_stoch_walk(StochArgs A) {
   if (A.stats && lane == 0) {
     atomicAdd(&A.qhdr->stats[0], n_node);
     atomicAdd(&A.qhdr->stats[1], n_pair);
-    atomicAdd(&A.qhdr->stats[2], n_groups);
+    if (w == 0) atomicAdd(&A.qhdr->stats[2], n_groups);
   }
 }
 
@@ -484,21 +516,29 @@ int run_stoch(int kind, bool quad, hipStream_t s, const float* pts, const float*
     A.seed = static_cast<uint32_t>(seed);
     A.out = out;
     A.stats = stats != nullptr;
-    const unsigned grid = grid_for(m, 64 * kWavesPerBlock, 256 * 8);
+    // a block per 64 queries up to what fits the chip (32 waves a CU)
+    const int team = m <= kWideQueries ? 16 : kTeam;
+    const unsigned grid = grid_for(m, 64, 256 * 32 / team), block = 64 * team;
     if (pr.on()) {
       SBH_HIP_TRY(hipEventRecord(pr.rec().ev[1], s));
       SBH_HIP_TRY(hipEventRecord(pr.rec().ev[2], s));
     }
+    auto walk = [&](auto wide, auto narrow) {
+      if (team == 16)
+        wide<<<grid, block, 0, s>>>(A);
+      else
+        narrow<<<grid, block, 0, s>>>(A);
+    };
     if (kind == kSForce && quad)
-      k_stoch_walk<kSForce, true><<<grid, kB, 0, s>>>(A);
+      walk(k_stoch_walk<kSForce, true, 16>, k_stoch_walk<kSForce, true, kTeam>);
     else if (kind == kSForce)
-      k_stoch_walk<kSForce, false><<<grid, kB, 0, s>>>(A);
+      walk(k_stoch_walk<kSForce, false, 16>, k_stoch_walk<kSForce, false, kTeam>);
     else if (kind == kSVjp && quad)
-      k_stoch_walk<kSVjp, true><<<grid, kB, 0, s>>>(A);
+      walk(k_stoch_walk<kSVjp, true, 16>, k_stoch_walk<kSVjp, true, kTeam>);
     else if (kind == kSVjp)
-      k_stoch_walk<kSVjp, false><<<grid, kB, 0, s>>>(A);
+      walk(k_stoch_walk<kSVjp, false, 16>, k_stoch_walk<kSVjp, false, kTeam>);
     else
-      k_stoch_walk<kSWn, false><<<grid, kB, 0, s>>>(A);
+      walk(k_stoch_walk<kSWn, false, 16>, k_stoch_walk<kSWn, false, kTeam>);
     SBH_LAUNCH_CHECK();
     if (pr.on()) {
       SBH_HIP_TRY(hipEventRecord(pr.rec().ev[3], s));
