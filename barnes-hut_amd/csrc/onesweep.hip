@@ -14,6 +14,8 @@
 //                stages them in LDS sorted by digit and writes them out so
 //                that consecutive threads fill consecutive slots of a digit
 //
+// Up to 4096 keys one launch (k_os_one) does all passes in one block.
+//
 // Code passes move (key, value) pairs, value = input row (the first pass
 // reads the keys in input order and makes the values); set passes move
 // values only, their digit being that of the set holding the row (sets are
@@ -307,6 +309,118 @@ __global__ __launch_bounds__(kBlock) void k_os_pass(
   }
 }
 
+// All passes of a sort of at most kOneBlock * kItems keys by one block: the keys
+// stay in registers and change places through LDS.  A launch and its waits for
+// memory cost more than such a pass (forces of 2003 points 105 -> 88 us, of 4096 126 ->
+// 112); with more keys a thread the one block ranks too long (8192 points 157 and 154
+// us, 10,000 with 16 keys a thread 166 -> 191).  keys_out may be codes.
+constexpr int kOneBlock = 1024;
+constexpr int64_t kOneMax = 4 * kOneBlock;
+
+template <int kItems>
+__global__ __launch_bounds__(kOneBlock) void k_os_one(
+    const uint32_t* codes, int n, int code_passes, int passes,
+    const int32_t* __restrict__ set_offs, int nsets, uint32_t* keys_out,
+    uint32_t* __restrict__ vals_out) {
+  constexpr int kWaveCount = kOneBlock / 64;
+  __shared__ uint32_t s_wcnt[kWaveCount][kRadix];
+  __shared__ uint32_t s_lstart[kRadix];
+  __shared__ uint32_t s_wave[kRadix / 64];
+  __shared__ uint32_t s_key[kOneBlock * kItems];
+  __shared__ uint32_t s_val[kOneBlock * kItems];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+  const int run = wave * (64 * kItems) + lane;  // a wave's keys are consecutive
+  uint32_t key[kItems], val[kItems], dig[kItems], loc[kItems];
+#pragma unroll
+  for (int r = 0; r < kItems; ++r) {
+    const int i = run + r * 64;
+    key[r] = i < n ? codes[i] : 0u;
+    val[r] = static_cast<uint32_t>(i);
+  }
+  for (int p = 0; p < passes; ++p) {
+    for (int k = tid; k < kWaveCount * kRadix; k += kOneBlock) (&s_wcnt[0][0])[k] = 0u;
+    const int shift = 8 * (p < code_passes ? p : p - code_passes);
+#pragma unroll
+    for (int r = 0; r < kItems; ++r) {
+      const bool ok = run + r * 64 < n;
+      uint32_t d = key[r];
+      if (p >= code_passes) d = ok ? static_cast<uint32_t>(row_set(set_offs, nsets, val[r])) : 0u;
+      dig[r] = ok ? (d >> shift) & 255u : kRadix;
+    }
+    __syncthreads();
+    // ranks within the wave, as in k_os_pass
+#pragma unroll
+    for (int r = 0; r < kItems; ++r) {
+      const bool ok = dig[r] < kRadix;
+      uint64_t peers = __ballot(ok);
+#pragma unroll
+      for (int b = 0; b < 8; ++b) {
+        const bool bit = (dig[r] >> b) & 1u;
+        const uint64_t bal = __ballot(bit);
+        peers &= bit ? bal : ~bal;
+      }
+      const uint32_t rank = static_cast<uint32_t>(__popcll(peers & lt));
+      const uint32_t have = ok ? s_wcnt[wave][dig[r]] : 0u;
+      loc[r] = have + rank;
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      if (ok && rank == 0) s_wcnt[wave][dig[r]] = have + static_cast<uint32_t>(__popcll(peers));
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+    // each wave's counts become the keys of the digit before its own; digit starts
+    uint32_t mine = 0, incl = 0;
+    if (tid < kRadix) {
+#pragma unroll
+      for (int w = 0; w < kWaveCount; ++w) {
+        const uint32_t c = s_wcnt[w][tid];
+        s_wcnt[w][tid] = mine;
+        mine += c;
+      }
+      incl = mine;
+      for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t t = __shfl_up(incl, d, 64);
+        if (lane >= d) incl += t;
+      }
+      if (lane == 63) s_wave[wave] = incl;
+    }
+    __syncthreads();
+    if (tid < kRadix) {
+      uint32_t before = 0;
+      for (int w = 0; w < wave; ++w) before += s_wave[w];
+      s_lstart[tid] = before + incl - mine;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kItems; ++r) {
+      if (dig[r] < kRadix) {
+        const uint32_t dst = s_lstart[dig[r]] + s_wcnt[wave][dig[r]] + loc[r];
+        s_key[dst] = key[r];
+        s_val[dst] = val[r];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kItems; ++r) {
+      const int i = run + r * 64;
+      if (i < n) {
+        key[r] = s_key[i];
+        val[r] = s_val[i];
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < kItems; ++r) {
+    const int i = run + r * 64;
+    if (i < n) {
+      keys_out[i] = key[r];
+      vals_out[i] = val[r];
+    }
+  }
+}
+
 }  // namespace
 
 size_t morton_sort_temp_bytes(int64_t n, int nsets) {
@@ -328,6 +442,20 @@ int morton_sort(hipStream_t s, const uint32_t* codes, int64_t n, int key_bits,
   while (nsets > 1 && (int64_t{1} << (8 * set_passes)) < nsets) ++set_passes;
   const int passes = code_passes + set_passes;
   if (code_passes > 4 || passes > kMaxPasses) return fail_invalid("sort key too wide");
+  if (n <= kOneMax) {
+    auto one = [&](auto kernel) {
+      kernel<<<1, kOneBlock, 0, s>>>(codes, static_cast<int>(n), code_passes, passes, set_offs,
+                                     nsets, keys_b, vals_b);
+    };
+    if (n <= 2 * kOneBlock)
+      one(k_os_one<2>);
+    else
+      one(k_os_one<4>);
+    SBH_LAUNCH_CHECK();
+    *keys = keys_b;
+    *perm = vals_b;
+    return SBH_OK;
+  }
   const OsLayout L = os_layout(n, passes);
   char* t = static_cast<char*>(temp);
   auto* hist = reinterpret_cast<uint32_t*>(t + L.hist);

@@ -9,12 +9,14 @@
 //                 scan -> emit (first and last points of each cell, topo.hpp)
 //   k_topo_finalize  record counts, group sizes, leaf moments (mass, centre of
 //                 mass, central second moment), one wavefront per node
-//   per level:    k_moments_internal bottom-up over the internal nodes
-// Walk (one wave = one group of 64 consecutive sorted points):
+//   per level:    k_moments_internal bottom-up over the internal nodes,
+//                 k_moments_top for the small levels at the end
+// Walks (a group of <= 64 consecutive sorted points by one wave, k_walk, or by a
+//   team of waves, k_walk_team):
 //   a node is used as a multipole for the whole group iff the distance from its
 //   cell centre to the group's bounding box is >= beta * cell diagonal (the
 //   reference's MAC, src/sbh_ffi.cu:1878-1893, made conservative for a group);
-//   rejected leaves are summed exactly.  Lanes test 64 candidate nodes at once;
+//   rejected leaves are summed exactly.  Lanes test candidate nodes side by side;
 //   accepted nodes and near leaves are batched in LDS and evaluated with all 64
 //   lanes sharing each node / source record, which is read once per wave
 //   through the scalar cache (the records are read-only during the walk).

@@ -32,8 +32,8 @@ struct Header {
   int32_t tq[8];       // the teams' work queues, as xq
 };
 
-// Tag of the walk schedule: the group costs in the workspace were measured
-// by a walk over `groups` groups (the tag is checked, never trusted: any
+// Tag of the schedule of the walks by single waves (monopole terms, sets from
+// kSinglePoints on): the group costs in the workspace were measured by a walk over `groups` groups (the tag is checked, never trusted: any
 // cost values give a valid claim order).
 constexpr uint32_t kSchedMagic = 0x5c4ed01eu;
 struct Sched {
@@ -90,8 +90,8 @@ __device__ __forceinline__ int set_of(const int32_t* __restrict__ offs, int nset
   return lo;
 }
 
-// Claim order of the next walk over the query groups of the tree in ws
-// (n points): the groups' own order, or heaviest first within each eighth by
+// Claim order of the next walk by single waves over the query groups of the tree
+// in ws (n points): the groups' own order, or heaviest first within each eighth by
 // the costs the previous walk of the same kind (0: forward-type walks, 1:
 // adjoint walks; else the other kind) measured in this workspace.  *order is
 // the permutation for gw::next_group, *cost where the walk stores each
@@ -143,8 +143,8 @@ int build_forest(hipStream_t s, char* ws, const Layout& L, const float* pts, con
 // ev_walk (may be null): two events recorded immediately before and after the
 // walk kernel on stream s.
 // Works on forests: each group walks the tree of its own set.  walk_blocks
-// (0: default) caps the persistent grid; walk_threads (0: 256, else 64, 128,
-// 256 or 512) sets its block size.
+// (0: default) caps the persistent grids; walk_threads (0: 256, else 64, 128,
+// 256 or 512) sets the block size of the walk by single waves.
 int walk(hipStream_t s, char* ws, const Layout& L, int64_t n, float beta, float softening,
          bool vjp, int order, float* forces, float* grad_points, float* grad_masses,
          bool want_stats, hipEvent_t* ev_walk = nullptr, int walk_blocks = 0,

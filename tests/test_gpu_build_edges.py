@@ -26,11 +26,12 @@ def _points(kind, n, seed):
     return p.astype(np.float32), rng.uniform(0.5, 1.5, n).astype(np.float32)
 
 
-# sort tiles of 1024 keys to 2^15 points, 2048 to 2^17, 4096 above; topology tiles of
-# 1024 points in rounds of 64 tiles; leaf sizes about the window's 2048; internal
-# nodes per level about 512 (at leaf size 16 reached near 8700 points)
+# sorts by one block, 2 keys a thread to 2048 points, 4 to 4096; then tiles of 1024
+# keys to 2^15, 2048 to 2^17, 4096 above; topology tiles of 1024 points in rounds of
+# 64 tiles; leaf sizes about the window's 2048; internal nodes per level about 512 (at leaf size 16 reached near 8700 points)
 @pytest.mark.parametrize("kind,n,depth,leaf", [
-    ("uniform", 1024, 10, 1), ("clumps", 1025, 10, 32), ("repeated", 4097, 10, 8),
+    ("uniform", 1024, 10, 1), ("clumps", 1025, 10, 32), ("repeated", 2048, 10, 8),
+    ("clumps", 2049, 5, 8), ("uniform", 4096, 10, 16), ("repeated", 4097, 10, 8),
     ("uniform", 8703, 10, 16), ("uniform", 8721, 10, 16), ("clumps", 32768, 10, 2048),
     ("clumps", 32769, 10, 2049), ("repeated", 65537, 4, 3000), ("uniform", 131072, 9, 32),
     ("clumps", 131073, 10, 24), ("uniform", 530001, 10, 100),
