@@ -263,8 +263,12 @@ __global__ __launch_bounds__(256) void k_direct_combine(const float* __restrict_
 // 1024 SIMDs (one block per chunk from 131,072 queries on, where the chunks
 // alone give 8 waves), at least 64 sources per wave (below that the wave's
 // start, the combine and its launch, about 4 us, cost more than they save),
-// at most 256 partials per query.
-int direct_blocks(int64_t n, int64_t nq) {
+// at most 256 partials per query.  Up to 1024 sources (512 with attenuation, whose
+// pairs take three times as long) a wave's quarter is short: 1000 sources 14.0 us a call
+// unsplit and 16.4 split, 2048 21 and 16; 700 attenuated 16.4 and 17.1, 1000 22.9 and
+// 16.9.
+int direct_blocks(int64_t n, int64_t nq, bool cut) {
+  if (n <= (cut ? 512 : 1024)) return 1;
   const int64_t chunks = (nq + 63) / 64;
   int64_t y = 2048 / chunks;
   y = y < n / (64 * kSplit) ? y : n / (64 * kSplit);
@@ -283,7 +287,7 @@ int launch_direct_as(hipStream_t s, const float* pts, const float* ms, const flo
                      const PairParams& P) {
   constexpr int C = kComps<KIND>;
   std::lock_guard<std::mutex> lock(g_direct_mu);
-  int blocks = direct_blocks(n, nq);
+  int blocks = direct_blocks(n, nq, CUT);
   float* part = nullptr;
   if (blocks > 1) {
     // unsplit under stream capture (the scratch could need an allocation)

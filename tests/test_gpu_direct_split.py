@@ -49,7 +49,8 @@ def test_attenuation_of_a_pair(gpu, rc):
 # around one source range per wave (64 each) and where the ranges of the last
 # block start beyond the sources; one block per chunk from 131,072 queries on.
 @pytest.mark.parametrize("n,m", [(1, 1), (7, 63), (8, 64), (9, 65), (255, 128), (257, 1),
-                                 (513, 191), (2049, 64), (16385, 3), (300, 131073)])
+                                 (513, 191), (1024, 70), (1025, 70), (2049, 64), (16385, 3),
+                                 (300, 131073)])
 @pytest.mark.parametrize("rc,periodic", [(np.inf, False), (np.inf, True), (0.3, False),
                                          (0.3, True)])
 def test_split_sums_match_oracle(gpu, n, m, rc, periodic):
