@@ -89,11 +89,18 @@ TRAFFIC_PROFILES = [os.path.join(ROOT, "profiles", f) for f in (
     "gravity_walk_plummer_n1048576_quad_hbm_traffic.md")]
 
 
+def walk_kernel(vjp, order, forces):
+    """Kernel of a single set of 2^20 points: monopole walks by single waves, the
+    others by teams of 8 waves."""
+    if order == 1:
+        return f"k_walk<{str(vjp).lower()},{str(forces).lower()},4>"
+    return f"k_walk_team<{str(vjp).lower()},{order},{str(forces).lower()},8>"
+
+
 def profiled_traffic(vjp, order, forces):
-    """HBM bytes per launch of k_walk<vjp, order, forces> at N = 2^20 measured
-    by the rocprofv3 --pmc passes recorded in profiles/, and that file (None,
-    None if not profiled)."""
-    key = f"k_walk<{str(vjp).lower()},{order},{str(forces).lower()}>"
+    """HBM bytes per launch of the walk at N = 2^20 measured by the rocprofv3 --pmc
+    passes recorded in profiles/, and that file (None, None if not profiled)."""
+    key = walk_kernel(vjp, order, forces)
     for path in TRAFFIC_PROFILES:
         try:
             with open(path) as fh:
@@ -457,11 +464,11 @@ def bench_gravity(args):
     ms_step = graph_ms if graph_ms is not None else eager_ms
     value = n / (ms_step * 1e-3)
 
-    # Each walk deals its query groups heaviest first by the costs that the
-    # previous walk of its kind over the same workspace measured (only the
+    # The monopole walks of a large set deal their query groups heaviest first by the
+    # costs that the previous one over the same workspace measured (only the
     # schedule depends on them).  A fresh workspace has none: its forward walk
-    # takes the groups in their own order and its adjoint walk orders by that
-    # forward walk's costs.  The first step on each of 3 zeroed workspaces:
+    # takes the groups in their own order.  The first step on each of 3 zeroed
+    # workspaces:
     cold = []
     for _ in range(3):
         wsc = torch.zeros_like(ws)
@@ -473,10 +480,10 @@ def bench_gravity(args):
         cold.append(ev0.elapsed_time(ev1))
         del wsc
     schedule = {"first_step_on_fresh_workspace_ms": float(np.mean(cold)),
-                "note": "timed steps reuse one workspace: each walk orders its groups by "
-                        "the costs the previous walk of its kind measured (heaviest "
-                        "first within each eighth of the groups); results do not depend "
-                        "on the order"}
+                "note": "timed steps reuse one workspace: the monopole walks of a "
+                        "large set order their groups by the costs the previous one "
+                        "measured (heaviest first within each eighth of the groups); "
+                        "results do not depend on the order"}
 
     # interaction counts (deterministic: identical every step)
     sf, sv = G.new_stats(dev), G.new_stats(dev)
@@ -609,7 +616,7 @@ def bench_gravity(args):
         "other_orders": alts,
         "direct_sum": direct,
         "roofline": valu_roofline(
-            f"k_walk<vjp=1,order={args.order},forces=0>", flops_vjp, flops_vjp_impl,
+            walk_kernel(True, args.order, False), flops_vjp, flops_vjp_impl,
             walk_vjp_ms,
             traffic=vjp_traffic[0],
             traffic_source=vjp_traffic[1],
@@ -661,10 +668,10 @@ def other_rooflines(args, n, sf, walk_fwd_ms, flops_fwd, flops_fwd_impl, prof, d
         out[tag] = {"bound": "hbm", "achieved": gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                     "frac": gbs / HBM_PEAK_GBS, "bytes": b, "ms": ms,
                     "design_bytes": build_bytes_design(n, sf["nodes"], vjp),
-                    "note": "24 dependent launches per build (10 of them the internal "
+                    "note": "21 dependent launches per build (7 of them the internal "
                             "moment levels); launch latency and the radix passes' "
                             "look-back set the time, not bandwidth"}
-    out["walk_fwd"] = valu_roofline(f"k_walk<vjp=0,order={args.fwd_order},forces=1>",
+    out["walk_fwd"] = valu_roofline(walk_kernel(False, args.fwd_order, True),
                                     flops_fwd, flops_fwd_impl, walk_fwd_ms,
                                     traffic=(profiled_traffic(False, args.fwd_order, True)[0]
                                              if n == 1 << 20 else None))
@@ -1677,7 +1684,7 @@ def measure_batched(args, dev, tune=True, cpu=False):
                          "vjp_build": prof[4] / max(prof[3], 1),
                          "vjp_walk_kernel": walk_vjp_ms},
            "roofline": valu_roofline(
-               f"k_walk<vjp=1,order={vjp_order},forces=0> (all sets)", flops_vjp,
+               walk_kernel(True, vjp_order, False) + " (all sets)", flops_vjp,
                flops_vjp_impl, walk_vjp_ms)}
     if cpu:
         big_args = argparse.Namespace(**vars(args))

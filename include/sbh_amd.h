@@ -538,9 +538,10 @@ int sbh_gravity_force_vjp(void* stream, const SbhBuffer* points,
  * set (the persistent walk drains the groups of all sets from one queue).
  * Per set, results equal sbh_gravity_force / sbh_gravity_force_vjp on that
  * set alone.  Offsets that do not rise from 0 to N leave every set empty and
- * set stats[5] (overflow) to 2.  walk_blocks: persistent walk grid in
- * blocks (0 = default, 8192 waves); walk_threads: its block size, 64, 128,
- * 256 or 512 (0 = 256).  No reference counterpart (the reference runs one launch per
+ * set stats[5] (overflow) to 2.  walk_blocks: cap on the persistent walk
+ * grids in blocks (0 = default); walk_threads: block size of the monopole walk of
+ * sets from 700,000 points on, 64, 128, 256 or 512 (0 = 256); the other walks run in
+ * blocks of their own size.  No reference counterpart (the reference runs one launch per
  * call, python/benchmark_octree8.py). */
 int64_t sbh_gravity_batch_workspace_bytes(int64_t total_points, int32_t num_sets,
                                           int32_t max_depth, int32_t leaf_size);
