@@ -1352,9 +1352,8 @@ __device__ __forceinline__ Lane load_lane(const WalkArgs& A, int base, int cnt, 
   return L;
 }
 
-// One query group (sorted points [base, base + cnt)) by one wave, monopole
-// terms.
-template <bool VJP, bool FORCES>
+// One query group (sorted points [base, base + cnt)) by one wave.
+template <bool VJP, int ORDER, bool FORCES>
 __device__ __forceinline__ void walk_group(const WalkArgs& A, int base, int cnt, int lane,
                                            int* stack, int* far, int* near, float* red,
                                            unsigned long long& n_far,
@@ -1378,8 +1377,9 @@ __device__ __forceinline__ void walk_group(const WalkArgs& A, int base, int cnt,
       for (; f0 + 2 * kChunk <= padded; f0 += 2 * kChunk)
         far_batch<VJP, 1, FORCES, 2 * kChunk>(A, L, far + f0, lane, fx, fy, fz, gx, gy, gz);
     }
-    for (; f0 < padded; f0 += kChunk)
-      far_batch<VJP, 1, FORCES, kChunk>(A, L, far + f0, lane, fx, fy, fz, gx, gy, gz);
+    constexpr int C = ORDER == 1 ? kChunk : kChunk / 2;
+    for (; f0 < padded; f0 += C)
+      far_batch<VJP, ORDER, FORCES, C>(A, L, far + f0, lane, fx, fy, fz, gx, gy, gz);
     __builtin_amdgcn_wave_barrier();
   };
 
@@ -1399,14 +1399,14 @@ __device__ __forceinline__ void walk_group(const WalkArgs& A, int base, int cnt,
         ++b;
       }
       s1 = __builtin_amdgcn_readfirstlane(s1);  // wave-uniform: keeps source loads scalar
-      near_range<VJP, 1, FORCES>(A, L, i, base, cnt, s0, s1, lane, fx, fy, fz, gx, gy, gz,
-                                 n_near);
+      near_range<VJP, ORDER, FORCES>(A, L, i, base, cnt, s0, s1, lane, fx, fy, fz, gx, gy, gz,
+                                     n_near);
     }
   };
 
   const int root = A.nsets > 1 ? set_of(A.offs, A.nsets, base) : 0;
-  traverse(A.hdr, &A.hdr->overflow, A.topo, A.geo, A.mp, A.beta, box, lane, root, stack,
-                 far, near, flush_far, flush_near);
+  traverse(A.hdr, &A.hdr->overflow, A.topo, A.geo, A.mp, A.beta, box, lane, root, stack, far,
+           near, flush_far, flush_near);
 
   if (lane < cnt) {
     const int64_t o = static_cast<int64_t>(A.perm[i]);
@@ -1514,8 +1514,9 @@ __global__ __launch_bounds__(1024) void k_group_order(Header* __restrict__ hdr,
 // it is up to 9% faster than the teams below, whose lists are padded and merged
 // in smaller pieces (2^20 points, Plummer / uniform / blobs: forces 6.6, 4.1, 3.4
 // against 7.1, 4.45, 3.6 ms, adjoint 16.1, 9.5, 7.8 against 16.6, 10.1, 8.0;
-// at 500,000 points forces 3.8, 2.06, 1.62 against 3.5, 1.95, 1.54).
-template <bool VJP, bool FORCES, int WPB>
+// at 500,000 points forces 3.8, 2.06, 1.62 against 3.5, 1.95, 1.54).  Also the
+// adjoints from kAlonePoints on.
+template <bool VJP, int ORDER, bool FORCES, int WPB>
 __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(VJP ? 4 : 7))) void k_walk(
     WalkArgs A) {
   __shared__ int s_stack[WPB][kRunStackWords];
@@ -1541,10 +1542,10 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(VJP ? 
     const int cnt = __builtin_amdgcn_readfirstlane(grp.y);
     if (cnt < 1 || cnt > 64 || base < 0 || base + cnt > A.n) continue;  // corrupt entry
     const uint64_t t0 = __builtin_amdgcn_s_memtime();
-    walk_group<VJP, FORCES>(A, base, cnt, lane, s_stack[w], s_far[w], s_near[w], s_red[w], n_far,
-                            n_near);
+    walk_group<VJP, ORDER, FORCES>(A, base, cnt, lane, s_stack[w], s_far[w], s_near[w], s_red[w],
+                                   n_far, n_near);
     const uint64_t t1 = __builtin_amdgcn_s_memtime();
-    if (lane == 0) A.gcost[g] = static_cast<float>(t1 - t0);
+    if (lane == 0 && A.gcost != nullptr) A.gcost[g] = static_cast<float>(t1 - t0);
     ++n_groups;
   }
   if (A.stats != nullptr && lane == 0) {
@@ -2143,15 +2144,28 @@ void launch_team(hipStream_t s, unsigned grid, bool vjp, int order, bool f, cons
 }
 
 template <int WPB>
-void launch_walk(hipStream_t s, unsigned grid, bool vjp, bool f, const WalkArgs& A) {
+void launch_walk(hipStream_t s, unsigned grid, bool vjp, int order, bool f, const WalkArgs& A) {
   const unsigned block = 64 * WPB;
   if (vjp && f)
-    k_walk<true, true, WPB><<<grid, block, 0, s>>>(A);
+    k_walk<true, 1, true, WPB><<<grid, block, 0, s>>>(A);
+  else if (vjp && order == 2)
+    k_walk<true, 2, false, WPB><<<grid, block, 0, s>>>(A);
+  else if (vjp && order == 3)
+    k_walk<true, 3, false, WPB><<<grid, block, 0, s>>>(A);
   else if (vjp)
-    k_walk<true, false, WPB><<<grid, block, 0, s>>>(A);
+    k_walk<true, 1, false, WPB><<<grid, block, 0, s>>>(A);
   else
-    k_walk<false, true, WPB><<<grid, block, 0, s>>>(A);
+    k_walk<false, 1, true, WPB><<<grid, block, 0, s>>>(A);
 }
+
+// Points in all from which on the adjoints (without forces, whose sums in a forest have
+// to be those of the sets alone) are walked by single waves in the groups' own order:
+// the launch then dwarfs the tail that the teams shorten.  Teams and single waves,
+// adjoints of order 1, 2 and 3 in ms: 40 sets of 2.6e6 points 11.7, 16.8, 13.3 and 11.4,
+// 16.8, 13.5; 52 sets of 4.1e6 21.3, 31.8, 25.0 and 19.9, 31.5, 24.8; 64 sets of 4.9e6 25.2,
+// 37.3, 29.4 and 22.9, 35.2, 27.9; one set of 2e6 (orders 2, 3) 26.1, 20.6 and 27.1, 21.8,
+// of 4e6 121.0, 91.7 and 119.6, 91.0.
+constexpr int64_t kAlonePoints = 3000000;
 }  // namespace
 
 int schedule_groups(hipStream_t s, char* ws, const Layout& L, int64_t n, int kind,
@@ -2199,13 +2213,16 @@ int walk(hipStream_t s, char* ws, const Layout& L, int64_t n, float beta, float 
   A.adjq = reinterpret_cast<float*>(ws + L.adjq);
   A.stats = want_stats ? hdr->stats : nullptr;
   // teams walk every set, except with monopole terms those of kSinglePoints
-  // and more (a forest may hold both kinds)
-  const bool singles = order == 1 && n >= kSinglePoints;
-  const bool teams = !singles || L.nsets > 1;
+  // and more (a forest may hold both kinds) and in adjoints of kAlonePoints in all
+  const bool f = forces != nullptr;
+  const bool alone =
+      vjp && !f && n >= kAlonePoints && (order != 1 || L.nsets > 1);
+  const bool singles = alone || (order == 1 && n >= kSinglePoints);
+  const bool teams = !alone && (!singles || L.nsets > 1);
   A.order = nullptr;
   A.gcost = nullptr;
   A.small = nullptr;
-  if (singles) {
+  if (singles && !alone) {
     const int* claims = nullptr;
     float* cost = nullptr;
     const int rc = schedule_groups(s, ws, L, n, vjp ? 1 : 0, &claims, &cost);
@@ -2220,7 +2237,6 @@ int walk(hipStream_t s, char* ws, const Layout& L, int64_t n, float beta, float 
     SBH_LAUNCH_CHECK();
   }
   if (ev_walk != nullptr) SBH_HIP_TRY(hipEventRecord(ev_walk[0], s));
-  const bool f = forces != nullptr;
   if (teams) {
     // persistent blocks: two (adjoint) or four (forward) of 8 waves fit on a
     // CU, half as many of 16
@@ -2245,10 +2261,10 @@ int walk(hipStream_t s, char* ws, const Layout& L, int64_t n, float beta, float 
     const unsigned grid =
         grid_for(n, 64 * wpb, static_cast<unsigned>((waves_cap + wpb - 1) / wpb));
     switch (wpb) {
-      case 1: launch_walk<1>(s, grid, vjp, f, A); break;
-      case 2: launch_walk<2>(s, grid, vjp, f, A); break;
-      case 8: launch_walk<8>(s, grid, vjp, f, A); break;
-      default: launch_walk<4>(s, grid, vjp, f, A); break;
+      case 1: launch_walk<1>(s, grid, vjp, order, f, A); break;
+      case 2: launch_walk<2>(s, grid, vjp, order, f, A); break;
+      case 8: launch_walk<8>(s, grid, vjp, order, f, A); break;
+      default: launch_walk<4>(s, grid, vjp, order, f, A); break;
     }
   }
   SBH_LAUNCH_CHECK();

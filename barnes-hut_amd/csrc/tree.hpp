@@ -32,9 +32,10 @@ struct Header {
   int32_t tq[8];       // the teams' work queues, as xq
 };
 
-// Tag of the schedule of the walks by single waves (monopole terms, sets from
-// kSinglePoints on): the group costs in the workspace were measured by a walk over `groups` groups (the tag is checked, never trusted: any
-// cost values give a valid claim order).
+// Tag of the schedule of the monopole walks by single waves (sets from
+// kSinglePoints on): the group costs in the workspace were measured by a walk over
+// `groups` groups (the tag is checked, never trusted: any cost values give a valid
+// claim order).
 constexpr uint32_t kSchedMagic = 0x5c4ed01eu;
 struct Sched {
   uint32_t magic;
