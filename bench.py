@@ -89,12 +89,13 @@ TRAFFIC_PROFILES = [os.path.join(ROOT, "profiles", f) for f in (
     "gravity_walk_plummer_n1048576_quad_hbm_traffic.md")]
 
 
-def walk_kernel(vjp, order, forces):
-    """Kernel of a single set of 2^20 points: monopole walks by single waves, the
-    others by teams of 8 waves."""
-    if order == 1:
-        return f"k_walk<{str(vjp).lower()},{str(forces).lower()},4>"
-    return f"k_walk_team<{str(vjp).lower()},{order},{str(forces).lower()},8>"
+def walk_kernel(vjp, order, forces, n=1 << 20):
+    """Kernel that walks a single set of n >= 700,000 points: monopole walks and
+    adjoints from 3,000,000 points on by single waves, the others by teams of 8."""
+    kind = f"{str(vjp).lower()},{order},{str(forces).lower()}"
+    if order == 1 or (vjp and not forces and n >= 3000000):
+        return f"k_walk<{kind},4>"
+    return f"k_walk_team<{kind},8>"
 
 
 def profiled_traffic(vjp, order, forces):
@@ -1684,7 +1685,7 @@ def measure_batched(args, dev, tune=True, cpu=False):
                          "vjp_build": prof[4] / max(prof[3], 1),
                          "vjp_walk_kernel": walk_vjp_ms},
            "roofline": valu_roofline(
-               walk_kernel(True, vjp_order, False) + " (all sets)", flops_vjp,
+               walk_kernel(True, vjp_order, False, n_total) + " (all sets)", flops_vjp,
                flops_vjp_impl, walk_vjp_ms)}
     if cpu:
         big_args = argparse.Namespace(**vars(args))
