@@ -375,7 +375,12 @@ __device__ __forceinline__ Leaf3 sload_leaf3(const Leaf3* leaf, uint32_t j) {
 constexpr int kRun = 4;              // points read together
 constexpr int kWStack = 96;          // >= 7 * 10 + 8 entries for max_depth 10
 constexpr uint32_t kRootEntry = ~0u;  // stack entry whose only child is node 0
-constexpr int kAccs = 4;             // partial sums per query
+constexpr int kAccs = 4;             // partial sums per query (kParts, kSplitParts)
+
+// How a query's contributions add up: kAccs partial sums by subtree, kept by one
+// wave or dealt to the kAccs waves of a block, or one running sum in the order
+// of the reference's DFS.
+enum WalkSums { kParts, kSplitParts, kRunning };
 
 // Partial sum of the node in child slot c: the 8 octants twice over the 4
 // sums, so that neighbours in every direction differ.
@@ -443,16 +448,21 @@ __device__ __forceinline__ bool outside(const Child& c, float x, float y, float 
 // the expression itself; likewise a displacement that may not be the minimum
 // image falls back to min_image_floor.
 //
-// Every query keeps kAccs partial sums, combined in a fixed order at the end.
-// A node of level split_level, with all below it, belongs to one of them by
+// kParts, kSplitParts: every query keeps kAccs partial sums, combined in a fixed
+// order at the end.  A node of level split_level, with all below it, belongs to one of them by
 // its child slot, and so does each node above (for its own far field or leaf
 // sum).  Each partial sum adds up in traversal order; a traversal restricted
 // to an ancestor-closed subset keeps its order, so a query's result depends
 // on the tree and on itself alone, bit for bit, not on the other lanes.  It
-// does not depend on SPLIT either: with SPLIT kAccs waves share a chunk of 64
+// is the same for both: with kSplitParts kAccs waves share a chunk of 64
 // queries, all of them walk the levels above split_level, and each takes the
 // subtrees and nodes of its own partial sum.  Queries run in Morton order
 // (order[t]) so that the lanes of a wave share most of their paths.
+//
+// kRunning (see running_sums()): one sum per query in the order of the
+// reference's DFS, the last child first, each with all below it before the next.
+// An opened child is descended into at once, its parent put back with the
+// children still to do, which costs the parent's fetch again.
 //
 // Bound by VALU issue where chunks fill the chip (the walk of a short-range
 // force tests 2000 children per chunk, a quarter of the lanes of which then use
@@ -469,7 +479,7 @@ __device__ __forceinline__ bool outside(const Child& c, float x, float y, float 
 // PER, CUT: periodicity and attenuation as template arguments: the walk without
 // them carries no such arithmetic, and no branch inside a run of points keeps
 // its loads from being issued together (same bits either way).
-template <int KIND, bool PER, bool CUT, bool SPLIT>
+template <int KIND, bool PER, bool CUT, WalkSums SUMS>
 __global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(
     KIND == kSoftVjp ? 5 : KIND == kSoftForce ? 6 : 8))) void k_walk8(const Leaf3* __restrict__ leaf,
                                               const Node8* __restrict__ nodes,
@@ -481,11 +491,15 @@ __global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(
                                               uint32_t split_level) {
   constexpr bool kScalar = o8::kScalarKind<KIND>;
   constexpr int kVec = kScalar ? 1 : 3;
+  constexpr bool SPLIT = SUMS == kSplitParts, RUNNING = SUMS == kRunning;
+  constexpr int kHeld = SUMS == kParts ? kAccs : 1;  // partial sums a wave holds
   static_assert(!SPLIT || kB / 64 == kAccs, "a split chunk is one block");
   P.periodic = PER ? 1 : 0;
   __shared__ uint32_t s_node[kB / 64][kWStack];
   __shared__ uint64_t s_lanes[kB / 64][kWStack];
-  __shared__ uint8_t s_key[kB / 64][kWStack];  // of a deep node (its children's too), else kAccs
+  // partial sum of a deep node (and all below it), else kAccs; RUNNING: mask of
+  // the children to do
+  __shared__ uint8_t s_key[kB / 64][kWStack];
   __shared__ Child s_child[kB / 64][8];
   __shared__ float s_sum[SPLIT ? kAccs - 1 : 1][kVec][64];
   const int lane = threadIdx.x & 63;
@@ -511,18 +525,18 @@ __global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(
   const float limit = P.box * (0.5f - 1e-5f);
   // sum: the partial sum in use, number cur (SPLIT: the wave's own); the
   // others rest in acc
-  float sum[3] = {}, acc[SPLIT ? 1 : kAccs][3] = {};
+  float sum[3] = {}, acc[kHeld][3] = {};
   uint32_t cur = SPLIT ? w : 0;
   auto use_sum = [&](uint32_t k) {
-    if (SPLIT || k == cur) return;
+    if (kHeld == 1 || k == cur) return;
 #pragma unroll
-    for (uint32_t m = 0; m < kAccs; ++m)
+    for (uint32_t m = 0; m < kHeld; ++m)
       if (cur == m)
-        for (int a = 0; a < kVec; ++a) acc[SPLIT ? 0 : m][a] = sum[a];
+        for (int a = 0; a < kVec; ++a) acc[m][a] = sum[a];
 #pragma unroll
-    for (uint32_t m = 0; m < kAccs; ++m)
+    for (uint32_t m = 0; m < kHeld; ++m)
       if (k == m)
-        for (int a = 0; a < kVec; ++a) sum[a] = acc[SPLIT ? 0 : m][a];
+        for (int a = 0; a < kVec; ++a) sum[a] = acc[m][a];
     cur = k;
   };
   uint32_t* stk_node = s_node[w];
@@ -538,7 +552,7 @@ __global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(
     if (lane == 0) {
       stk_node[0] = kRootEntry;
       stk_lanes[0] = all;
-      stk_key[0] = kAccs;
+      stk_key[0] = RUNNING ? 0xff : kAccs;
     }
     top = 1;
   }
@@ -609,11 +623,11 @@ __global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(
         slab[lane] = c;
       }
     }
-    uint32_t todo = static_cast<uint32_t>(__ballot(have)) & 0xffu;
+    uint32_t todo = static_cast<uint32_t>(__ballot(have)) & (RUNNING ? key : 0xffu);
     __builtin_amdgcn_wave_barrier();
     while (todo != 0) {
-      const int slot = __builtin_ctz(todo);
-      todo &= todo - 1;
+      const int slot = RUNNING ? 31 - __builtin_clz(todo) : __builtin_ctz(todo);
+      todo &= ~(1u << slot);
       const Child c = slab[slot];
       const uint32_t own = __builtin_amdgcn_readfirstlane(c.key);
       const bool ours = !SPLIT || own == static_cast<uint32_t>(w);
@@ -703,11 +717,20 @@ __global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(
         }
       }
       const uint64_t open = use & ~far;
+      if (RUNNING && open != 0 && todo != 0 && top < kWStack) {
+        if (lane == 0) {
+          stk_node[top] = id;
+          stk_lanes[top] = lanes;
+          stk_key[top] = static_cast<uint8_t>(todo);
+        }
+        ++top;
+        todo = 0;
+      }
       if (open != 0 && top < kWStack) {
         if (lane == 0) {
           stk_node[top] = c.id;
           stk_lanes[top] = open;
-          stk_key[top] = static_cast<uint8_t>(c.deep ? own : kAccs);
+          stk_key[top] = static_cast<uint8_t>(RUNNING ? 0xff : c.deep ? own : kAccs);
         }
         ++top;
       }
@@ -722,12 +745,14 @@ __global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(
     if (w > 0 || !valid) return;
     for (int a = 0; a < kVec; ++a)
       r[a] = (sum[a] + s_sum[0][a][lane]) + (s_sum[1][a][lane] + s_sum[2][a][lane]);
+  } else if constexpr (RUNNING) {
+    if (!valid) return;
+    for (int a = 0; a < kVec; ++a) r[a] = sum[a];
   } else {
     if (!valid) return;
     use_sum(0);
     for (int a = 0; a < kVec; ++a)
-      r[a] = (sum[a] + acc[1 % (SPLIT ? 1 : kAccs)][a]) +
-             (acc[2 % (SPLIT ? 1 : kAccs)][a] + acc[3 % (SPLIT ? 1 : kAccs)][a]);
+      r[a] = (sum[a] + acc[1 % kHeld][a]) + (acc[2 % kHeld][a] + acc[3 % kHeld][a]);
   }
   if constexpr (kScalar) {
     out[q] = r[0];
@@ -750,21 +775,47 @@ uint64_t total_nodes8(int max_depth) {
 using o8::check_walk_common;
 using o8::make_walk_params;
 
-template <int KIND, bool SOFT, bool SPLIT>
+template <int KIND, bool SOFT, WalkSums SUMS>
 auto pick_walk(const WalkParams& P) {
+  constexpr bool kPer = SUMS != kRunning;  // running sums: never periodic
   if constexpr (SOFT) {
     if (P.cutoff)
-      return P.periodic ? k_walk8<KIND, true, true, SPLIT> : k_walk8<KIND, false, true, SPLIT>;
+      return P.periodic ? k_walk8<KIND, kPer, true, SUMS> : k_walk8<KIND, false, true, SUMS>;
   }
-  return P.periodic ? k_walk8<KIND, true, false, SPLIT> : k_walk8<KIND, false, false, SPLIT>;
+  return P.periodic ? k_walk8<KIND, kPer, false, SUMS> : k_walk8<KIND, false, false, SUMS>;
+}
+
+int tree_depth(uint32_t num_nodes) {
+  int depth = 0;
+  while (depth < 10 && total_nodes8(depth) < num_nodes) ++depth;
+  return depth;
 }
 
 // Level whose nodes the partial sums divide: two above the leaves, so that a
 // query's neighbourhood spreads over all sums while few nodes lie above.
-uint32_t split_level(uint32_t num_nodes) {
-  int depth = 0;
-  while (depth < 10 && total_nodes8(depth) < num_nodes) ++depth;
-  return static_cast<uint32_t>(depth > 3 ? depth - 2 : 1);
+uint32_t split_level(int depth) { return static_cast<uint32_t>(depth > 3 ? depth - 2 : 1); }
+
+// Whether a query's contributions go to one running sum (kRunning): large clouds
+// in trees of few levels, whose full leaves give a query 1e5 terms and more.  A
+// running sum loses terms below half an ulp of it, partial sums fewer of them:
+// they are up to five times closer to 64 bits there, but move a force by 5e-5
+// from what the reference's order gives (Plummer sphere of 262,144 points,
+// depth 5, cutoff 0.5; 3e-5 at depth 6, 1.3e-5 at depth 7; without cutoff 1.8e-5,
+// 1e-5 and 8e-6), and callers compare with that order.  From 98,304 points on at
+// depth 5 (half as many more per level, twice as many without cutoff, whose tail
+// of small terms is missing) the difference passes 1e-5: running sums, which give
+// the same as the walk of one query after another to 3e-7.  Below, and in periodic
+// boxes (short sums, 5e-7), partial sums: forces and VJP of 65,537 points at
+// depth 6 with cutoff 9.4 ms against 15.5.  Above, little is lost: 150,001 points at
+// depth 5 54 ms against 43, 262,144 126 against 123 (134 and 293 with a node
+// at a time).  The rule looks at the tree alone, so that a query's bits do not
+// depend on how many are asked.
+bool running_sums(const WalkParams& P, uint32_t num_leaves, int depth) {
+  if (P.periodic) return false;
+  double line = P.cutoff ? 98304.0 : 196608.0;
+  for (int d = 5; d < depth; ++d) line *= 1.5;
+  for (int d = 5; d > depth; --d) line /= 1.5;
+  return num_leaves >= line;
 }
 
 // Chunks of 64 queries below which each is walked by kAccs waves: 4096 chunks
@@ -789,16 +840,20 @@ int launch_walk(void* stream, const SbhBuffer* leaf_bytes, const SbhBuffer* node
     if (rc != SBH_OK) return rc;
   }
   const auto num_nodes = static_cast<uint32_t>(byte_count(node_bytes) / sizeof(Node8));
-  const bool split = (nq + 63) / 64 < kSplitChunks;
+  const auto num_leaves = static_cast<uint32_t>(byte_count(leaf_bytes) / sizeof(Leaf3));
+  const int depth = tree_depth(num_nodes);
+  const bool running = running_sums(P, num_leaves, depth);
+  const bool split = !running && (nq + 63) / 64 < kSplitChunks;
   constexpr bool kSoft = o8::kPrunedKind<KIND>;
-  auto* walk = split ? pick_walk<KIND, kSoft, true>(P) : pick_walk<KIND, kSoft, false>(P);
+  auto* walk = running ? pick_walk<KIND, kSoft, kRunning>(P)
+               : split ? pick_walk<KIND, kSoft, kSplitParts>(P)
+                       : pick_walk<KIND, kSoft, kParts>(P);
   walk<<<split ? grid_for(nq, 64) : grid_for(nq, kB), kB, 0, s>>>(
       static_cast<const Leaf3*>(leaf_bytes->data), static_cast<const Node8*>(node_bytes->data),
       static_cast<const float*>(queries->data),
       cot ? static_cast<const float*>(cot->data) : nullptr, nq, order,
       static_cast<float*>(out->data),
-      P, num_nodes, static_cast<uint32_t>(byte_count(leaf_bytes) / sizeof(Leaf3)),
-      split_level(num_nodes));
+      P, num_nodes, num_leaves, split_level(depth));
   SBH_LAUNCH_CHECK();
   return SBH_OK;
 }
