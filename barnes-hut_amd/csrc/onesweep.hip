@@ -39,7 +39,19 @@ constexpr int kBlock = 512;
 // keys 7 us a pass with 2 and 12 with 8 (2^20 keys: 21 with 8, 27 with 2048 keys a
 // tile).
 constexpr int kMaxItems = 8;
-int items_for(int64_t n) { return n <= (int64_t{1} << 15) ? 2 : n <= (int64_t{1} << 17) ? 4 : 8; }
+constexpr int64_t kTwoItems = int64_t{1} << 15, kFourItems = int64_t{1} << 17;
+int items_for(int64_t n) { return n <= kTwoItems ? 2 : n <= kFourItems ? 4 : kMaxItems; }
+int64_t tiles_for(int64_t n) {
+  const int64_t tile = static_cast<int64_t>(kBlock) * items_for(n);
+  return (n + tile - 1) / tile;
+}
+// Tiles to reserve scratch for: those of any sort of at most n keys (the tiles
+// grow at kTwoItems and kFourItems, so that a larger sort may have fewer), so that
+// scratch of a given size also holds every smaller sort.
+int64_t tiles_reserved(int64_t n) {
+  return std::max({tiles_for(n), tiles_for(std::min(n, kTwoItems)),
+                   tiles_for(std::min(n, kFourItems))});
+}
 constexpr int kRadix = 256;
 constexpr int kWaves = kBlock / 64;
 constexpr int kHistBlocks = 128;
@@ -68,8 +80,7 @@ struct OsLayout {
 
 OsLayout os_layout(int64_t n, int passes) {
   auto align = [](size_t x) { return (x + 255) & ~size_t{255}; };
-  const int64_t tile = static_cast<int64_t>(kBlock) * items_for(n);
-  const size_t tiles = static_cast<size_t>((n + tile - 1) / tile);
+  const size_t tiles = static_cast<size_t>(tiles_reserved(n));
   OsLayout L;
   size_t o = 0;
   L.hist = o; o = align(o + 4ull * hist_blocks(n) * kMaxPasses * kRadix);
@@ -463,8 +474,7 @@ int morton_sort(hipStream_t s, const uint32_t* codes, int64_t n, int key_bits,
   auto* ticket = reinterpret_cast<uint32_t*>(t + L.ticket);
   auto* status = reinterpret_cast<uint32_t*>(t + L.status);
   const int items = items_for(n);
-  const int64_t tile = static_cast<int64_t>(kBlock) * items;
-  const int64_t tiles = (n + tile - 1) / tile;
+  const int64_t tiles = tiles_for(n);
   const int blocks = hist_blocks(n);
   k_os_hist<<<blocks, kHistBlock, 0, s>>>(codes, n, code_passes, set_passes, set_offs, nsets,
                                             hist, status,
