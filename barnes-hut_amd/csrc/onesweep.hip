@@ -24,8 +24,9 @@
 //
 // Every wait ends: a block spins only on tiles with smaller tickets, which
 // were taken by blocks already running that publish their counts before
-// they wait themselves; a spin that exceeds kSpinLimit reads (a fault
-// elsewhere) raises bit 16 of *flag and stops.
+// they wait themselves.  A thread that has spun kSpinLimit times all the same
+// counts its digit in the earlier tiles itself, so that the result is right in any
+// case.
 #include "common.hpp"
 #include "tree.hpp"
 
@@ -177,7 +178,7 @@ __global__ __launch_bounds__(kBlock) void k_os_pass(
     const uint32_t* __restrict__ keys_in, const uint32_t* __restrict__ vals_in, int64_t n,
     int shift, const uint32_t* __restrict__ offs, uint32_t* __restrict__ ticket,
     uint32_t* __restrict__ status, const int32_t* __restrict__ set_offs, int nsets,
-    uint32_t* __restrict__ keys_out, uint32_t* __restrict__ vals_out, int32_t* __restrict__ flag) {
+    uint32_t* __restrict__ keys_out, uint32_t* __restrict__ vals_out) {
   constexpr int kTile = kBlock * kItems;
   __shared__ uint32_t s_tile;
   __shared__ uint32_t s_base[kRadix];
@@ -195,18 +196,21 @@ __global__ __launch_bounds__(kBlock) void k_os_pass(
   const uint32_t tile = s_tile;
   const int64_t base = static_cast<int64_t>(tile) * kTile;
   const int64_t run = base + wave * (64 * kItems) + lane;
+  auto value = [&](int64_t i) {
+    return vals_in != nullptr ? vals_in[i] : static_cast<uint32_t>(i);
+  };
+  auto digit_of = [&](uint32_t k, uint32_t v) {
+    const uint32_t d = SET_PASS ? static_cast<uint32_t>(row_set(set_offs, nsets, v)) : k;
+    return (d >> shift) & 255u;
+  };
   uint32_t key[kItems], val[kItems], dig[kItems], loc[kItems];
 #pragma unroll
   for (int r = 0; r < kItems; ++r) {
     const int64_t i = run + r * 64;
     const bool ok = i < n;
-    key[r] = (ok && keys_in != nullptr) ? keys_in[i] : 0u;
-    val[r] = ok ? (vals_in != nullptr ? vals_in[i] : static_cast<uint32_t>(i)) : 0u;
-    if (SET_PASS)
-      dig[r] = ok ? (static_cast<uint32_t>(row_set(set_offs, nsets, val[r])) >> shift) & 255u
-                  : kRadix;
-    else
-      dig[r] = ok ? (key[r] >> shift) & 255u : kRadix;
+    key[r] = ok ? keys_in[i] : 0u;
+    val[r] = ok ? value(i) : 0u;
+    dig[r] = ok ? digit_of(key[r], val[r]) : kRadix;
   }
   // rank the keys in (wave, round, lane) order, the input's: loc = the key's
   // offset among its wave's keys of the digit.  Only this wave touches its counts
@@ -271,7 +275,8 @@ __global__ __launch_bounds__(kBlock) void k_os_pass(
     k -= used;
     if (used == 0) {
       if (++spins >= kSpinLimit) {
-        atomicOr(flag, 1 << 16);
+        for (int64_t i = 0; i < (k + 1) * kTile; ++i)
+          excl += digit_of(keys_in[i], value(i)) == static_cast<uint32_t>(tid) ? 1u : 0u;
         break;
       }
       __builtin_amdgcn_s_sleep(1);
@@ -442,7 +447,7 @@ size_t morton_sort_temp_bytes(int64_t n, int nsets) {
 
 int morton_sort(hipStream_t s, const uint32_t* codes, int64_t n, int key_bits,
                 const int32_t* set_offs, int nsets, uint32_t* keys_a, uint32_t* vals_a,
-                uint32_t* keys_b, uint32_t* vals_b, void* temp, int32_t* flag,
+                uint32_t* keys_b, uint32_t* vals_b, void* temp,
                 const uint32_t** keys, const uint32_t** perm) {
   *keys = nullptr;
   *perm = nullptr;
@@ -493,7 +498,7 @@ int morton_sort(hipStream_t s, const uint32_t* codes, int64_t n, int key_bits,
     auto pass = [&](auto kernel) {
       kernel<<<static_cast<unsigned>(tiles), kBlock, 0, s>>>(
           kin, vin, n, 8 * (set_pass ? p - code_passes : p), offs + p * kRadix, ticket + p, st,
-          set_offs, nsets, kout, vout, flag);
+          set_offs, nsets, kout, vout);
     };
     if (items == 2)
       set_pass ? pass(k_os_pass<true, 2>) : pass(k_os_pass<false, 2>);
@@ -515,20 +520,18 @@ __global__ __launch_bounds__(kBlock) void k_rows(uint32_t* __restrict__ vals, in
   const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
   if (i < n) vals[i] = static_cast<uint32_t>(i);
 }
-size_t flag_bytes() { return 256; }
 }  // namespace
 
 size_t order_temp_bytes(int64_t n) {
-  return n < kMaxKeys ? morton_sort_temp_bytes(n, 1) + flag_bytes() : radix_sort_temp_bytes(n);
+  return n < kMaxKeys ? morton_sort_temp_bytes(n, 1) : radix_sort_temp_bytes(n);
 }
 
 int order_by_key(hipStream_t s, uint32_t* keys, int64_t n, int key_bits, uint32_t* vals,
                  uint32_t* keys2, uint32_t* vals2, void* temp, const uint32_t** sorted,
                  const uint32_t** perm) {
   if (n < kMaxKeys)
-    return morton_sort(s, keys, n, key_bits, nullptr, 1, keys2, vals2, keys, vals,
-                       static_cast<char*>(temp) + flag_bytes(), static_cast<int32_t*>(temp),
-                       sorted, perm);
+    return morton_sort(s, keys, n, key_bits, nullptr, 1, keys2, vals2, keys, vals, temp, sorted,
+                       perm);
   k_rows<<<grid_for(n, kBlock), kBlock, 0, s>>>(vals, n);
   SBH_LAUNCH_CHECK();
   *sorted = keys2;

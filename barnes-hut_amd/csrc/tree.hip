@@ -2009,7 +2009,7 @@ int build_rest(hipStream_t s, char* ws, const Layout& L, const float* pts, const
     const uint32_t* order = nullptr;
     const uint32_t* sorted = nullptr;
     int rc = morton_sort(s, codes_in, n, 3 * max_depth, offs, nsets, keys, vals, codes, perm,
-                         ws + L.sort_tmp, &hdr->overflow, &sorted, &order);
+                         ws + L.sort_tmp, &sorted, &order);
     if (rc != SBH_OK) return rc;
     k_gather<<<grid_for(n, kB), kB, 0, s>>>(pts, ms, cot, n, order, sorted, perm, codes, sp, sc);
     SBH_LAUNCH_CHECK();
