@@ -1440,12 +1440,18 @@ __global__ __launch_bounds__(1024) void k_group_order(Header* __restrict__ hdr,
                                                       const Sched* sched_other) {
   __shared__ float s_max[16];
   __shared__ int s_bin[kOrderBins];
+  __shared__ int s_own, s_other;
   const int ng = hdr->num_groups;
   const int2 r = gw::eighth_range(ng, static_cast<int>(blockIdx.x));
-  // block 0 rewrites the own tag below; a block that reads the new tag early
-  // orders by stale costs, which changes only the schedule
-  const bool own = sched_own->magic == kSchedMagic && sched_own->groups == ng;
-  const bool other = sched_other->magic == kSchedMagic && sched_other->groups == ng;
+  // Block 0 rewrites the own tag below; a block that reads the new tag early
+  // orders by stale costs, which changes only the schedule, as long as all of its
+  // threads read the same: one reads for all.
+  if (threadIdx.x == 0) {
+    s_own = sched_own->magic == kSchedMagic && sched_own->groups == ng ? 1 : 0;
+    s_other = sched_other->magic == kSchedMagic && sched_other->groups == ng ? 1 : 0;
+  }
+  __syncthreads();
+  const bool own = s_own != 0, other = s_other != 0;
   const float* gcost = own ? cost_own : cost_other;
   const bool cost = own || other;
   if (nsets > 1) {
