@@ -2165,16 +2165,19 @@ void launch_walk(hipStream_t s, unsigned grid, bool vjp, int order, bool f, cons
 }
 
 // Points in all from which on the adjoints (without forces, whose sums in a forest have
-// to be those of the sets alone) are walked by single waves in the groups' own order:
-// the launch then dwarfs the tail that the teams shorten.  Teams and single waves,
-// adjoints of order 1, 2 and 3 in ms: 40 sets of 2.6e6 points 11.7, 16.8, 13.3 and 11.4,
-// 16.8, 13.5; 52 sets of 4.1e6 21.3, 31.8, 25.0 and 19.9, 31.5, 24.8; 64 sets of 4.9e6 25.2,
-// 37.3, 29.4 and 22.9, 35.2, 27.9; one set of 2e6 (orders 2, 3) 26.1, 20.6 and 27.1, 21.8,
-// of 4e6 121.0, 91.7 and 119.6, 91.0.
+// to be those of the sets alone) are walked by single waves, heaviest groups first:
+// the launch then dwarfs the tail that the teams shorten.  Teams and single waves in
+// the groups' own order, adjoints of order 1, 2 and 3 in ms: 40 sets of 2.6e6 points 11.7,
+// 16.8, 13.3 and 11.4, 16.8, 13.5; 52 sets of 4.1e6 21.3, 31.8, 25.0 and 19.9, 31.5, 24.8;
+// 64 sets of 4.9e6 25.2, 37.3, 29.4 and 22.9, 35.2, 27.9; one set of 2e6 (orders 2, 3)
+// 26.1, 20.6 and 27.1, 21.8, of 4e6 121.0, 91.7 and 119.6, 91.0.  Own order and heaviest
+// first (another run): 45 sets of 3.4e6 16.4, 24.5, 19.7 and 15.8, 23.7, 18.8; 52 sets 20.7,
+// 32.2, 25.4 and 20.2, 31.3, 24.7; 64 sets 23.7, 36.5, 29.1 and 23.8, 36.5, 28.9; one set
+// of 3e6 47.6, 36.8 and 47.4, 36.3, of 4e6 122.4, 92.9 and 123.6, 93.2.
 constexpr int64_t kAlonePoints = 3000000;
 }  // namespace
 
-int schedule_groups(hipStream_t s, char* ws, const Layout& L, int64_t n, int kind,
+int schedule_groups(hipStream_t s, char* ws, const Layout& L, int64_t n, int kind, bool all,
                     const int** order, float** cost) {
   auto* costs = reinterpret_cast<float*>(ws + L.gcost);
   auto* tags = reinterpret_cast<Sched*>(ws + L.sched);
@@ -2182,7 +2185,8 @@ int schedule_groups(hipStream_t s, char* ws, const Layout& L, int64_t n, int kin
   *order = reinterpret_cast<const int*>(ws + L.gorder);
   *cost = costs + own * nn;
   k_group_order<<<8, 1024, 0, s>>>(reinterpret_cast<Header*>(ws + L.header),
-                                   reinterpret_cast<const int32_t*>(ws + L.offs), L.nsets,
+                                   reinterpret_cast<const int32_t*>(ws + L.offs),
+                                   all ? 1 : L.nsets,
                                    reinterpret_cast<const int2*>(ws + L.groups), *cost,
                                    costs + (1 - own) * nn, reinterpret_cast<int*>(ws + L.gorder),
                                    tags + own, tags + (1 - own));
@@ -2228,14 +2232,14 @@ int walk(hipStream_t s, char* ws, const Layout& L, int64_t n, float beta, float 
   A.order = nullptr;
   A.gcost = nullptr;
   A.small = nullptr;
-  if (singles && !alone) {
+  if (singles) {
     const int* claims = nullptr;
     float* cost = nullptr;
-    const int rc = schedule_groups(s, ws, L, n, vjp ? 1 : 0, &claims, &cost);
+    const int rc = schedule_groups(s, ws, L, n, vjp ? 1 : 0, alone, &claims, &cost);
     if (rc != SBH_OK) return rc;
     A.order = claims;
     A.gcost = cost;
-    if (L.nsets > 1) A.small = hdr->small;
+    if (L.nsets > 1 && !alone) A.small = hdr->small;
   }
   if (vjp) {
     k_zero_adjoint<<<grid_for(4 * n + 12 * L.cap, kB, 8192), kB, 0, s>>>(hdr, n, A.sgrad, A.adj,

@@ -96,8 +96,10 @@ __device__ __forceinline__ int set_of(const int32_t* __restrict__ offs, int nset
 // the costs the previous walk of the same kind (0: forward-type walks, 1:
 // adjoint walks; else the other kind) measured in this workspace.  *order is
 // the permutation for gw::next_group, *cost where the walk stores each
-// group's measured cost.  Only the schedule depends on them.
-int schedule_groups(hipStream_t s, char* ws, const Layout& L, int64_t n, int kind,
+// group's measured cost.  Only the schedule depends on them.  all: single waves
+// walk every group, else (forests) those of sets from kSinglePoints on, and the
+// others come first.
+int schedule_groups(hipStream_t s, char* ws, const Layout& L, int64_t n, int kind, bool all,
                     const int** order, float** cost);
 
 // Data bounds of n points on the device (no host synchronisation): min - 1e-3

@@ -54,3 +54,29 @@ def test_schedule_of_single_waves_changes_no_result(gpu, sizes):
         # gradients: float atomics in arrival order
         for a, b in ((gx, gx0), (gm, gm0)):
             assert ((a - b).double().norm() / b.double().norm()).item() < 1e-5
+
+
+# Adjoints of 3,000,000 points and more in all go by single waves too, every group
+# of every set, and by cost: the walk leaves its costs' tag (a mark, then the
+# number of groups) in the workspace for the next one.
+@pytest.mark.parametrize("sizes,order", [((3000000,), 3), ((1690000, 690000, 65, 620011), 1),
+                                         ((1690000, 690000, 65, 620011), 2)])
+def test_large_adjoints_are_ordered_by_cost(gpu, sizes, order):
+    G = _G()
+    n = sum(sizes)
+    P, M, C = (torch.cat(t) for t in zip(*(_points(k, k) for k in sizes)))
+    offs = G.set_offsets(sizes)
+    ws = G.new_batch_workspace(n, len(sizes), 10, 32).zero_()
+    runs = []
+    for _ in range(3):
+        st = G.new_stats()
+        gx, gm = G.gravity_force_vjp_batch(P, M, C, offs, softening_scale=0.005, leaf_size=32,
+                                           multipole_order=order, workspace=ws, stats=st)
+        runs.append((gx, gm, G.stats_dict(st)))
+    words = ws[: ws.numel() // 4 * 4].view(torch.int32)
+    tags = words[1:][words[:-1] == 0x5C4ED01E]
+    assert runs[0][2]["groups"] in tags.tolist()
+    for gx, gm, st in runs[1:]:
+        assert st == runs[0][2]
+        for a, b in ((gx, runs[0][0]), (gm, runs[0][1])):
+            assert ((a - b).double().norm() / b.double().norm()).item() < 1e-5
