@@ -1278,8 +1278,8 @@ __device__ __forceinline__ void near_batch(const WalkArgs& A, const Lane& L, int
     scatter_batch<4 * CH, 4, 4, true, true>(part, L.red, lane, A.sgrad, 4, nullptr, -1, j0, s1);
 }
 
-// Near sources [s0, s1) (sorted points), wave-uniform bounds.
-template <bool VJP, int ORDER, bool FORCES>
+// Near sources [s0, s1) (sorted points), wave-uniform bounds, B at a time.
+template <bool VJP, int ORDER, bool FORCES, int B>
 __device__ __forceinline__ void near_range(const WalkArgs& A, const Lane& L, int i, int base,
                                            int nvalid, int s0, int s1, int lane, float& fx,
                                            float& fy, float& fz, float& gx, float& gy, float& gz,
@@ -1290,29 +1290,28 @@ __device__ __forceinline__ void near_range(const WalkArgs& A, const Lane& L, int
   // self pairs are skipped
   n_near += static_cast<unsigned long long>(s1 - s0) * nvalid -
             static_cast<unsigned long long>(max(0, min(s1, base + nvalid) - max(s0, base)));
-  // batches of 8, then the rest exactly (4, 2, 1); the quadrupole adjoint
-  // and the adjoint that also returns forces pad their last batch of 8
-  // instead (tail variants push them past their register budget and cost
-  // more than the padding saves)
-  if constexpr (VJP && (ORDER == 2 || FORCES)) {
+  // batches of B, then the rest exactly (4, 2, 1); the quadrupole adjoint pads its
+  // last batch of 8 instead (tail variants push it past its register budget and
+  // cost more than the padding saves)
+  if constexpr (VJP && ORDER == 2) {
     for (int j0 = s0; j0 < s1; j0 += kChunk)
       near_batch<VJP, FORCES, kChunk, true, true>(A, L, i, j0, s1, lane, fx, fy, fz, gx, gy, gz);
   } else {
     int j0 = s0;
-    if constexpr (VJP) {
+    if constexpr (VJP && !FORCES) {
       // ranges away from the group's own points skip the self-pair test
       if (s1 <= base || s0 >= base + nvalid) {
-        for (; j0 + kChunk <= s1; j0 += kChunk)
-          near_batch<VJP, FORCES, kChunk, false>(A, L, i, j0, s1, lane, fx, fy, fz, gx, gy, gz);
+        for (; j0 + B <= s1; j0 += B)
+          near_batch<VJP, FORCES, B, false>(A, L, i, j0, s1, lane, fx, fy, fz, gx, gy, gz);
       }
     }
     if constexpr (kWide) {
       for (; j0 + 2 * kChunk <= s1; j0 += 2 * kChunk)
         near_batch<VJP, FORCES, 2 * kChunk>(A, L, i, j0, s1, lane, fx, fy, fz, gx, gy, gz);
     }
-    for (; j0 + kChunk <= s1; j0 += kChunk)
-      near_batch<VJP, FORCES, kChunk>(A, L, i, j0, s1, lane, fx, fy, fz, gx, gy, gz);
-    if (j0 + 4 <= s1) {
+    for (; j0 + B <= s1; j0 += B)
+      near_batch<VJP, FORCES, B>(A, L, i, j0, s1, lane, fx, fy, fz, gx, gy, gz);
+    if (B > 4 && j0 + 4 <= s1) {
       near_batch<VJP, FORCES, 4>(A, L, i, j0, s1, lane, fx, fy, fz, gx, gy, gz);
       j0 += 4;
     }
@@ -1399,8 +1398,8 @@ __device__ __forceinline__ void walk_group(const WalkArgs& A, int base, int cnt,
         ++b;
       }
       s1 = __builtin_amdgcn_readfirstlane(s1);  // wave-uniform: keeps source loads scalar
-      near_range<VJP, ORDER, FORCES>(A, L, i, base, cnt, s0, s1, lane, fx, fy, fz, gx, gy, gz,
-                                     n_near);
+      near_range<VJP, ORDER, FORCES, kChunk>(A, L, i, base, cnt, s0, s1, lane, fx, fy, fz, gx,
+                                             gy, gz, n_near);
     }
   };
 
@@ -1606,7 +1605,13 @@ k_walk_team(WalkArgs A) {
   static_assert(64 * TEAM >= kTeamWidth && kShares % TEAM == 0, "team size");
   constexpr int kVals = (FORCES ? 3 : 0) + (VJP ? 3 : 0);
   constexpr int kPer = kTeamRun<ORDER>;
-  constexpr int C = (VJP && ORDER != 1) ? kChunk / 2 : (!VJP && ORDER == 1) ? kPer : kChunk;
+  // Nodes and sources at a time: fewer where the node has 10 partials, and in the
+  // adjoint that also returns forces (monopole terms: with 8, the last sources
+  // padded, it spilled 16 to 26 registers a thread: 64 sets of 4.9e6 points orders 1
+  // and 3 32.4 and 38.1 ms, now 27.8 and 32.1, one wave per group 29.2 and 35.0; 100,003
+  // Plummer points 2.38 and 2.81, 2.04 and 2.50, 4.42 and 5.70).
+  constexpr int C = VJP && (ORDER != 1 || FORCES) ? kChunk / 2 : (!VJP && ORDER == 1) ? kPer : kChunk;
+  constexpr int B = VJP && FORCES ? kChunk / 2 : kChunk;
   constexpr int kSoft = kTeamSoft<FORCES>, kStack = kSoft + 8 * 24;
   constexpr int kNear = kTeamNear<FORCES>;
   __shared__ int s_stack[kStack];
@@ -1750,8 +1755,8 @@ k_walk_team(WalkArgs A) {
               ++e;
               continue;
             }
-            near_range<VJP, ORDER, FORCES>(A, L, i, base, cnt, s0, s1, lane, fx, fy, fz, gx, gy,
-                                           gz, pairs);
+            near_range<VJP, ORDER, FORCES, B>(A, L, i, base, cnt, s0, s1, lane, fx, fy, fz, gx,
+                                              gy, gz, pairs);
           }
         }
         // large leaves (points that share a cell at the depth limit, or a large
@@ -1763,8 +1768,8 @@ k_walk_team(WalkArgs A) {
           if (s1 - s0 <= kTeamBig) continue;
 #pragma unroll 1
           for (int j = s0 + 64 * v; j < s1; j += 64 * kShares)
-            near_range<VJP, ORDER, FORCES>(A, L, i, base, cnt, j, min(j + 64, s1), lane, fx, fy,
-                                           fz, gx, gy, gz, pairs);
+            near_range<VJP, ORDER, FORCES, B>(A, L, i, base, cnt, j, min(j + 64, s1), lane, fx,
+                                              fy, fz, gx, gy, gz, pairs);
         }
         if (lane == 0) s_pairs[w] += pairs;
         float* sum = &s_sum[v][0][lane];
