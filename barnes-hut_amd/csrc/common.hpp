@@ -237,13 +237,22 @@ __device__ __forceinline__ uint32_t morton3(uint32_t x, uint32_t y, uint32_t z) 
   return spread3(x) | (spread3(y) << 1) | (spread3(z) << 2);
 }
 
-constexpr float kTwoOverSqrtPi = 2.0f / 1.772453850905516f;
-constexpr float kTwoSqrtPi = 2.0f * 1.772453850905516f;
-
 // 1/sqrt(x) by the hardware instruction (about 1 ulp).  Callers pass
 // r^2 + eps^2 + 1e-12 >= 1e-12, far from the denormal range that rsqrtf's
 // extra compare-and-scale (three more VALU operations) handles.
 __device__ __forceinline__ float rsq_softened(float x) { return __builtin_amdgcn_rsqf(x); }
+
+// The constants of a cutoff are rounded once, from 64 bits (loop-invariant: a wave
+// computes them before its sums), and finite for every cutoff > 0, so that they
+// times an exponential of 0 stay 0.
+__device__ __forceinline__ float cutoff_constant(double x) {
+  return static_cast<float>(fmin(fmax(x, -3.4e38), 3.4e38));
+}
+// 1 / (2 sqrt(pi) rc^3), of the radial term of the gradients.
+__device__ __forceinline__ float radial_cutoff(float rc) {
+  const double c = rc;
+  return cutoff_constant(1.0 / (2.0 * 1.7724538509055160 * c * c * c));
+}
 
 // Short-range attenuation erfc(u) + 2u/sqrt(pi) exp(-u^2), u = r / (2 r_c)
 // (src/sbh_ffi.cu:151-157).  Also returns exp(-u^2) and r.
@@ -251,21 +260,27 @@ __device__ __forceinline__ float rsq_softened(float x) { return __builtin_amdgcn
 // Both terms share exp(-u^2): att = exp(-u^2) (1 + z) with
 // z = erfcx(u) - 1 + 2u/sqrt(pi) = w S(v), v = p u / (1 + p u), w = p u v,
 // p = 0.45 (z is u^2 at first order and 2u/sqrt(pi) at large u, so S is smooth
-// and bounded), and S a least-maximum fit of degree 7 on u in [0, 10]: 1.4e-8 of
-// 1 + z.  The product form keeps z's rounding relative to z, which vanishes
-// with u, where close pairs lie.  The hardware square root, reciprocal and
-// exponential (1 ulp each) make it 28 issue slots where erfcf, expf, sqrtf
-// and a division took about 110; against 64 bits att is as exact as with those
-// (root mean square of a pair's error, the softened kernel's rounding
-// included, for u <= 0.5 1.1e-7 against 1.2e-7, in (0.5, 1] 9.0e-8 against
-// 9.8e-8, in (1, 1.5] 5.2e-8 against 5.3e-8).  Periodic TreePM force of 128^3
-// particles (build and walk): 20.0 -> 17.8 ms.
+// and bounded), and S a least-maximum fit of degree 7 on u in [0, 10]: with the
+// coefficients as written within 3.0e-8 of 1 + z.  The product form keeps z's
+// rounding relative to z, which vanishes with u, where close pairs lie.  The
+// hardware square root, reciprocal and exponential (1 ulp each) make it 28 issue
+// slots where erfcf, expf, sqrtf and a division took about 110.
+// Measured against 64 bits, relative error of a pair's force (root mean square over 8
+// cutoffs from 0.05 to 30, the rounding of r s^3 included), here and with those
+// functions: u < 0.5 1.11e-7 and 1.18e-7, [0.5, 1) 1.20e-7 and 1.27e-7, [1, 1.5)
+// 1.45e-7 and 1.50e-7, [1.5, 2) 1.93e-7 and 1.79e-7, [2, 3) 3.1e-7 and 3.7e-7, [3, 4) 5.6e-7
+// and 5.3e-7, [4, 6) 1.1e-6 and 1.4e-6, [6, 8) 2.15e-6 and 2.10e-6: the rounding of u^2, which
+// falls on other steps (att is 0.21 at u = 1.5, 0.046 at 2, 4e-4 at 3).  Periodic TreePM
+// force of 128^3 particles (build and walk): 20.0 -> 17.8 ms.
 __device__ __forceinline__ float attenuation(float r2, float rc, float* exp_u2,
                                              float* dist) {
+  const double c = rc;
+  const float k = cutoff_constant(-0.25 * 1.4426950408889634 / (c * c));
+  const float p = cutoff_constant(0.225 / c);
   const float t = r2 + 1e-12f;
   const float r = __builtin_amdgcn_sqrtf(t);
-  const float e = __builtin_amdgcn_exp2f(t * ((-0.25f * 1.4426950408889634f / rc) / rc));
-  const float pu = r * (0.225f / rc);
+  const float e = __builtin_amdgcn_exp2f(t * k);
+  const float pu = r * p;
   const float v = pu * __builtin_amdgcn_rcpf(1.0f + pu);
   float q = -0.0074539776f;
   q = fmaf(q, v, 0.125911623f);

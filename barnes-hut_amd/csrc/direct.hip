@@ -54,7 +54,7 @@ __device__ __forceinline__ void pair_kernel(float dx, float dy, float dz, const 
     float e, dist;
     const float att = attenuation(r2, P.rc, &e, &dist);
     lin = att * s3;
-    rad = fmaf(3.0f * s2, lin, s3 * (dist * e) * (1.0f / (kTwoSqrtPi * P.rc * P.rc * P.rc)));
+    rad = fmaf(3.0f * s2, lin, s3 * (dist * e) * radial_cutoff(P.rc));
   } else {
     const float s =
         rsq_softened(fmaf(dz, dz, fmaf(dy, dy, fmaf(dx, dx, P.eps2 + 1e-12f))));

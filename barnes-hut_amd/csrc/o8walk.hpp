@@ -165,7 +165,7 @@ __device__ __forceinline__ void pair_terms(float dx, float dy, float dz, float m
       float e, dist;
       lin = attenuation(r2, P.rc, &e, &dist) * s3;
       if constexpr (KIND == kSoftVjp)
-        cc = s3 * (dist * e) * (1.0f / (kTwoSqrtPi * P.rc * P.rc * P.rc));
+        cc = s3 * (dist * e) * radial_cutoff(P.rc);
     } else {
       lin = s3;
     }
