@@ -107,8 +107,10 @@ __device__ __forceinline__ void add_pair(Query& q, float sx, float sy, float sz,
     q.ay = fmaf(t, dy, q.ay);
     q.az = fmaf(t, dz, q.az);
   } else {
-    // the self pair is zero in exact arithmetic (its two halves cancel)
-    if (self) lin = rad = 0.0f;
+    // the self pair is zero in exact arithmetic (its two halves cancel); left out,
+    // not weighted with 0: its cotangent may be infinite or NaN, and the
+    // point's mass gradient does not depend on that
+    if (self) return;
     const float u = fmaf(dz, q.gz, fmaf(dy, q.gy, dx * q.gx));
     const float v = fmaf(dz, cz, fmaf(dy, cy, dx * cx));
     const float t = rad * fmaf(sm, u, -(q.m * v));
