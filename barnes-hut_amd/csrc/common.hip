@@ -16,6 +16,13 @@ struct WsEntry {
   void* ptr = nullptr;
   size_t bytes = 0;
 };
+// The calling thread's capture mode set to relaxed while it lives.
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 std::mutex g_ws_mutex;
 std::map<std::tuple<int, hipStream_t, int>, WsEntry> g_ws;
 }  // namespace
@@ -44,6 +51,9 @@ void* workspace(hipStream_t stream, int slot, size_t bytes) {
   std::lock_guard<std::mutex> lock(g_ws_mutex);
   WsEntry& e = g_ws[std::make_tuple(dev, stream, slot)];
   if (e.bytes >= bytes) return e.ptr;
+  // the allocation has nothing to do with what another host thread may be
+  // capturing, which it would invalidate in the default mode
+  RelaxedCapture relaxed;
   if (e.ptr != nullptr) {
     // Work queued on this stream may still read the old buffer.
     if (hipStreamSynchronize(stream) != hipSuccess) return nullptr;
