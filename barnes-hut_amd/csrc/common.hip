@@ -63,7 +63,10 @@ void* workspace(hipStream_t stream, int slot, size_t bytes) {
   }
   size_t rounded = (bytes + (1u << 20) - 1) & ~static_cast<size_t>((1u << 20) - 1);
   void* p = nullptr;
-  if (hipMalloc(&p, rounded) != hipSuccess) return nullptr;
+  if (hipMalloc(&p, rounded) != hipSuccess) {
+    (void)hipGetLastError();  // a caller that can do without goes on: not its next launch's error
+    return nullptr;
+  }
   e.ptr = p;
   e.bytes = rounded;
   return p;

@@ -391,8 +391,10 @@ int launch_direct_as(hipStream_t s, const float* pts, const float* ms, const flo
   int blocks = direct_blocks(n, nq, CUT);
   float* part = nullptr;
   if (blocks > 1) {
-    // unsplit under stream capture (the scratch could need an allocation)
-    if (!stream_capturing(s))
+    // unsplit under stream capture (the scratch could need an allocation), on the
+    // per-thread default stream (one handle, but a stream for each host thread), and
+    // where there is no memory for the scratch
+    if (s != hipStreamPerThread && !stream_capturing(s))
       part = static_cast<float*>(
           workspace(s, kWsDirect, sizeof(float) * C * static_cast<size_t>(blocks) * nq));
     if (part == nullptr) blocks = 1;
