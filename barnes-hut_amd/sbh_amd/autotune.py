@@ -8,13 +8,18 @@ sets and, separately, on every set sampled with at least 16 rows (rows are
 dealt to the sets in proportion to their size, 4 to 64 each, so the largest
 sets, where the error is largest, are checked on their own).  The search is
 coordinate-wise by default (adjoint orders x leaf sizes, then forward orders,
-grids and block sizes at the best so far: 10 + 1 + 2 + 3 captures) or the
-full product.  Results are cached per workload key (device, total points,
-set sizes, a digest of the per-set bounding boxes and the physics
-parameters) for the life of the process, and optionally in a JSON file.
+grids and block sizes at the best so far) or the full product.  The block size
+acts on walks by single waves alone (monopole walks of sets of 700,000 points,
+adjoints of 3,000,000 points in all), and teams of waves fill the chip with far
+fewer blocks: by default a batch without the former is timed with two grids and one
+block size (10 + 1 + 1 captures, else 10 + 1 + 2 + 3).  Results are cached per workload
+key (device, library build, total points, set sizes, a digest of the per-set
+bounding boxes and the physics parameters) for the life of the process, and
+optionally in a JSON file.
 """
 from __future__ import annotations
 
+import functools
 import hashlib
 import json
 import os
@@ -24,13 +29,20 @@ from typing import Iterable, Optional
 import torch
 
 from . import gravity as G
+from ._lib import library_path
 from .graph import Graph
 
 _CACHE: dict = {}
 
 DEFAULT_LEAF = (8, 16, 24, 32, 48)
+# walks by single waves: grids and block sizes (256 is the library default)
 DEFAULT_BLOCKS = (0, 1024, 4096)
-DEFAULT_THREADS = (256, 64, 128, 512)  # walk block size; 256 is the library default
+DEFAULT_THREADS = (256, 64, 128, 512)
+# walks by teams alone: 256 to 1024 blocks by default, their own block size
+TEAM_BLOCKS = (0, 256)
+TEAM_THREADS = (256,)
+SINGLE_WAVE_SET = 700000       # points of a set from which monopole walks are by single waves
+SINGLE_WAVE_POINTS = 3000000   # points in all from which every adjoint is
 # adjoint expansions: the second-moment adjoint (cheaper), then the full quadrupole
 DEFAULT_VJP_ORDERS = (G.SECOND_MOMENT_ADJOINT, 2)
 # forward expansions: the quadrupole first (the more accurate), then the monopole
@@ -55,12 +67,27 @@ def _set_boxes(points: torch.Tensor, offsets: torch.Tensor) -> torch.Tensor:
     return torch.cat([lo, hi], 1)
 
 
+def _single_waves(offsets: torch.Tensor, orders: Iterable[int]) -> bool:
+    """Whether a walk of this batch with one of the expansion `orders` runs by
+    single waves (else all by teams, whose block size is fixed)."""
+    sizes = offsets[1:] - offsets[:-1]
+    large = int(sizes.max()) if sizes.numel() else 0
+    return (1 in orders and large >= SINGLE_WAVE_SET) or int(offsets[-1]) >= SINGLE_WAVE_POINTS
+
+
+@functools.lru_cache(maxsize=None)
+def _library_digest(path: str) -> str:
+    with open(path, "rb") as fh:
+        return hashlib.sha1(fh.read()).hexdigest()[:12]
+
+
 def _key(points: torch.Tensor, offsets: torch.Tensor, kw: dict) -> str:
     h = hashlib.sha1(offsets.cpu().numpy().tobytes())
     h.update(_set_boxes(points, offsets).cpu().numpy().tobytes())
     dev = torch.cuda.get_device_name(points.device).replace(" ", "_")
     phys = ",".join(f"{k}={kw[k]}" for k in sorted(kw))
-    return f"{dev}_n{int(offsets[-1])}_s{offsets.shape[0] - 1}_{h.hexdigest()[:16]}_{phys}"
+    lib = _library_digest(library_path())
+    return f"{dev}_lib{lib}_n{int(offsets[-1])}_s{offsets.shape[0] - 1}_{h.hexdigest()[:16]}_{phys}"
 
 
 def direct_rows_fp64(P, M, C, rows, eps):
@@ -178,8 +205,8 @@ def time_graph(step, reps: int = 3) -> float:
 
 
 def tune_batch(P, M, C, offsets, *, leaf_sizes: Iterable[int] = DEFAULT_LEAF,
-               walk_blocks: Iterable[int] = DEFAULT_BLOCKS,
-               walk_threads: Iterable[int] = DEFAULT_THREADS,
+               walk_blocks: Optional[Iterable[int]] = None,
+               walk_threads: Optional[Iterable[int]] = None,
                vjp_orders: Optional[Iterable[int]] = None,
                fwd_orders: Optional[Iterable[int]] = None, search: str = "coordinate",
                reps: int = 3, cache_file: Optional[str] = None, gate: float = REL_L2_GATE,
@@ -194,7 +221,10 @@ def tune_batch(P, M, C, offsets, *, leaf_sizes: Iterable[int] = DEFAULT_LEAF,
     candidate reached (the timings are kept) and says so in the result's
     "gate".  vjp_orders / fwd_orders: adjoint and forward expansions to try
     (defaults DEFAULT_VJP_ORDERS / DEFAULT_FWD_ORDERS, or kw["multipole_order"]
-    / kw["fwd_multipole_order"] alone when given).  search: "coordinate"
+    / kw["fwd_multipole_order"] alone when given).  walk_blocks / walk_threads: grids
+    and block sizes to try (defaults DEFAULT_BLOCKS / DEFAULT_THREADS where a walk by
+    single waves is among the candidates, else TEAM_BLOCKS / TEAM_THREADS; a grid
+    only caps the walks' own).  search: "coordinate"
     (adjoint order x leaf size at the first forward order, then the other
     forward orders, then grid, then block size, the others at their best so
     far) or "grid" (every combination).  kw: beta, softening_scale,
@@ -206,8 +236,13 @@ def tune_batch(P, M, C, offsets, *, leaf_sizes: Iterable[int] = DEFAULT_LEAF,
         vjp_orders = DEFAULT_VJP_ORDERS if given is None else (given,)
     if fwd_orders is None:
         fwd_orders = DEFAULT_FWD_ORDERS if given_fwd is None else (given_fwd,)
-    leaf_sizes, walk_blocks, walk_threads = list(leaf_sizes), list(walk_blocks), list(walk_threads)
     vjp_orders, fwd_orders = list(vjp_orders), list(fwd_orders)
+    single = _single_waves(offsets, vjp_orders + fwd_orders)
+    if walk_blocks is None:
+        walk_blocks = DEFAULT_BLOCKS if single else TEAM_BLOCKS
+    if walk_threads is None:
+        walk_threads = DEFAULT_THREADS if single else TEAM_THREADS
+    leaf_sizes, walk_blocks, walk_threads = list(leaf_sizes), list(walk_blocks), list(walk_threads)
     if search not in ("coordinate", "grid"):
         raise ValueError("search must be 'coordinate' or 'grid'")
     if on_fail not in ("raise", "relax"):
