@@ -163,15 +163,15 @@ int radix_sort_pairs(hipStream_t stream, uint32_t* keys_in, uint32_t* vals_in,
 // Sorted keys (uint32, their low key_bits bits) and the rows in that order, ties in
 // row order; keys, vals, keys2 and vals2 (n entries each) are scratch, and
 // *sorted and *perm point at two of them.  temp holds order_temp_bytes(n).  Below
-// 2^30 rows by morton_sort (2 + passes launches; 2^21 rows of 21 bits 0.11 ms),
+// 2^30 rows by morton_sort (2^21 rows of 21 bits 0.11 ms),
 // from there on, where its counts no longer fit a word beside their flags, by
 // radix_sort_pairs (5 per pass; 0.38 ms).
 size_t order_temp_bytes(int64_t n);
 int order_by_key(hipStream_t stream, uint32_t* keys, int64_t n, int key_bits, uint32_t* vals,
                  uint32_t* keys2, uint32_t* vals2, void* temp, const uint32_t** sorted,
                  const uint32_t** perm);
-// Stable order of n rows by (set, code, row) in 2 + ceil(key_bits / 8) +
-// set-byte launches (onesweep.hip): codes (n, input order, key_bits wide),
+// Stable order of n rows by (set, code, row) in one launch up to 4096 rows, else in
+// 2 + ceil(key_bits / 8) + set-byte launches (onesweep.hip): codes (n, input order, key_bits wide),
 // set_offs the nsets + 1 row offsets of the sets (contiguous row ranges).
 // keys_a/vals_a and keys_b/vals_b are ping-pong buffers of n entries; *keys
 // and *perm point at the ones holding the sorted codes and rows.  temp holds

@@ -180,7 +180,10 @@ __device__ __forceinline__ void add_run(Query& q, cfloat* pts, cfloat* ms, cfloa
 // 0.10 ms; 65,536 sources at 4,099 queries with cutoff and periodic box 6.05 ->
 // 0.28 ms; 131,072 x 131,072 pairs (chip full both ways) force 6.94 -> 5.27,
 // query-side VJP 10.7 -> 7.2, full adjoint 18.7 -> 11.6 ms; 262,144 sources at
-// 64 queries 9.05 -> 0.034 ms.  The shorter sums are also more exact (10,000
+// 64 queries 9.05 -> 0.034 ms (a captured call has one block per chunk: 2.3).  The
+// bits of a query depend on the number of blocks, and so on how many queries are
+// asked and on capture (ranges and an order of adding that do not took 5 to 15% longer
+// in attenuated sums).  The shorter sums are also more exact (10,000
 // points: 1.4e-6 -> 7.5e-8 against 64 bits).
 template <int KIND, bool CUT, bool PER>
 __global__ __launch_bounds__(64 * kSplit) void k_direct(
@@ -352,11 +355,12 @@ bool running_sums(int64_t n, bool cut, bool periodic) {
 // 9.5 and 10.9, at 131,072 52 and 82).
 constexpr int64_t kFourLanes = 16384;
 
-// Blocks per chunk of 64 queries: enough for about 8 waves on each of the
-// 1024 SIMDs (one block per chunk from 131,072 queries on, where the chunks
-// alone give 8 waves), at least 64 sources per wave (below that the wave's
-// start, the combine and its launch, about 4 us, cost more than they save),
-// at most 256 partials per query.  Up to 1024 sources (512 with attenuation, whose
+// Blocks per chunk of 64 queries: as many whole blocks as give at most 8 waves to
+// each of the 1024 SIMDs (more than 2048 blocks would end in a second, nearly empty
+// round: 65,536 attenuated sources at 4099 queries 0.29 ms with 31 blocks per chunk,
+// 0.33 with 32), one from 65,537 queries on; at least 64 sources per wave (below
+// that the wave's start, the combine and its launch, about 4 us, cost more than
+// they save); at most 256 partials per query.  Up to 1024 sources (512 with attenuation, whose
 // pairs take three times as long) a wave's quarter is short: 1000 sources 14.0 us a call
 // unsplit and 16.4 split, 2048 21 and 16; 700 attenuated 16.4 and 17.1, 1000 22.9 and
 // 16.9.

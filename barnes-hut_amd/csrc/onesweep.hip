@@ -1,5 +1,6 @@
 // Stable LSD radix sort of 30-bit Morton codes (and of set ids) producing the
-// sorted order as a permutation, in 2 + passes launches (Adinets & Merrill,
+// sorted order as a permutation, in 2 + passes launches above 4096 keys, else in
+// one (Adinets & Merrill,
 // "Onesweep: A Faster Least Significant Digit Radix Sort for GPUs", 2022):
 //
 //   k_os_hist    per-block digit histograms of every pass (one read of the

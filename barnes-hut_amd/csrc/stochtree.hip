@@ -261,7 +261,7 @@ __device__ __forceinline__ float centre_ratio(const Q& L, float4 g) {
 //
 // Bound by VALU and scalar issue (the draws) once the chip is full.  With a wave
 // per group, 262,144 queries made 4400 groups for 4096 resident waves, and the
-// // second round was nearly empty; subdomains differ, too.  Forces of 262,144 points
+// second round was nearly empty; subdomains differ, too.  Forces of 262,144 points
 // 1.89 -> 1.57 ms in all, 65,536 1.00 -> 0.50, 4000 0.43 -> 0.22, 2^20 8.96 -> 8.72.
 constexpr int kShares = 16;
 constexpr int kTeam = 4;
@@ -351,7 +351,7 @@ __global__ __launch_bounds__(64 * TEAM) void k_stoch_walk(StochArgs A) {
             const float ratio = centre_ratio(L, gc);
             float tp;
             {
-  #pragma clang fp contract(off)
+#pragma clang fp contract(off)
               tp = fminf(cur_beta / ratio, 1.0f);
             }
             const float pu = sbh_uniform(A.seed, key, static_cast<uint32_t>(k),

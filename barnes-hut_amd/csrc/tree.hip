@@ -1936,7 +1936,7 @@ Layout layout(int64_t n, int max_depth, int leaf_size, int nsets) {
   L.perm = o; o = align(o + 4 * nn);
   L.keys_tmp = o; o = align(o + 4 * nn);
   L.vals_tmp = o; o = align(o + 4 * nn);
-  // radix sort temporaries, reused by the scan of the group counts
+  // temporaries of the sort
   L.sort_tmp = o;
   o = align(o + morton_sort_temp_bytes(n, nsets));
   L.bbox_tmp = o; o = align(o + 6 * 4 * (kBboxBlocks + 1));
@@ -2134,7 +2134,6 @@ int build_forest(hipStream_t s, char* ws, const Layout& L, const float* pts, con
 namespace {
 template <int TEAM>
 void launch_team(hipStream_t s, unsigned grid, bool vjp, int order, bool f, const WalkArgs& A) {
-
   const unsigned block = 64 * TEAM;
   if (vjp && order == 2 && f)
     k_walk_team<true, 2, true, TEAM><<<grid, block, 0, s>>>(A);
