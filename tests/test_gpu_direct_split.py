@@ -47,10 +47,11 @@ def test_attenuation_of_a_pair(gpu, rc):
 
 # Edges of the split: queries around a chunk of 64, sources around a run of 8,
 # around one source range per wave (64 each) and where the ranges of the last
-# block start beyond the sources; one block per chunk from 131,072 queries on.
+# block start beyond the sources; one block per chunk up to 1024 sources (512
+# attenuated) and from 65,537 queries on, for many sources two up to there.
 @pytest.mark.parametrize("n,m", [(1, 1), (7, 63), (8, 64), (9, 65), (255, 128), (257, 1),
                                  (513, 191), (1024, 70), (1025, 70), (2049, 64), (16385, 3),
-                                 (300, 131073)])
+                                 (300, 131073), (1500, 65536), (1500, 65537), (1500, 131073)])
 @pytest.mark.parametrize("rc,periodic", [(np.inf, False), (np.inf, True), (0.3, False),
                                          (0.3, True)])
 def test_split_sums_match_oracle(gpu, n, m, rc, periodic):
@@ -69,7 +70,9 @@ def test_split_sums_match_oracle(gpu, n, m, rc, periodic):
     # sums of n products of about 8 roundings each, their terms partly cancelling
     np.testing.assert_allclose(f[rows], rf, rtol=2e-4, atol=2e-6 * np.abs(rf).max())
     np.testing.assert_allclose(g[rows], rg, rtol=2e-4, atol=2e-6 * np.abs(rg).max())
-    if m == 1 or n > 4000:
+    # the full adjoint has no queries; among the 1500^2 pairs of the last rows some lie
+    # half a box apart to 3e-8, where 32 and 64 bits may pick opposite images
+    if m == 1 or n > 4000 or m > 65536:
         return
     cp = rng.normal(size=p.shape).astype(np.float32)
     gx, gm = ffi.softened_direct_force_full_vjp(p, w, cp, **kw)
