@@ -690,7 +690,7 @@ def other_rooflines(args, n, sf, walk_fwd_ms, flops_fwd, flops_fwd_impl, prof, d
                     "minimal_bytes": (40 + extra) * n + 48 * sf["nodes"]}
     if direct is not None:
         t = direct["direct_fwd_tflops"]
-        out["direct_sum_fwd"] = {"bound": "valu", "compute": "fp32 VALU, LDS-tiled",
+        out["direct_sum_fwd"] = {"bound": "valu", "compute": "fp32 VALU, scalar source loads",
                                  "achieved": t, "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
                                  "frac": t / FP32_PEAK_TFLOPS, "flops_per_pair": 20}
     return out
